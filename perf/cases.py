@@ -184,9 +184,10 @@ def _adjacency(x, degree, g):
             d = sq[o][:, None, :] + sq[o][:, :, None] - 2 * torch.bmm(y, y.transpose(1, 2).contiguous())
             d.masked_fill_(o[:, None, :] == o[:, :, None], math.inf)
             v, i = d.topk(near, largest=False, sorted=True)
-            at = o.reshape(-1)
-            got[at] = o.gather(1, i.view(len(o), -1)).view(-1, near)
-            far[at] = v.view(-1, near)
+            # the rows that fill up the last group have a place of their own
+            at = o.reshape(-1)[: n - s * group]
+            got[at] = o.gather(1, i.view(len(o), -1)).view(-1, near)[: len(at)]
+            far[at] = v.view(-1, near)[: len(at)]
         ids.append(got)
         dist.append(far)
     longs = degree - 2 * near
