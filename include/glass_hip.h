@@ -167,9 +167,11 @@ int glass_hip_searcher_set_query_waves(glass_hip_searcher *s, int32_t waves);
 /* Waves per query of the last launch, and optimize()'s choice for small
  * batches at the current ef. */
 int glass_hip_searcher_get_query_waves(const glass_hip_searcher *s, int32_t *last, int32_t *tuned);
-/* LDS visited-table entries per query (power of two in [256, 16384]; 0 =
- * tuned / sized from ef).  A query that visits more than half as many nodes
- * continues on the global bitset of its slot. */
+/* LDS visited-set size per query in entries of 4 bytes (power of two in
+ * [256, 16384]; 0 = tuned / sized per launch).  A graph of at most 32 rows per
+ * entry is a bitset there; else a query that visits more than 1.5 times as
+ * many nodes (0.75 times above 8,192 rows per entry) continues on the global
+ * bitset of its slot. */
 int glass_hip_searcher_set_visited_capacity(glass_hip_searcher *s, int32_t entries);
 /* Shape of the last launch: team, waves per workgroup, workgroups,
  * visited-table entries (a batch with per-query ef runs with the tuning of

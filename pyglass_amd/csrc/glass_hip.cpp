@@ -242,7 +242,13 @@ struct glass_hip_searcher {
 
     // launch configuration, tuned per ef bucket by Optimize
     struct Tune {
-        int32_t team = 8, waves_per_block = 4, vis_hash = 0;  // vis_hash 0: size from ef
+        // vis_hash 0: sized per launch (untuned_vis).  One wave per workgroup:
+        // a workgroup of w waves starts only when w wave slots of one CU are
+        // free, and its w queries must all end before they are handed on.
+        // 1, 2 and 4 waves over nine quantizers, ef 16-512 and 64-8,192
+        // queries: 1 is the fastest or within 2% of it everywhere (300k x 128
+        // SQ4U, ef 64, 8,192 queries: 462 / 467 / 481 us per batch).
+        int32_t team = 8, waves_per_block = 1, vis_hash = 0;
         int32_t spec = 1;  // integer codes: gather all neighbours' rows before the visited test
         int32_t qwaves_small = 1;  // waves per query for batches that leave wave slots idle
     };
@@ -261,13 +267,6 @@ struct glass_hip_searcher {
         int b = 0;
         for (int32_t e = 16; b < kBuckets - 1 && ef > e; e <<= 1) ++b;
         return b;
-    }
-    // LDS visited table sized to stay under half full for a typical search
-    // visiting ~16-24 nodes per unit of ef.
-    static int32_t auto_vis(int32_t ef) {
-        int32_t v = 1024;
-        while (v < 48 * ef && v < 4096) v <<= 1;
-        return v;
     }
 
     // device-resident index
@@ -727,14 +726,20 @@ int32_t grid_blocks(const glass_hip_searcher &s, const LaunchConfig &lc, int32_t
 // one when its waves share a query.
 int32_t slots_per_block(const LaunchConfig &lc) { return lc.qwaves > 1 ? 1 : lc.waves_per_block; }
 
-// Dirty-list words per slot: the bitset words a query may record as set
-// first; a query that sets more clears its whole bitset at its end.
-constexpr int32_t kDirtyWords = 4096;
+// Dirty-list words per slot: the bitset words a query may record as set; a
+// query that sets more clears its whole bitset at its end.  Above 2M rows that
+// is 256 KB and more, and the list is longer: a query's first thousands of
+// ids come from its table, recorded one word each.  Above 64M rows it is short
+// again: the fixed scratch array of the no-alloc entry point is nearly used up
+// by four bitsets there.
+int32_t dirty_words(const glass_hip_searcher &s) {
+    return s.graph.N > (2 << 20) && s.graph.N <= (64 << 20) ? 16384 : 4096;
+}
 
 // Words of slot scratch per resident wave: the PQ8 lookup table, the dirty
 // list, then an N-bit visited bitset (each a multiple of 4 words).
 int64_t slot_stride(const glass_hip_searcher &s) {
-    return s.lut_words + kDirtyWords + ((int64_t)(s.graph.N + 31) / 32 + 3) / 4 * 4;
+    return s.lut_words + dirty_words(s) + ((int64_t)(s.graph.N + 31) / 32 + 3) / 4 * 4;
 }
 
 // Slot areas start zeroed (the visited bitsets must be all zero between
@@ -791,6 +796,42 @@ int32_t round_cap(int32_t cap) { return (std::max(cap, 1) + 15) / 16 * 16; }
 // LDS of one CU (CDNA4: 160 KiB); a workgroup's per-wave areas must fit it.
 constexpr size_t kLdsPerCu = 160 * 1024;
 
+// Visited-set words of a launch that nothing has tuned: the most that cost no
+// resident wave the batch has a query for.  LDS per wave, most of it these
+// words, decides how many waves a CU holds, and waves in flight are what hides
+// the chain of gathers; a table too small moves its queries to their slots'
+// bitsets.  Measured (us per batch): 100k x 768 SQ8 IP, ef 64, 8,192 queries:
+// 256 words (12 waves per CU) 4,814, 512 (11 waves) 5,465, 4,096 (4 waves)
+// 13,432; 1M x 128 SQ4U, ef 64, 8,192 queries: 2,048 (16 waves) 447, 1,024
+// (16 waves) 705, 4,096 (8 waves) 701; 300k x 128 SQ4U, ef 128, 64 queries:
+// 4,096 238, 1,024 265.  A wave or two are given for a table that holds what a
+// search is expected to visit, 3/8 of the rows that it expands, where the
+// other would not: 1M x 128 SQ2U, ef 128, 20,000 queries: 2,048 words (15
+// waves) 2,482, 1,024 (16 waves) 4,596, 4,096 (8 waves) 3,048.  Batches that
+// leave LDS unused take the words that make the set a bitset of every row
+// (graphs of up to 524k rows); a table beyond 4,096 words, 6,144 ids, would be
+// cleared for nothing.
+int32_t untuned_vis(const glass_hip_searcher &s, LaunchConfig lc, int64_t nq, int32_t max_ef) {
+    const DeviceIndex ix = s.index();
+    const int64_t cus = std::max(1, s.cu_count);
+    const int32_t per_block = lc.qwaves > 1 ? 1 : lc.waves_per_block;  // queries of a workgroup
+    auto blocks = [&](int32_t v) {
+        lc.vis_hash = v;
+        return (int64_t)max_blocks_per_cu(ix, lc);
+    };
+    const int64_t want = std::min(blocks(256), (nq + per_block * cus - 1) / (per_block * cus));
+    for (int32_t v = 8192; v <= 16384; v *= 2)
+        if (ix.N > 16 * v && ix.N <= 32 * v && blocks(v) >= want) return v;
+    const int64_t visits = 3 * (int64_t)ix.K * max_ef / 8;
+    auto holds = [&](int32_t v) { return ix.N <= 32 * v || 3 * (int64_t)v / 2 >= visits + visits / 4; };
+    int32_t v = 4096;
+    while (v > 256 && blocks(v) < want) v /= 2;
+    if (!holds(v))
+        for (int32_t u = 2 * v; u <= 4096 && 20 * blocks(u) >= 17 * want; u *= 2)
+            if (holds(u)) return u;
+    return v;
+}
+
 // The pool lives in LDS: a capacity is served when one wave's area fits a CU
 // with the smallest visited table (about 19,000 entries at 128 dimensions).
 int check_cap(const glass_hip_searcher &s, int32_t max_cap) {
@@ -826,7 +867,7 @@ int run_batch(glass_hip_searcher &s, const float *qs_dev, int32_t nq, const int3
     if (!team_valid(s.index(), lc.team)) lc.team = default_team(s.index());
     lc.waves_per_block = s.force_wpb ? s.force_wpb : tn.waves_per_block;
     lc.cap_max = round_cap(max_cap);
-    lc.vis_hash = s.vis_override ? s.vis_override : (tn.vis_hash ? tn.vis_hash : glass_hip_searcher::auto_vis(max_ef));
+    lc.vis_hash = s.vis_override ? s.vis_override : tn.vis_hash;
     lc.spec = s.force_spec >= 0 ? s.force_spec : tn.spec;
     lc.qwaves = 1;
     {
@@ -849,6 +890,7 @@ int run_batch(glass_hip_searcher &s, const float *qs_dev, int32_t nq, const int3
                     mw.qwaves = w;
                     mw.waves_per_block = w;
                     mw.spec = 0;
+                    if (!mw.vis_hash) mw.vis_hash = 4096;
                     return (int64_t)std::max(1, max_blocks_per_cu(s.index(), mw)) * std::max(1, s.cu_count);
                 };
                 while (qw > 1 && (int64_t)nq > rounds * resident_queries(qw)) qw /= 2;
@@ -860,6 +902,7 @@ int run_batch(glass_hip_searcher &s, const float *qs_dev, int32_t nq, const int3
             }
         }
     }
+    if (!lc.vis_hash) lc.vis_hash = untuned_vis(s, lc, nq, max_ef);
     // Large pools: fewer waves per workgroup, then a smaller visited table
     // (exact at any size: it moves to the global bitset when it fills), until
     // a workgroup's LDS fits the CU.
@@ -896,7 +939,7 @@ int run_batch(glass_hip_searcher &s, const float *qs_dev, int32_t nq, const int3
     ss.visited = bs ? bs->visited : st->visited.p;
     ss.vis_stride = s.vis_stride;
     ss.lut_words = s.lut_words;
-    ss.dirty_words = kDirtyWords;
+    ss.dirty_words = dirty_words(s);
     ss.nslots = bs ? bs->max_slots : st->nslots;
     ss.work_counter = counter;
     const DeviceIndex ix = s.index();
@@ -1678,7 +1721,16 @@ int glass_hip_searcher_get_launch(const glass_hip_searcher *s, int32_t *team, in
         if (team) *team = s->force_team ? s->force_team : tn.team;
         if (waves_per_block) *waves_per_block = s->force_wpb ? s->force_wpb : tn.waves_per_block;
         if (blocks) *blocks = 0;
-        if (slots) *slots = s->vis_override ? s->vis_override : (tn.vis_hash ? tn.vis_hash : glass_hip_searcher::auto_vis(s->ef));
+        if (slots) *slots = s->vis_override ? s->vis_override : tn.vis_hash;
+        if (slots && !*slots && s->has_data) {
+            LaunchConfig lc{};
+            lc.team = s->force_team ? s->force_team : tn.team;
+            lc.waves_per_block = s->force_wpb ? s->force_wpb : tn.waves_per_block;
+            lc.cap_max = round_cap(s->ef);
+            lc.spec = s->force_spec >= 0 ? s->force_spec : tn.spec;
+            lc.qwaves = 1;
+            *slots = untuned_vis(*s, lc, INT32_MAX, s->ef);
+        }
         return GLASS_HIP_OK;
     } catch (...) {
         return exception_status();

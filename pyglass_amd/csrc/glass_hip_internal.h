@@ -72,7 +72,7 @@ struct LaunchConfig {
     int32_t waves_per_block;
     int32_t blocks;          // persistent grid size
     int32_t cap_max;         // LDS pool capacity per wave (>= every query's max(k',ef))
-    int32_t vis_hash;        // LDS visited-table entries per wave (power of two >= 256)
+    int32_t vis_hash;        // LDS visited-set words per wave (power of two >= 256)
     int32_t spec;            // integer codes: gather every neighbour's row before the visited test
     int32_t qwaves;          // waves per query: 1, or 2 / 4 (waves_per_block) waves of a workgroup on one query
 };

@@ -20,6 +20,7 @@
 //     order) keys, and `cur_` is the first unchecked index.
 // A persistent grid pulls queries from a device work counter, so one launch
 // serves any number of queries with per-query ef / k.
+#include <atomic>
 #include <mutex>
 
 #include "glass_hip.h"
@@ -174,7 +175,7 @@ constexpr bool is_int_variant(int v) { return v < 10; }
 
 // Per-wave LDS layout.  All offsets are multiples of 16 bytes.
 struct WaveLds {
-    uint32_t *vt;   // visited hash table, id+1 per slot, 0 = empty [vis_hash]
+    uint32_t *vt;   // visited table (or bitset) words [vis_hash]
     uint32_t *pk;   // pool keys [cap_max]
     uint32_t *pid;  // pool ids (bit 31 = checked) [cap_max]
     uint32_t *ck;   // candidate keys [64]
@@ -952,21 +953,43 @@ __device__ __forceinline__ void float_distances(const DeviceIndex &ix, const Wav
 }
 
 // ---------------------------------------------------------------------------
-// Exact visited set (Bitset, glass/neighbor.hpp:31-79) as an open-addressing
-// hash table in LDS holding id+1.  Ids tested together come from one
-// deduplicated adjacency row, so they are distinct: each lane either finds
-// its id or claims an empty slot with a compare-and-swap.  The table is kept
-// below half full; a query that would exceed that switches to the slot's
-// global bitset for the ids it has not seen yet, and keeps consulting the
-// table for the ids inserted before.  The bitset is all zero whenever no
-// query is using it: a query records each word it is the first to set (the
-// lane whose fetch-or returns 0) in the slot's dirty list, and clears those
-// words when it ends (the whole bitset if the list overflowed).  A query
-// thus writes about as many bitset words as it sets, instead of clearing
-// N/8 bytes (1.25 MB at 10M rows) when it switches.
+// Exact visited set (Bitset, glass/neighbor.hpp:31-79) in the wave's LDS
+// words (lc.vis_hash of them), in one of two forms:
+//   * graphs of at most 32 rows per word: a bitset, one ds_or per test;
+//   * larger ones: a hash table of 64-bit buckets of short entries.
+//     Multiplying by an odd number maps the b-bit ids onto themselves; the
+//     product's high bits are the home bucket and its low rb bits the
+//     remainder, so bucket, displacement and remainder name the id exactly
+//     and an entry holds only (displacement << rb | remainder) + 1, 0 meaning
+//     empty: four 16-bit entries per bucket when rb <= 14 (up to 16.7M rows at
+//     2,048 words), else two of 32 bits.  A bucket fills from its low end, and
+//     an id goes into the first bucket with room at or after its home, so a
+//     test reads the home bucket, looks at all of its entries at once, and
+//     claims the first empty one with a compare-and-swap of the whole bucket.
+//     Full buckets are rare below the limit, so the slowest of the wave's
+//     lanes rarely needs a second one, where probing one entry at a time
+//     waits for the longest of up to 64 chains.  Ids tested together come from
+//     one deduplicated adjacency row, so they are distinct.
+// The table is kept below kVisLoad / 8 full.  A query that would exceed that
+// moves its ids to the slot's global bitset and goes on there (and a lane
+// whose displacement does not fit puts its one id there).  That bitset is what
+// bounds a deep search: every test on it is a dependent fetch-or in memory, of
+// its own N/8-byte area.  Entries of 16 bits hold twice the ids of whole
+// 32-bit ids in the same LDS.
+// The bitset is all zero whenever no query is using it: a query records each
+// word it is the first to set (the lane whose fetch-or returns 0) in the
+// slot's dirty list, and clears those words when it ends (the whole bitset if
+// the list overflowed).  A query thus writes about as many bitset words as it
+// sets, instead of clearing N/8 bytes (1.25 MB at 10M rows).
+constexpr uint32_t kVisLoad = 6;  // eighths
+
 struct VisitedSet {
+    // odd, and its inverse modulo 2^32 (and so, masked, modulo any 2^b)
+    static constexpr uint32_t kMul = 0x9E3779B1u, kMulInverse = 0x0E8B2F51u;
     uint32_t *tab;
-    uint32_t mask, shift;
+    uint32_t bmask, rb, smask;  // id bits, remainder bits, buckets - 1
+    bool wide;           // 32-bit entries
+    bool direct;         // the LDS words are a bitset of every row
     int32_t count, thr;
     bool global;
     uint32_t *gbits;
@@ -974,75 +997,182 @@ struct VisitedSet {
     uint32_t *dirty;     // the slot's dirty list: bitset words this query set first
     int32_t dirty_cap;   // its capacity in words
     int32_t ndirty;      // words recorded (past dirty_cap: the whole bitset is cleared)
+    bool pend = false;   // this lane's compare-and-swap of test_set is still to be looked at:
+    uint32_t p_at, p_e, p_old, p_got;  // its word, entry, and the word before and as found
 
-    __device__ __forceinline__ void reset(uint32_t *t, int32_t size, uint32_t *g, int64_t gw, uint32_t *dl,
+    __device__ __forceinline__ void reset(uint32_t *t, int32_t words, int32_t n, uint32_t *g, int64_t gw, uint32_t *dl,
                                           int32_t dcap) {
         tab = t;
-        mask = (uint32_t)size - 1u;
-        shift = 32u - (uint32_t)__builtin_ctz((uint32_t)size);
+        direct = n <= 32 * words;
+        const uint32_t sb = (uint32_t)__builtin_ctz((uint32_t)words) - 1u;  // bucket bits
+        const uint32_t nb = 32u - (uint32_t)__builtin_clz((uint32_t)(n - 1) | 1u);
+        const uint32_t b = nb > sb ? nb : sb;
+        rb = b - sb;
+        wide = rb > 14u;
+        bmask = (1u << b) - 1u;  // rows are counted in 31 bits
+        smask = ((uint32_t)words >> 1) - 1u;
         count = 0;
-        thr = size / 2;
+        thr = direct ? 0x7fffffff : (int32_t)((uint32_t)words * kVisLoad / (wide ? 8u : 4u));
         global = false;
         gbits = g;
         gwords = gw;
         dirty = dl;
         dirty_cap = dcap;
         ndirty = 0;
+        pend = false;
+        p_at = p_e = p_old = p_got = 0u;
+        const int32_t used = direct ? (n + 31) >> 5 : words;
         uint4 *t4 = (uint4 *)t;
-        for (int i = lane_id(); i < size / 4; i += 64) t4[i] = make_uint4(0, 0, 0, 0);
+        for (int i = lane_id(); i < (used + 3) >> 2; i += 64) t4[i] = make_uint4(0, 0, 0, 0);
         wave_sync();
     }
 
-    __device__ __forceinline__ uint32_t home(uint32_t v) const { return (v * 0x9E3779B1u) >> shift; }
+    // Records the bitset words of the lanes of `m` as set by this query.
+    __device__ __forceinline__ void record(uint64_t m, uint32_t v) {
+        const int pos = ndirty + mbcnt(m);
+        if (((m >> lane_id()) & 1) && pos < dirty_cap) dirty[pos] = v >> 5;
+        ndirty += __builtin_popcountll(m);
+    }
+
+    // Looks v up in the table.  The home bucket, or the first one after it with
+    // room, decides: ids tested together are distinct, so a lane without a hit
+    // is new whether its compare-and-swap (issued here) succeeds or another
+    // lane of the wave took the entry; finish() looks at that later, off the
+    // path to the new ids.  Returns 0 visited, 1 new, 2 for the bitset.
+    template <bool kWide>
+    __device__ __forceinline__ int look(uint32_t v) {
+        constexpr uint32_t kMost = kWide ? 0xffffffffu : 0xffffu;
+        const uint32_t h = (v * kMul) & bmask;
+        uint32_t s = h >> rb;
+        uint32_t e = (h & ((1u << rb) - 1u)) + 1u;
+        uint2 *tb = (uint2 *)tab;
+        for (;;) {
+            const uint2 w = tb[s];
+            bool hit, full;
+            if (kWide) {
+                hit = w.x == e || w.y == e;
+                full = w.y != 0u;
+            } else {
+                // a zero half of x or y: an entry equal to e
+                const uint32_t ee = e | (e << 16), x = w.x ^ ee, y = w.y ^ ee;
+                hit = (((x - 0x00010001u) & ~x) | ((y - 0x00010001u) & ~y)) & 0x80008000u;
+                full = w.y > 0xffffu;
+            }
+            if (hit) return 0;
+            if (!full) {
+                // the bucket's first word with room: its entry, or its second one
+                const bool second = kWide ? w.x != 0u : w.x > 0xffffu;
+                const uint32_t o = second ? w.y : w.x;
+                p_at = 2u * s + (second ? 1u : 0u);
+                p_e = e;
+                p_old = o;
+                p_got = atomicCAS(&tab[p_at], o, kWide || o == 0u ? e : o | (e << 16));
+                return 1;
+            }
+            // the next bucket, its displacement one more
+            if (e > kMost - (1u << rb)) return 2;
+            e += 1u << rb;
+            s = (s + 1u) & smask;
+        }
+    }
 
     // true when v had not been visited; marks it visited.
     __device__ __forceinline__ bool test_set(uint32_t v, bool active) {
-        bool isnew = false, fresh = false;
-        if (active) {
-            const uint32_t key = v + 1u;
-            uint32_t h = home(v);
-            if (!global) {
-                // the first probe decides almost always: it stays out of the loop
-                uint32_t old = atomicCAS(&tab[h], 0u, key);
-                while (old != 0u && old != key) {
-                    h = (h + 1u) & mask;
-                    old = atomicCAS(&tab[h], 0u, key);
-                }
-                isnew = old == 0u;
+        const uint32_t bit = 1u << (v & 31u);
+        pend = false;
+        if (direct) {
+            bool isnew = false;
+            if (active) isnew = !(atomicOr(&tab[v >> 5], bit) & bit);
+            return isnew;
+        }
+        bool isnew = false, spill = active;
+        if (!global) {
+            int r = 0;
+            if (wide) {
+                if (active) r = look<true>(v);
             } else {
-                bool found = false;
-                for (;;) {
-                    const uint32_t cur = tab[h];
-                    if (cur == key) {
-                        found = true;
-                        break;
-                    }
-                    if (cur == 0u) break;
-                    h = (h + 1u) & mask;
-                }
-                if (!found) {
-                    const uint32_t bit = 1u << (v & 31u);
-                    const uint32_t old =
-                        __hip_atomic_fetch_or(&gbits[v >> 5], bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    isnew = !(old & bit);
-                    fresh = old == 0u;  // lanes on one word are serialised: one sees 0
-                }
+                if (active) r = look<false>(v);
             }
+            isnew = pend = r == 1;
+            spill = r == 2;
+            if (ballot(spill) == 0) return isnew;
         }
-        if (global) {
-            const uint64_t fm = ballot(fresh);
-            if (fm) {
-                const int pos = ndirty + mbcnt(fm);
-                if (fresh && pos < dirty_cap) dirty[pos] = v >> 5;
-                ndirty += __builtin_popcountll(fm);
-            }
+        bool fresh = false;
+        if (spill) {
+            const uint32_t was =
+                __hip_atomic_fetch_or(&gbits[v >> 5], bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            isnew = !(was & bit);
+            fresh = was == 0u;  // lanes on one word are serialised: one sees 0
         }
+        const uint64_t fm = ballot(fresh);
+        if (fm) record(fm, v);
         return isnew;
+    }
+
+    // The entries that test_set's compare-and-swap did not get: tried again
+    // from the word the other lane left.
+    __device__ __forceinline__ void finish(uint32_t v) {
+        bool again = pend && p_got != p_old;
+        while (ballot(again)) {
+            if (again) {
+                again = false;
+                const uint32_t room = wide ? 1u : 0x10000u;  // words from here on are full
+                uint32_t at = p_at, e = p_e, w = p_got;
+                for (;;) {
+                    if (w < room) {
+                        const uint32_t got = atomicCAS(&tab[at], w, w == 0u ? e : w | (e << 16));
+                        if (got == w) break;
+                        w = got;
+                        continue;
+                    }
+                    at = (at + 1u) & (2u * smask + 1u);
+                    if ((at & 1u) == 0u) {  // the next bucket
+                        if (e > (wide ? 0xffffffffu : 0xffffu) - (1u << rb)) {
+                            again = true;  // the bitset takes it, below
+                            break;
+                        }
+                        e += 1u << rb;
+                    }
+                    w = tab[at];
+                }
+            }
+            if (ballot(again)) {
+                bool fresh = false;
+                if (again)
+                    fresh = __hip_atomic_fetch_or(&gbits[v >> 5], 1u << (v & 31u), __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_WORKGROUP) == 0u;
+                const uint64_t fm = ballot(fresh);
+                if (fm) record(fm, v);
+            }
+            again = false;
+        }
+        pend = false;
+    }
+
+    // Moves the table's ids to the bitset.  Their words are recorded without
+    // waiting for what they held, so a word may be recorded twice.
+    __device__ __forceinline__ void migrate() {
+        const unsigned long long *tb = (const unsigned long long *)tab;
+        for (uint32_t i = lane_id(); i <= smask; i += 64) {  // a multiple of 64 buckets
+            const unsigned long long w = tb[i];
+            for (uint32_t at = 0; at < 64u; at += wide ? 32u : 16u) {
+                const uint32_t e = (uint32_t)(w >> at) & (wide ? 0xffffffffu : 0xffffu);
+                const uint64_t m = ballot(e != 0u);
+                if (m == 0) break;
+                const uint32_t home = (i - ((e - 1u) >> rb)) & smask;
+                const uint32_t v = (((home << rb) | ((e - 1u) & ((1u << rb) - 1u))) * kMulInverse) & bmask;
+                if (e != 0u)
+                    (void)__hip_atomic_fetch_or(&gbits[v >> 5], 1u << (v & 31u), __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_WORKGROUP);
+                record(m, v);
+            }
+        }
+        global = true;
     }
 
     // End of a query: the bitset words it set back to zero.
     __device__ __forceinline__ void cleanup() {
-        if (!global) return;
+        if (ndirty == 0) return;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_s_waitcnt(0);
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
@@ -1054,16 +1184,15 @@ struct VisitedSet {
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_s_waitcnt(0);
-        global = false;
     }
 
-    // Account for the ids a row inserted; switch to the global bitset (all
-    // zero, see above) before the table could pass half full (a row inserts
+    // Account for the ids v that test_set found new; switch to the global bitset (all
+    // zero, see above) before the table could pass its limit (a row inserts
     // at most 64 ids).
-    __device__ __forceinline__ void account(int inserted) {
-        if (global) return;
+    __device__ __forceinline__ void account(int inserted, uint32_t v) {
+        finish(v);
         count += inserted;
-        if (count > thr - 64) global = true;
+        if (count > thr - 64 && !global) migrate();
     }
 };
 
@@ -1375,10 +1504,12 @@ __device__ __forceinline__ void put_result(const QueryBatch &qb, int64_t pos, in
 // pools, long rows and visited bookkeeping spill at 128, and its launches are
 // mostly held to fewer waves by LDS anyway.  The shared-query path runs at 3
 // too: at 2, a batch of 1,000 queries at 4 waves each does not fit the device
-// in one round (it spills at 128).  Its SQ2U instance with 16 dwords per lane
-// spills at 168 and runs at 2.
+// in one round (it spills at 128).  Of the instances with 16 dwords per lane,
+// SQ2U and SQ4U shared queries spill at 168 and run at 2, and SQ2U's common
+// path spills at 128 and runs at 3.
 template <int V, int DPL, int P>
-constexpr int kWavesPerEu = P == 1 ? 4 : ((P == 2 && V == V_SQ2U && DPL == 16) ? 2 : 3);
+constexpr int kWavesPerEu = P == 1 ? (V == V_SQ2U && DPL == 16 ? 3 : 4)
+                                   : ((P == 2 && (V == V_SQ2U || V == V_SQ4U) && DPL == 16) ? 2 : 3);
 
 template <int V, int DPL, int P>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<V, DPL, P>))) void search_kernel(DeviceIndex ix,
@@ -1495,7 +1626,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu
         if (is_int_variant(V)) iq.init(ix, w);
         // empty visited set (Bitset::reset, neighbor.hpp:67-74)
         VisitedSet vs;
-        if (lead) vs.reset(w.vt, lc.vis_hash, vis, ss.vis_stride - ss.lut_words - ss.dirty_words, dlist, ss.dirty_words);
+        if (lead) vs.reset(w.vt, lc.vis_hash, ix.N, vis, ss.vis_stride - ss.lut_words - ss.dirty_words, dlist, ss.dirty_words);
 
         auto dists = [&](int m, int32_t mode) __attribute__((always_inline)) {
             if (is_int_variant(V)) {
@@ -1559,7 +1690,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu
                 w.pid[0] = u;
             }
             vs.test_set(u, l == 0);
-            vs.account(1);
+            vs.count = 1;  // the table was empty: nothing to try again, no limit near
             ps.size = 1;
             ps.cur = 0;
             wave_sync();
@@ -1583,7 +1714,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu
                     pool_merge_lds(w, ps, nep);
                 }
                 vs.test_set(ep, l < nep);
-                vs.account(nep);
+                vs.account(nep, ep);
             }
         }
 
@@ -1620,7 +1751,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu
                         const uint64_t nm = ballot(isnew);
                         if (nm) {
                             m = __builtin_popcountll(nm);
-                            vs.account(m);
+                            vs.account(m, (uint32_t)v);
                             if (isnew) w.ci[mbcnt(nm)] = (uint32_t)v;
                             break;
                         }
@@ -1683,8 +1814,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu
                     continue;
                 }
                 const int m = __builtin_popcountll(nm);
-                vs.account(m);
                 const uint32_t kj = key_of_int(iq.row_dist(c4, valid));
+                vs.account(m, (uint32_t)v);
                 cnt_d += m;
                 if (kFast || at_use(lc.cap_max) <= 128) {
                     pred = pool_merge_reg<2>(ix, w, ps, kj, (uint32_t)v, isnew, nm, nj, pred_row);
@@ -1718,9 +1849,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu
                 const uint64_t nm = ballot(isnew);
                 if (nm) {
                     const int m = __builtin_popcountll(nm);
-                    vs.account(m);
                     if (isnew) w.ci[mbcnt(nm)] = (uint32_t)vc;
                     wave_sync();
+                    vs.account(m, (uint32_t)vc);
                     dists(m, qb.mode);
                     cnt_d += m;
                     if (kFast || at_use(lc.cap_max) <= 128) {
@@ -1916,15 +2047,30 @@ hipError_t launch_one(const DeviceIndex &ix, const QueryBatch &qb, const LaunchC
     return hipGetLastError();
 }
 
+// VGPRs of the kernel a launch runs, asked of the runtime once per kernel
+// (the launch rules look at several shapes per call).  0 on error.
+template <int V, int DPL>
+int vgprs_one(const DeviceIndex &ix, const LaunchConfig &lc) {
+    static std::atomic<int> known[3] = {};
+    const int path = lc.qwaves > 1 ? 2 : (fast_path<V, DPL>(ix, lc) ? 1 : 0);
+    int v = known[path].load(std::memory_order_relaxed);
+    if (v == 0) {
+        hipFuncAttributes attr;
+        if (hipFuncGetAttributes(&attr, kernel_fn<V, DPL>(ix, lc)) != hipSuccess) return 0;
+        v = attr.numRegs;
+        known[path].store(v, std::memory_order_relaxed);
+    }
+    return v;
+}
+
 // Resident workgroups per CU from the kernel's register count and the CDNA
 // limits: 4 SIMDs x 512 VGPRs per lane (granule 8), at most 8 waves per SIMD,
 // 160 KiB of LDS per CU.
 template <int V, int DPL>
 int occupancy_one(const DeviceIndex &ix, const LaunchConfig &lc) {
     const size_t lds = block_lds_bytes(ix, lc);
-    hipFuncAttributes attr;
-    if (hipFuncGetAttributes(&attr, kernel_fn<V, DPL>(ix, lc)) != hipSuccess) return 0;
-    int vgpr = attr.numRegs > 0 ? attr.numRegs : 128;
+    int vgpr = vgprs_one<V, DPL>(ix, lc);
+    if (vgpr <= 0) return 0;
     vgpr = (vgpr + 7) / 8 * 8;
     int waves_simd = 512 / vgpr;
     if (waves_simd > 8) waves_simd = 8;
@@ -1991,13 +2137,6 @@ size_t lds_bytes_per_wave(const DeviceIndex &ix, int32_t cap_max, int32_t vis_ha
 }
 
 size_t lds_bytes_per_block(const DeviceIndex &ix, const LaunchConfig &lc) { return block_lds_bytes(ix, lc); }
-
-template <int V, int DPL>
-int vgprs_one(const DeviceIndex &ix, const LaunchConfig &lc) {
-    hipFuncAttributes attr;
-    if (hipFuncGetAttributes(&attr, kernel_fn<V, DPL>(ix, lc)) != hipSuccess) return 0;
-    return attr.numRegs;
-}
 
 template <int V>
 int vgprs_int(const DeviceIndex &ix, const LaunchConfig &lc) {
