@@ -2,8 +2,9 @@
 // PQ8 trainer and the Clustering object of the C ABI share.  Seeding and the
 // centroid update follow the reference step by step on the host (both are
 // order-dependent: every k-means++ pick depends on the previous one, and a
-// centroid is a float sum over its rows in row order); the distance sweeps
-// run on a backend, the GPU for the Clustering object.
+// centroid is a float sum over its rows in row order) for PQ8's small
+// sub-spaces; the Clustering object's sweeps, updates and distances run on
+// the GPU (cluster_kernels.hip).
 //
 // Float steps are those of the reference as GCC -Ofast compiles it:
 //   distances     helpa::l2_fp32_fp32 (l2 below, l2_helpa on the device)
@@ -89,92 +90,84 @@ double seed_total(const float *d, int32_t n) {
     return S;
 }
 
-struct HostBackend : Backend {
-    const float *x;
-    int32_t m, d;
-    int dist_to(const float *row, float *out) override {
-        for (int32_t i = 0; i < m; ++i) out[i] = l2(row, x + (int64_t)i * d, d);
-        return 0;
-    }
-    int assign(const float *cent, int32_t k, int32_t *ids) override {
-        for (int32_t i = 0; i < m; ++i) {
-            float best = HUGE_VALF;
-            int32_t bid = -1;
-            for (int32_t j = 0; j < k; ++j) {
-                const float v = l2(x + (int64_t)i * d, cent + (int64_t)j * d, d);
-                if (v < best) {
-                    best = v;
-                    bid = j;
-                }
-            }
-            ids[i] = bid;
-        }
-        return 0;
-    }
-};
-
 }  // namespace
 
-Backend *host_backend(const float *samples, int32_t m, int32_t d, void *) {
-    auto *b = new HostBackend;
-    b->x = samples;
-    b->m = m;
-    b->d = d;
-    return b;
-}
-
-int fit(const float *rows, int32_t n, int32_t d, int32_t k, int32_t epochs, bool kmeanspp, float *centroids,
-        Backend *(*make)(const float *samples, int32_t m, int32_t d, void *ctx), void *ctx) {
+std::vector<int32_t> sample_rows(int32_t n) {
     const int32_t m = std::min(n - 1, 100000);  // kSampleNum (clustering.hpp:24,75)
     std::vector<int32_t> samples(std::max(m, 1));
     std::mt19937 rng;
     gen_random(rng, samples.data(), m, n);
+    samples.resize(std::max(m, 0));
+    return samples;
+}
+
+std::vector<int32_t> random_picks(int32_t m, int32_t k) {
+    std::mt19937 r;
+    std::vector<int32_t> idx(k);
+    gen_random(r, idx.data(), k, m);
+    return idx;
+}
+
+int kmeanspp_picks(int32_t m, int32_t k, const std::function<int(int32_t, float *)> &dist_to,
+                   std::vector<int32_t> &picked) {
+    std::mt19937 r;
+    std::uniform_real_distribution<> dart_dist(0, 1);
+    std::uniform_int_distribution<int32_t> first(0, m - 1);
+    std::vector<float> dist(std::max(m, 1)), fresh(std::max(m, 1));
+    const int32_t init_id = first(r);
+    picked.assign(1, init_id);
+    if (int e = dist_to(init_id, dist.data())) return e;
+    bool sum_flag = false;
+    while ((int32_t)picked.size() < k) {
+        double dart = dart_dist(r);
+        const double sum = seed_total(dist.data(), m);
+        if (sum < 1e-6) sum_flag = true;
+        dart *= sum;
+        double prefix = 0.0;
+        int32_t pivot = 0;
+        for (int32_t i = 0; i < m; ++i) {
+            pivot = i;
+            const double next = prefix + (double)dist[i];
+            if (dart >= prefix && dart < next) break;
+            prefix = next;
+        }
+        if (std::find(picked.begin(), picked.end(), pivot) != picked.end() && !sum_flag) continue;
+        picked.push_back(pivot);
+        if (int e = dist_to(pivot, fresh.data())) return e;
+        for (int32_t i = 0; i < m; ++i) dist[i] = std::min(dist[i], fresh[i]);
+    }
+    return 0;
+}
+
+// Lloyd steps: compute_dist + find_index, update_mediods (clustering.hpp:198-256)
+void fit_host(const float *rows, int32_t n, int32_t d, int32_t k, int32_t epochs, float *centroids) {
+    const std::vector<int32_t> samples = sample_rows(n);
+    const int32_t m = (int32_t)samples.size();
     std::vector<float> tr((size_t)d * std::max(m, 1));
     for (int32_t i = 0; i < m; ++i) std::memcpy(&tr[(size_t)d * i], rows + (int64_t)d * samples[i], 4 * (size_t)d);
-    std::fill(centroids, centroids + (size_t)d * k, 0.0f);
-    std::unique_ptr<Backend> be(make(tr.data(), m, d, ctx));
-    if (!be) return GLASS_HIP_ENOMEM;
-    if (kmeanspp) {  // init_kmeanspp (clustering.hpp:138-196)
-        std::mt19937 r;
-        std::uniform_real_distribution<> dart_dist(0, 1);
-        std::uniform_int_distribution<int32_t> first(0, m - 1);
-        std::vector<float> dist(std::max(m, 1)), fresh(std::max(m, 1));
-        std::vector<int32_t> picked;
-        const int32_t init_id = first(r);
-        picked.push_back(init_id);
-        std::memcpy(centroids, &tr[(size_t)d * init_id], 4 * (size_t)d);
-        if (int e = be->dist_to(&tr[(size_t)d * init_id], dist.data())) return e;
-        bool sum_flag = false;
-        while ((int32_t)picked.size() < k) {
-            double dart = dart_dist(r);
-            const double sum = seed_total(dist.data(), m);
-            if (sum < 1e-6) sum_flag = true;
-            dart *= sum;
-            double prefix = 0.0;
-            int32_t pivot = 0;
-            for (int32_t i = 0; i < m; ++i) {
-                pivot = i;
-                const double next = prefix + (double)dist[i];
-                if (dart >= prefix && dart < next) break;
-                prefix = next;
-            }
-            if (std::find(picked.begin(), picked.end(), pivot) != picked.end() && !sum_flag) continue;
-            std::memcpy(centroids + (size_t)d * picked.size(), &tr[(size_t)d * pivot], 4 * (size_t)d);
-            picked.push_back(pivot);
-            if (int e = be->dist_to(&tr[(size_t)d * pivot], fresh.data())) return e;
-            for (int32_t i = 0; i < m; ++i) dist[i] = std::min(dist[i], fresh[i]);
-        }
-    } else {  // init_random (clustering.hpp:127-136)
-        std::mt19937 r;
-        std::vector<int32_t> idx0(k);
-        gen_random(r, idx0.data(), k, m);
-        for (int32_t i = 0; i < k; ++i) std::memcpy(centroids + (size_t)d * i, &tr[(size_t)d * idx0[i]], 4 * (size_t)d);
-    }
-    // Lloyd steps: compute_dist + find_index, update_mediods (clustering.hpp:198-256)
+    std::vector<int32_t> picks;
+    (void)kmeanspp_picks(
+        m, k,
+        [&](int32_t p, float *out) {
+            for (int32_t i = 0; i < m; ++i) out[i] = l2(&tr[(size_t)d * p], &tr[(size_t)d * i], d);
+            return 0;
+        },
+        picks);
+    for (int32_t c = 0; c < k; ++c) std::memcpy(centroids + (size_t)d * c, &tr[(size_t)d * picks[c]], 4 * (size_t)d);
     std::vector<int32_t> idx(std::max(m, 1)), cnt(k);
     std::vector<float> nm((size_t)d * k);
     for (int32_t e = 0; e < epochs; ++e) {
-        if (int r = be->assign(centroids, k, idx.data())) return r;
+        for (int32_t i = 0; i < m; ++i) {
+            float best = HUGE_VALF;
+            idx[i] = -1;
+            for (int32_t c = 0; c < k; ++c) {
+                const float v = l2(&tr[(size_t)d * i], centroids + (size_t)d * c, d);
+                if (v < best) {
+                    best = v;
+                    idx[i] = c;
+                }
+            }
+        }
         std::fill(nm.begin(), nm.end(), 0.0f);
         std::fill(cnt.begin(), cnt.end(), 0);
         for (int32_t i = 0; i < m; ++i) {
@@ -191,23 +184,32 @@ int fit(const float *rows, int32_t n, int32_t d, int32_t k, int32_t epochs, bool
         }
         std::copy(nm.begin(), nm.end(), centroids);
     }
-    return 0;
 }
 
 }  // namespace km
 
 namespace {
 
-template <typename T>
-struct DevArr {
-    T *p = nullptr;
-    DevArr() = default;
-    DevArr(const DevArr &) = delete;
-    DevArr &operator=(const DevArr &) = delete;
-    ~DevArr() {
+// One device allocation that the arrays of a call are placed in.
+struct Arena {
+    uint8_t *p = nullptr;
+    size_t used = 0;
+    Arena() = default;
+    Arena(const Arena &) = delete;
+    Arena &operator=(const Arena &) = delete;
+    ~Arena() {
         if (p) (void)hipFree(p);
     }
-    hipError_t alloc(size_t count) { return hipMalloc((void **)&p, std::max<size_t>(count, 1) * sizeof(T)); }
+    size_t add(size_t bytes) {  // offset of the next array
+        const size_t at = used;
+        used += (bytes + 255) / 256 * 256;
+        return at;
+    }
+    hipError_t alloc() { return hipMalloc((void **)&p, std::max<size_t>(used, 1)); }
+    template <typename T>
+    T *at(size_t offset) const {
+        return (T *)(p + offset);
+    }
 };
 
 int hip_fail(hipError_t e, const char *what) {
@@ -221,59 +223,95 @@ int hip_fail(hipError_t e, const char *what) {
         if (_e != hipSuccess) return hip_fail(_e, #expr); \
     } while (0)
 
-// Distance sweeps on the GPU: the sample rows stay resident, centroids and
-// picked rows are copied in per call.
-struct DeviceBackend : km::Backend {
-    int32_t m = 0, d = 0, kmax = 0;
-    DevArr<float> x, cent, row, out;
-    DevArr<int32_t> ids;
-    int dist_to(const float *r, float *o) override {
-        CL_TRY(hipMemcpy(row.p, r, 4 * (size_t)d, hipMemcpyHostToDevice));
-        CL_TRY(launch_cluster_dist(x.p, m, d, row.p, out.p, nullptr));
-        CL_TRY(hipMemcpy(o, out.p, 4 * (size_t)m, hipMemcpyDeviceToHost));
-        return 0;
+// Clustering::fit with everything but the seeding's picks on the device.  The
+// sample is gathered there too unless it is a small part of the rows.
+int fit_device(const float *rows, int32_t n, int32_t d, int32_t k, int32_t epochs, bool kmeanspp, float *centroids) {
+    const std::vector<int32_t> samples = km::sample_rows(n);
+    const int32_t m = (int32_t)samples.size();
+    const bool whole = (int64_t)n <= 4 * (int64_t)m;
+    Arena a;
+    const size_t o_all = a.add(whole ? 4 * (size_t)n * d : 0), o_rows = a.add(4 * (size_t)std::max(m, k)),
+                 o_x = a.add(4 * (size_t)m * d), o_cent = a.add(4 * (size_t)k * d), o_ids = a.add(4 * (size_t)m),
+                 o_dist = a.add(4 * (size_t)m), o_scratch = a.add(AssignScratch::bytes(m, k));
+    CL_TRY(a.alloc());
+    float *x = a.at<float>(o_x), *cent = a.at<float>(o_cent);
+    int32_t *idx = a.at<int32_t>(o_rows), *ids = a.at<int32_t>(o_ids);
+    AssignScratch s;
+    s.place(a.p + o_scratch, m, k);
+    if (whole) {
+        CL_TRY(hipMemcpy(a.at<float>(o_all), rows, 4 * (size_t)n * d, hipMemcpyHostToDevice));
+        CL_TRY(hipMemcpy(idx, samples.data(), 4 * (size_t)m, hipMemcpyHostToDevice));
+        CL_TRY(launch_cluster_gather(a.at<float>(o_all), idx, m, d, x, nullptr));
+    } else {
+        std::vector<float> tr((size_t)d * m);
+        for (int32_t i = 0; i < m; ++i) std::memcpy(&tr[(size_t)d * i], rows + (int64_t)d * samples[i], 4 * (size_t)d);
+        CL_TRY(hipMemcpy(x, tr.data(), 4 * (size_t)m * d, hipMemcpyHostToDevice));
     }
-    int assign(const float *c, int32_t k, int32_t *o) override {
-        CL_TRY(hipMemcpy(cent.p, c, 4 * (size_t)d * k, hipMemcpyHostToDevice));
-        CL_TRY(launch_cluster_assign(x.p, m, d, cent.p, k, ids.p, nullptr));
-        CL_TRY(hipMemcpy(o, ids.p, 4 * (size_t)m, hipMemcpyDeviceToHost));
-        return 0;
+    std::vector<int32_t> picks;
+    if (kmeanspp) {
+        float *dist = a.at<float>(o_dist);
+        const int e = km::kmeanspp_picks(
+            m, k,
+            [&](int32_t p, float *out) -> int {
+                CL_TRY(launch_cluster_dist(x, m, d, x + (int64_t)p * d, dist, nullptr));
+                CL_TRY(hipMemcpy(out, dist, 4 * (size_t)m, hipMemcpyDeviceToHost));
+                return 0;
+            },
+            picks);
+        if (e) return e;
+    } else {
+        picks = km::random_picks(m, k);
     }
-};
-
-struct DeviceCtx {
-    int32_t k;
-    int error = 0;
-};
-
-km::Backend *device_backend(const float *samples, int32_t m, int32_t d, void *ctx) {
-    auto *c = (DeviceCtx *)ctx;
-    auto b = std::make_unique<DeviceBackend>();
-    b->m = m;
-    b->d = d;
-    b->kmax = c->k;
-    hipError_t e;
-    if ((e = b->x.alloc((size_t)m * d)) != hipSuccess || (e = b->cent.alloc((size_t)c->k * d)) != hipSuccess ||
-        (e = b->row.alloc(d)) != hipSuccess || (e = b->out.alloc(m)) != hipSuccess ||
-        (e = b->ids.alloc(m)) != hipSuccess ||
-        (e = hipMemcpy(b->x.p, samples, 4 * (size_t)m * d, hipMemcpyHostToDevice)) != hipSuccess) {
-        c->error = hip_fail(e, "clustering device buffers");
-        return nullptr;
+    CL_TRY(hipMemcpy(idx, picks.data(), 4 * (size_t)k, hipMemcpyHostToDevice));
+    CL_TRY(launch_cluster_gather(x, idx, k, d, cent, nullptr));
+    CL_TRY(launch_cluster_norms(x, m, d, s, nullptr));
+    for (int32_t e = 0; e < epochs; ++e) {
+        CL_TRY(launch_cluster_assign(x, m, d, cent, k, ids, s, nullptr));
+        CL_TRY(launch_cluster_update(x, m, d, ids, k, cent, nullptr));
     }
-    return b.release();
+    CL_TRY(hipMemcpy(centroids, cent, 4 * (size_t)k * d, hipMemcpyDeviceToHost));
+    return GLASS_HIP_OK;
 }
 
-// nearest centroid of every row, on the device
+// Nearest centroid of every row.  Rows go to the device in pieces of about
+// 16 MB while the piece before is worked on: the copy bounds the call.
 int predict_device(const float *cent, int32_t k, int32_t d, const float *x, int32_t n, int32_t *ids) {
-    DevArr<float> dx, dc;
-    DevArr<int32_t> di;
-    CL_TRY(dx.alloc((size_t)n * d));
-    CL_TRY(dc.alloc((size_t)k * d));
-    CL_TRY(di.alloc(n));
-    CL_TRY(hipMemcpy(dx.p, x, 4 * (size_t)n * d, hipMemcpyHostToDevice));
-    CL_TRY(hipMemcpy(dc.p, cent, 4 * (size_t)k * d, hipMemcpyHostToDevice));
-    CL_TRY(launch_cluster_assign(dx.p, n, d, dc.p, k, di.p, nullptr));
-    CL_TRY(hipMemcpy(ids, di.p, 4 * (size_t)n, hipMemcpyDeviceToHost));
+    const int64_t piece = std::max<int64_t>(64, ((int64_t)4 << 20) / d / 64 * 64);
+    const int32_t rows = (int32_t)std::min<int64_t>(n, piece);
+    const int32_t bufs = n > rows ? 2 : 1;
+    Arena a;
+    const size_t o_x = a.add(4 * (size_t)rows * d * bufs), o_cent = a.add(4 * (size_t)k * d),
+                 o_ids = a.add(4 * (size_t)n), o_scratch = a.add(AssignScratch::bytes(rows, k));
+    CL_TRY(a.alloc());
+    struct Lane {
+        hipStream_t stream = nullptr;
+        hipEvent_t done[2] = {nullptr, nullptr};
+        ~Lane() {
+            if (stream) (void)hipStreamSynchronize(stream);
+            for (hipEvent_t e : done)
+                if (e) (void)hipEventDestroy(e);
+            if (stream) (void)hipStreamDestroy(stream);
+        }
+    } ln;
+    CL_TRY(hipStreamCreateWithFlags(&ln.stream, hipStreamNonBlocking));
+    for (int32_t b = 0; b < bufs; ++b) CL_TRY(hipEventCreateWithFlags(&ln.done[b], hipEventDisableTiming));
+    float *dc = a.at<float>(o_cent);
+    int32_t *di = a.at<int32_t>(o_ids);
+    AssignScratch s;
+    CL_TRY(hipMemcpy(dc, cent, 4 * (size_t)k * d, hipMemcpyHostToDevice));
+    int32_t b = 0, turn = 0;
+    for (int64_t at = 0; at < n; at += rows, b ^= bufs - 1, ++turn) {
+        const int32_t c = (int32_t)std::min<int64_t>(rows, n - at);
+        float *dx = a.at<float>(o_x) + (size_t)b * rows * d;
+        if (turn >= bufs) CL_TRY(hipEventSynchronize(ln.done[b]));
+        CL_TRY(hipMemcpy(dx, x + at * d, 4 * (size_t)c * d, hipMemcpyHostToDevice));
+        s.place(a.p + o_scratch, c, k);
+        CL_TRY(launch_cluster_norms(dx, c, d, s, ln.stream));
+        CL_TRY(launch_cluster_assign(dx, c, d, dc, k, di + at, s, ln.stream));
+        CL_TRY(hipEventRecord(ln.done[b], ln.stream));
+    }
+    CL_TRY(hipStreamSynchronize(ln.stream));
+    CL_TRY(hipMemcpy(ids, di, 4 * (size_t)n, hipMemcpyDeviceToHost));
     return GLASS_HIP_OK;
 }
 
@@ -312,13 +350,12 @@ void glass_hip_clustering_free(glass_hip_clustering *c) { delete c; }
 int glass_hip_clustering_fit(glass_hip_clustering *c, const float *data, int32_t n, int32_t dim) {
     try {
         if (!c || !data || dim <= 0) return set_error(GLASS_HIP_EINVAL, "bad clustering input");
-        // the fit samples min(n - 1, 100000) rows; random seeding draws k distinct ones of them
-        if (n < 2 || (!c->kmeanspp && std::min(n - 1, 100000) < c->k))
+        // the fit samples min(n - 1, 100000) rows; random seeding draws k
+        // distinct ones of them (GenRandom's draws are modulo their difference)
+        if (n < 2 || (!c->kmeanspp && std::min(n - 1, 100000) <= c->k))
             return set_error(GLASS_HIP_EINVAL, "too few sampled rows for the number of clusters");
         std::vector<float> cent((size_t)c->k * dim);
-        DeviceCtx ctx{c->k};
-        const int r = km::fit(data, n, dim, c->k, c->epochs, c->kmeanspp, cent.data(), device_backend, &ctx);
-        if (r) return ctx.error ? ctx.error : r;
+        if (const int r = fit_device(data, n, dim, c->k, c->epochs, c->kmeanspp, cent.data())) return r;
         c->centroids.swap(cent);
         c->dim = dim;
         return GLASS_HIP_OK;

@@ -6,7 +6,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <functional>
 #include <random>
+#include <vector>
 
 namespace glass_hip {
 
@@ -123,36 +125,50 @@ int exception_status() noexcept;
 // GenRandom (glass/utils.hpp:13-27): size sorted, distinct, rotated draws in [0, N).
 void gen_random(std::mt19937 &rng, int32_t *addr, int32_t size, int32_t N);
 
-// k-means as glass::Clustering::fit runs it (glass/algorithms/clustering.hpp),
-// over sample rows the backend evaluates distances for.
+// k-means as glass::Clustering::fit runs it (glass/algorithms/clustering.hpp).
 namespace km {
 
 // helpa::l2_fp32_fp32 in the reference's compiled order, on the host.
 float l2(const float *x, const float *y, int32_t d);
 
-struct Backend {
-    virtual ~Backend() = default;
-    // out[i] = l2(row, sample i) for every sample (k-means++ seeding)
-    virtual int dist_to(const float *row, float *out) = 0;
-    // ids[i] = first nearest of the k centroids to sample i (a Lloyd step)
-    virtual int assign(const float *cent, int32_t k, int32_t *ids) = 0;
-};
+// The row sample of Clustering::fit: min(n - 1, 100000) rows drawn by GenRandom.
+std::vector<int32_t> sample_rows(int32_t n);
 
-// Clustering::fit on n rows of d floats: samples min(n - 1, 100000) rows with
-// GenRandom, seeds k centroids (kmeans++ or random), runs `epochs` Lloyd
-// steps.  `make` builds the backend over the sampled rows.  Returns 0 or an
-// error code (the backend's).
-int fit(const float *rows, int32_t n, int32_t d, int32_t k, int32_t epochs, bool kmeanspp, float *centroids,
-        Backend *(*make)(const float *samples, int32_t m, int32_t d, void *ctx), void *ctx);
+// init_random (clustering.hpp:127-136): k distinct sample positions.
+std::vector<int32_t> random_picks(int32_t m, int32_t k);
 
-// A backend evaluating on the host (small d, e.g. PQ8's 4-dim sub-spaces).
-Backend *host_backend(const float *samples, int32_t m, int32_t d, void *ctx);
+// init_kmeanspp (clustering.hpp:138-196): k sample positions; dist(i, out)
+// gives sample i's distance to each of the m samples and returns 0 or an
+// error code, which ends the seeding and is returned.
+int kmeanspp_picks(int32_t m, int32_t k, const std::function<int(int32_t, float *)> &dist, std::vector<int32_t> &picks);
+
+// Clustering::fit on n rows of d floats, on the host (small d, e.g. PQ8's
+// 4-dim sub-spaces), seeded by k-means++.
+void fit_host(const float *rows, int32_t n, int32_t d, int32_t k, int32_t epochs, float *centroids);
 
 }  // namespace km
 
+// Device scratch of launch_cluster_assign for n rows and k centroids.
+struct AssignScratch {
+    float *x2, *c2, *m1, *m2;  // squared norms of rows and centroids, least and second least values
+    int32_t *i1, *list, *count;
+    uint32_t *c2max;
+    static size_t bytes(int32_t n, int32_t k);
+    void place(void *p, int32_t n, int32_t k);
+};
+
+// Squared norms of the rows into s.x2, once for any number of sweeps.
+hipError_t launch_cluster_norms(const float *x, int32_t n, int32_t d, const AssignScratch &s, hipStream_t stream);
+// ids[i] = first nearest of the k centroids to row i (-1: none compares less than +inf).
 hipError_t launch_cluster_assign(const float *x, int32_t n, int32_t d, const float *cent, int32_t k, int32_t *ids,
-                                 hipStream_t stream);
+                                 const AssignScratch &s, hipStream_t stream);
 hipError_t launch_cluster_dist(const float *x, int32_t n, int32_t d, const float *pivot, float *out,
                                hipStream_t stream);
+// cent[c] = mean of the rows with ids[i] == c, zero where there is none.
+hipError_t launch_cluster_update(const float *x, int32_t n, int32_t d, const int32_t *ids, int32_t k, float *cent,
+                                 hipStream_t stream);
+// out[i] = x[rows[i]], m rows.
+hipError_t launch_cluster_gather(const float *x, const int32_t *rows, int32_t m, int32_t d, float *out,
+                                 hipStream_t stream);
 
 }  // namespace glass_hip
