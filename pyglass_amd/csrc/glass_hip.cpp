@@ -833,8 +833,11 @@ constexpr size_t kLdsPerCu = 160 * 1024;
 // waves) 2,482, 1,024 (16 waves) 4,596, 4,096 (8 waves) 3,048.  Batches that
 // leave LDS unused take the words that make the set a bitset of every row
 // (graphs of up to 524k rows); a table beyond 4,096 words, 6,144 ids, would be
-// cleared for nothing.
-int32_t untuned_vis(const glass_hip_searcher &s, LaunchConfig lc, int64_t nq, int32_t max_ef) {
+// cleared for nothing.  A host call's batch is alone on the device until it
+// returns; one on a caller's stream leaves LDS for another like it (200k x 100
+// FP16, ef 64, 1,000 queries, alone and over two streams: 8,192 words 320 and
+// 230, 4,096 words 353 and 193).
+int32_t untuned_vis(const glass_hip_searcher &s, LaunchConfig lc, int64_t nq, int32_t max_ef, bool alone) {
     const DeviceIndex ix = s.index();
     const int64_t cus = std::max(1, s.cu_count);
     const int32_t per_block = lc.qwaves > 1 ? 1 : lc.waves_per_block;  // queries of a workgroup
@@ -843,8 +846,9 @@ int32_t untuned_vis(const glass_hip_searcher &s, LaunchConfig lc, int64_t nq, in
         return (int64_t)max_blocks_per_cu(ix, lc);
     };
     const int64_t want = std::min(blocks(256), (nq + per_block * cus - 1) / (per_block * cus));
+    const int64_t room = std::min(blocks(256), alone ? want : 2 * want);
     for (int32_t v = 8192; v <= 16384; v *= 2)
-        if (ix.N > 16 * v && ix.N <= 32 * v && blocks(v) >= want) return v;
+        if (ix.N > 16 * v && ix.N <= 32 * v && blocks(v) >= room) return v;
     const int64_t visits = 3 * (int64_t)ix.K * max_ef / 8;
     auto holds = [&](int32_t v) { return ix.N <= 32 * v || 3 * (int64_t)v / 2 >= visits + visits / 4; };
     int32_t v = 4096;
@@ -879,7 +883,7 @@ struct BatchState {
 int run_batch(glass_hip_searcher &s, const float *qs_dev, int32_t nq, const int32_t *ef_dev, const int32_t *k_dev,
               int32_t ef_uniform, int32_t k_uniform, int32_t max_cap, int32_t max_ef, int32_t mode,
               const int64_t *off_dev, int32_t *ids_dev, float *dists_dev, int32_t *counters_dev, hipStream_t stream,
-              const BatchState *bs = nullptr, bool graph = false) {
+              const BatchState *bs = nullptr, bool graph = false, bool alone = false) {
     if (!s.has_data) return fail(GLASS_HIP_ESTATE, "search before set_data");
     if (nq <= 0) return GLASS_HIP_OK;
     if (int r = ensure_stream(s)) return r;
@@ -925,7 +929,7 @@ int run_batch(glass_hip_searcher &s, const float *qs_dev, int32_t nq, const int3
             }
         }
     }
-    if (!lc.vis_hash) lc.vis_hash = untuned_vis(s, lc, nq, max_ef);
+    if (!lc.vis_hash) lc.vis_hash = untuned_vis(s, lc, nq, max_ef, alone);
     // Large pools: fewer waves per workgroup, then a smaller visited table
     // (exact at any size: it moves to the global bitset when it fills), until
     // a workgroup's LDS fits the CU.
@@ -1071,7 +1075,7 @@ int host_batch(glass_hip_searcher &s, const float *qs, int32_t nq, const int32_t
         d_off = s.d_off.p;
     }
     int r = run_batch(s, s.d_q.p, nq, d_ef, d_k, s.ef, k_uniform, max_cap, max_ef, mode, d_off, s.d_ids.p, s.d_dists.p,
-                      s.d_counters.p, s.stream);
+                      s.d_counters.p, s.stream, nullptr, false, true);
     if (r) return r;
     HIP_TRY(hipMemcpyAsync(dst, s.d_ids.p, 4 * (size_t)total, hipMemcpyDeviceToHost, s.stream));
     if (scores)
@@ -1752,7 +1756,7 @@ int glass_hip_searcher_get_launch(const glass_hip_searcher *s, int32_t *team, in
             lc.cap_max = round_cap(s->ef);
             lc.spec = s->force_spec >= 0 ? s->force_spec : tn.spec;
             lc.qwaves = 1;
-            *slots = untuned_vis(*s, lc, INT32_MAX, s->ef);
+            *slots = untuned_vis(*s, lc, INT32_MAX, s->ef, false);
         }
         return GLASS_HIP_OK;
     } catch (...) {

@@ -314,43 +314,49 @@ struct IntQuery {
     uint32_t q[DPL];
     int32_t qq;      // sum x^2 over this lane's slice (squared-L2 variants)
     int32_t slot;    // lanes per candidate (power of two)
-    int32_t nparts;  // active parts per candidate
-    int32_t part;    // this lane's part
+    int32_t part;    // this lane's part: 16-byte words part, part + slot, ... of a row, so that
+                     // a group's lanes read consecutive words at a time
 
     __device__ __forceinline__ void init(const DeviceIndex &ix, const WaveLds &w) {
-        const int code_dw = ix.code_size / 4;
-        nparts = (code_dw + DPL - 1) / DPL;
+        const int code_q = ix.code_size / 16;
+        const int nparts = (code_q + DPL / 4 - 1) / (DPL / 4);
         slot = 1;
         while (slot < nparts) slot <<= 1;
         part = lane_id() & (slot - 1);
-        const uint32_t *qd = (const uint32_t *)w.qcode;
+        const uint4 *qd = (const uint4 *)w.qcode;
         uint32_t acc = 0;
 #pragma unroll
-        for (int i = 0; i < DPL; ++i) {
-            int d = part * DPL + i;
-            q[i] = (part < nparts && d < code_dw) ? qd[d] : 0u;
-            if (V == V_SQ8U_L2) acc = udot4(q[i], q[i], acc);
-            if (V == V_SQ4U) acc = udot8(q[i], q[i], acc);
-            if (V == V_SQ2U) {
-                const uint32_t a0 = q[i] & 0x33333333u, a1 = (q[i] >> 2) & 0x33333333u;
-                acc = udot8(a0, a0, acc);
-                acc = udot8(a1, a1, acc);
+        for (int i = 0; i < DPL / 4; ++i) {
+            const int qi = i * slot + part;
+            const uint4 x = qi < code_q ? qd[qi] : make_uint4(0, 0, 0, 0);
+            const uint32_t xs[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t v = xs[r];
+                q[4 * i + r] = v;
+                if (V == V_SQ8U_L2) acc = udot4(v, v, acc);
+                if (V == V_SQ4U) acc = udot8(v, v, acc);
+                if (V == V_SQ2U) {
+                    const uint32_t a0 = v & 0x33333333u, a1 = (v >> 2) & 0x33333333u;
+                    acc = udot8(a0, a0, acc);
+                    acc = udot8(a1, a1, acc);
+                }
             }
         }
         qq = (int32_t)acc;
     }
 
-    // This lane's slice of code row `id` (zeros for slices past the row).
+    // This lane's slice of code row `id` (zeros for words past the row).
     // Unconditional loads (no exec-mask branch per load): a lane with no row
-    // (on false) reads row 0, whose distance is never used; slices past the
+    // (on false) reads row 0, whose distance is never used; words past the
     // row read as zero.
     __device__ __forceinline__ void load_row(const DeviceIndex &ix, uint32_t id, bool on, uint4 (&c4)[DPL / 4]) const {
         const int code_q = ix.code_size / 16;  // uint4 per row
         const uint4 *src = (const uint4 *)(ix.codes + (int64_t)(on ? id : 0u) * ix.code_size);
 #pragma unroll
         for (int i = 0; i < DPL / 4; ++i) {
-            const int qi = part * (DPL / 4) + i;
-            const bool ok = part < nparts && qi < code_q;
+            const int qi = i * slot + part;
+            const bool ok = qi < code_q;
             const uint4 x = src[ok ? qi : 0];
             c4[i] = ok ? x : make_uint4(0, 0, 0, 0);
         }
@@ -416,17 +422,31 @@ struct IntQuery {
 
     // Distances of candidates ci[0..m) -> keys ck[0..m).  With several waves
     // on one query, wave `first` of `stride` takes passes first, first +
-    // stride, ... of 64 / slot rows each.
+    // stride, ... of 64 / slot rows each.  The loads of kAhead passes are
+    // issued together, so that a node's neighbours wait on memory once per
+    // kAhead passes: a 960-byte row takes 16 lanes, and its 64 neighbours 16
+    // passes (100k x 960 SQ8U, 1,000 queries of ef 16-512: 2,150 us per batch
+    // at one pass, 1,820 at two).
+    template <int kAhead>
     __device__ __forceinline__ void distances(const DeviceIndex &ix, const WaveLds &w, int m, int first = 0, int stride = 1) const {
         const int l = lane_id();
         const int cpr = 64 / slot;
         const int cj = l / slot;
-        for (int base = first * cpr; base < m; base += stride * cpr) {
-            const int j = base + cj;
-            uint4 c4[DPL / 4];
-            load_row(ix, j < m ? w.ci[j] : 0u, j < m, c4);
-            const int32_t d = row_dist(c4, j < m);
-            if (j < m && part == 0) w.ck[j] = key_of_int(d);
+        const int step = stride * cpr;
+        for (int base = first * cpr; base < m; base += kAhead * step) {
+            uint4 c4[kAhead][DPL / 4];
+#pragma unroll
+            for (int a = 0; a < kAhead; ++a) {
+                const int j = base + a * step + cj;
+                if (a == 0 || base + a * step < m) load_row(ix, j < m ? w.ci[j] : 0u, j < m, c4[a]);
+            }
+#pragma unroll
+            for (int a = 0; a < kAhead; ++a) {
+                const int j = base + a * step + cj;
+                if (a > 0 && base + a * step >= m) break;
+                const int32_t d = row_dist(c4[a], j < m);
+                if (j < m && part == 0) w.ck[j] = key_of_int(d);
+            }
         }
     }
 };
@@ -434,141 +454,225 @@ struct IntQuery {
 // ---------------------------------------------------------------------------
 // Float distances in the reference's AVX-512 order.  The compiled reference
 // keeps 16 accumulators, acc[l] summing elements j = l, l+16, ... in
-// increasing j, then reduces the 16 partial sums in a fixed tree.  Here four
-// lanes share one row: lane p owns accumulators 4p..4p+3 and reads elements
-// 16t + 4p .. 16t + 4p + 3 (one dword of codes or one float4) per step t, so
-// every accumulator sees exactly the reference's operand sequence, and 16
-// rows are evaluated per pass.
+// increasing j, then reduces the 16 partial sums in a fixed tree.  Here L = 4,
+// 8 or 16 lanes share one row: lane p owns accumulators A p .. A p + A - 1,
+// A = 16 / L, and reads those elements of every step of 16, so every
+// accumulator sees exactly the reference's operand sequence.
 //   E5M2  glass::L2SqrE5M2 / IPE5M2   (glass/simd/avx512.hpp:15-38)
 //   SQ8   glass::L2SqrSQ8_ext / IPSQ8_ext (glass/simd/avx512.hpp:40-77)
 //   FP32  helpa::l2_fp32_fp32 / dot_fp32_fp32 (x86/l2_impl.hpp:50-71, x86/dot_impl.hpp:52-71)
 // The fused multiply-adds are where the compiled reference fuses them.
 
-struct Acc4 {
-    float a[4];
-};
-
-// Tree over the 16 partial sums held 4 per lane by a 4-lane group.
+// Tree over the 16 partial sums held A per lane by an L-lane group; valid in
+// the group's first lane.
 //   glass::reduce_add_f32x16 (glass/simd/avx512_utils.hpp:12-22):
 //     b_i = a_i + a_{i+8}, c_i = b_i + b_{i+4}, result (c0+c1)+(c2+c3)
 //   GCC _mm512_reduce_add_ps as helpa uses it (x86/utils.hpp:61-64):
 //     same b and c, result (c0+c2)+(c1+c3)
-// Lane p holds a_{4p+r}; a_{i+8} sits two lanes up, b_{i+4} one lane up.
-template <bool kGlassTree>
-__device__ __forceinline__ float reduce16_4lanes(Acc4 v) {
+// Lane p holds a_(Ap+r): a_(i+8) sits L/2 lanes up and b_(i+4) L/4 lanes up.
+// The moves by 4 and 8 lanes leave the right value in the lanes that still
+// matter only (those below L/2, then L/4).
+template <int L>
+__device__ __forceinline__ float lanes_up(float v, int step) {
+    const int32_t x = __float_as_int(v);
+    return __int_as_float(step == 1 ? dpp_xor1(x) : step == 2 ? dpp_xor2(x) : step == 4 ? dpp_down4(x) : dpp_down8(x));
+}
+
+template <int L, bool kGlassTree>
+__device__ __forceinline__ float reduce16(float (&a)[16 / L]) {
+    constexpr int A = 16 / L;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) v.a[r] = v.a[r] + dpp_xor2(v.a[r]);
+    for (int r = 0; r < A; ++r) a[r] = a[r] + lanes_up<L>(a[r], L / 2);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) v.a[r] = v.a[r] + dpp_xor1(v.a[r]);
-    return kGlassTree ? (v.a[0] + v.a[1]) + (v.a[2] + v.a[3]) : (v.a[0] + v.a[2]) + (v.a[1] + v.a[3]);
+    for (int r = 0; r < A; ++r) a[r] = a[r] + lanes_up<L>(a[r], L / 4);
+    if (A == 4) return kGlassTree ? (a[0] + a[1]) + (a[2 % A] + a[3 % A]) : (a[0] + a[2 % A]) + (a[1 % A] + a[3 % A]);
+    if (A == 2) {  // lanes 0, 1: (c0, c1), (c2, c3)
+        if (kGlassTree) {
+            const float s = a[0] + a[1 % A];
+            return s + lanes_up<L>(s, 1);
+        }
+        return (a[0] + lanes_up<L>(a[0], 1)) + (a[1 % A] + lanes_up<L>(a[1 % A], 1));
+    }
+    const float s = a[0] + lanes_up<L>(a[0], kGlassTree ? 1 : 2);
+    return s + lanes_up<L>(s, kGlassTree ? 2 : 1);
 }
 
 __device__ __forceinline__ float e5m2_to_float(uint32_t byte) {
     return __half2float(__ushort_as_half((unsigned short)(byte << 8)));
 }
 
-// One row shared by a 4-lane group (p = lane & 3); returns the reduced sum in
-// every lane of the group.  The row is read in batches of KB steps of 16
-// elements whose loads are all issued before any arithmetic, so a row of
-// 16 * KB * n elements waits on memory n times (a 768-d SQ8 row at KB = 8:
-// 6 times, against 12 at KB = 4); each accumulator still sums its elements
-// in increasing order.  FP32 rows load a float4 per step and use half of KB.
-template <int V, int KB = 8>
-__device__ __forceinline__ float float_row4(const DeviceIndex &ix, const WaveLds &w, const uint8_t *row, int p,
-                                            int32_t mode, int32_t da) {
-    Acc4 acc = {{0.0f, 0.0f, 0.0f, 0.0f}};
-    if (V == V_E5M2_L2 || V == V_E5M2_IP || V == V_SQ8_L2 || V == V_SQ8_IP) {
-        constexpr int kB = KB;  // one code dword per step and lane
-        const int ql = qf_len(ix);
-        const float *m256 = w.qm + ql, *dif = w.qm + 2 * ql;
-        for (int t0 = 0; t0 < da; t0 += 16 * kB) {
-            uint32_t cw[kB];
-#pragma unroll
-            for (int b = 0; b < kB; ++b) {
-                const int t = t0 + 16 * b;
-                cw[b] = t < da ? *(const uint32_t *)(row + t + 4 * p) : 0u;
-            }
-#pragma unroll
-            for (int b = 0; b < kB; ++b) {
-                const int t = t0 + 16 * b;
-                if (t >= da) break;
-                const int j = t + 4 * p;
-                if (V == V_E5M2_L2 || V == V_E5M2_IP) {
-                    const float4 x = *(const float4 *)(w.qf + j);
-                    const float xs[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float y = e5m2_to_float((cw[b] >> (8 * r)) & 0xffu);
-                        if (V == V_E5M2_L2) {
-                            const float d = xs[r] - y;
-                            acc.a[r] = fmaf(d, d, acc.a[r]);
-                        } else {
-                            acc.a[r] = fmaf(xs[r], y, acc.a[r]);
-                        }
-                    }
-                } else {
-                    // SearchImpl2 and initialize_search contexts (in Search too):
-                    // yy = fma(c, dif, 256min), d = 256x - yy.  Search's expansions and a
-                    // bare computer: d = fma(-c, dif, 256x - 256min).  One 16-byte LDS read
-                    // per row and 4 dimensions (every LDS row starts on 16 bytes, j % 4 == 0).
-                    const bool bform = (mode & 3) == MODE_BATCH || (mode & kInitCtx);
-                    const float4 dv = *(const float4 *)(dif + j), mv = *(const float4 *)(m256 + j);
-                    const float4 xv = *(const float4 *)((V == V_SQ8_L2 && !bform ? w.qm : w.qf) + j);
-                    const float dif4[4] = {dv.x, dv.y, dv.z, dv.w}, m4[4] = {mv.x, mv.y, mv.z, mv.w};
-                    const float x4[4] = {xv.x, xv.y, xv.z, xv.w};
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float c = (float)((cw[b] >> (8 * r)) & 0xffu) + 0.5f;
-                        if (V == V_SQ8_L2) {
-                            const float d =
-                                bform ? x4[r] * 256.0f - fmaf(c, dif4[r], m4[r]) : fmaf(-c, dif4[r], x4[r]);
-                            acc.a[r] = fmaf(d, d, acc.a[r]);
-                        } else {
-                            const float yy = fmaf(c, dif4[r], m4[r]);
-                            acc.a[r] = fmaf(x4[r], yy, acc.a[r]);
-                        }
-                    }
-                }
-            }
+constexpr int elt_bytes(int v) {
+    return v == V_FP32_L2 || v == V_FP32_IP ? 4 : (is_f16_variant(v) || is_bf16_variant(v) ? 2 : 1);
+}
+
+// A consecutive elements of a row as they lie in memory, widened on use.
+template <int B>
+struct Raw {
+    uint32_t d[B < 4 ? 1 : B / 4];
+    __device__ __forceinline__ void load(const uint8_t *p) {
+        if (B == 16) {
+            const uint4 x = *(const uint4 *)p;
+            d[0] = x.x;
+            d[1 % (B < 4 ? 1 : B / 4)] = x.y;
+            d[2 % (B < 4 ? 1 : B / 4)] = x.z;
+            d[3 % (B < 4 ? 1 : B / 4)] = x.w;
+        } else if (B == 8) {
+            const uint2 x = *(const uint2 *)p;
+            d[0] = x.x;
+            d[1 % (B < 4 ? 1 : B / 4)] = x.y;
+        } else if (B == 4) {
+            d[0] = *(const uint32_t *)p;
+        } else if (B == 2) {
+            d[0] = *(const uint16_t *)p;
+        } else {
+            d[0] = *p;
         }
-        return reduce16_4lanes<true>(acc);
-    } else {  // FP32, FP16, BF16
-        constexpr bool kWide = V == V_FP32_L2 || V == V_FP32_IP;
-        constexpr int kB = kWide ? KB / 2 : KB;  // 2 KB VGPRs of loads per batch
-        for (int t0 = 0; t0 < da; t0 += 16 * kB) {
-            float4 yv[kB];
-#pragma unroll
-            for (int b = 0; b < kB; ++b) {
-                const int t = t0 + 16 * b;
-                const int j = t + 4 * p;
-                if (t >= da) {
-                    yv[b] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                } else if (kWide) {
-                    yv[b] = *(const float4 *)((const float *)row + j);
-                } else {
-                    yv[b] = widen4<V>(*(const uint2 *)((const uint16_t *)row + j));
-                }
-            }
-#pragma unroll
-            for (int b = 0; b < kB; ++b) {
-                const int t = t0 + 16 * b;
-                if (t >= da) break;
-                const int j = t + 4 * p;
-                const float4 x = *(const float4 *)(w.qf + j);
-                const float xs[4] = {x.x, x.y, x.z, x.w}, ys[4] = {yv[b].x, yv[b].y, yv[b].z, yv[b].w};
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    if (is_l2_float(V)) {
-                        const float d = xs[r] - ys[r];
-                        acc.a[r] = fmaf(d, d, acc.a[r]);
-                    } else {
-                        acc.a[r] = fmaf(xs[r], ys[r], acc.a[r]);
-                    }
-                }
-            }
-        }
-        return reduce16_4lanes<false>(acc);
     }
+};
+
+template <int V, int B>
+__device__ __forceinline__ float widen(const Raw<B> &w, int a) {
+    constexpr int n = B < 4 ? 1 : B / 4;
+    if (elt_bytes(V) == 4) return __uint_as_float(w.d[a % n]);
+    if (elt_bytes(V) == 2) {
+        const uint32_t x = w.d[(a >> 1) % n];
+        if (is_bf16_variant(V)) return __uint_as_float(a & 1 ? x & 0xffff0000u : x << 16);
+        return __half2float(__ushort_as_half((unsigned short)(a & 1 ? x >> 16 : x & 0xffffu)));
+    }
+    const uint32_t x = (w.d[0] >> (8 * a)) & 0xffu;
+    return V == V_E5M2_L2 || V == V_E5M2_IP ? e5m2_to_float(x) : (float)x + 0.5f;
+}
+
+template <int A>
+__device__ __forceinline__ void lds_read(const float *p, float (&x)[A]) {
+    if (A == 4) {
+        const float4 v = *(const float4 *)p;
+        x[0] = v.x;
+        x[1 % A] = v.y;
+        x[2 % A] = v.z;
+        x[3 % A] = v.w;
+    } else if (A == 2) {
+        const float2 v = *(const float2 *)p;
+        x[0] = v.x;
+        x[1 % A] = v.y;
+    } else {
+        x[0] = *p;
+    }
+}
+
+// R rows at a time on each L-lane group (p = lane in the group).  The rows are
+// read in batches of steps of 16 elements, at most VG registers of loads issued
+// before any arithmetic, so a row waits on memory once per batch; the query and
+// the calibration are read from LDS once per step for the R rows.
+template <int V, int L, int R>
+struct FloatRows {
+    static constexpr int A = 16 / L, E = elt_bytes(V), B = A * E;
+    static constexpr int kRegs = R * (B < 4 ? 1 : B / 4);  // per step
+    static constexpr bool kSq8 = V == V_SQ8_L2 || V == V_SQ8_IP;
+    static constexpr bool kL2 = V == V_SQ8_L2 || V == V_E5M2_L2 || is_l2_float(V);
+    float acc[R][A];
+    const uint8_t *at[R];                 // this lane's elements of the next step
+    const float *xq, *qdif, *qmin;        // and its query and calibration
+
+    // `left` steps remain, of which this batch takes up to KB; the loads past
+    // the last one (kAll: there are none) read it again.
+    template <int KB, bool kAll, bool kBform>
+    __device__ __forceinline__ void batch(int32_t left) {
+        Raw<B> raw[R][KB];
+#pragma unroll
+        for (int b = 0; b < KB; ++b) {
+            const int s = kAll || b < left ? b : left - 1;
+#pragma unroll
+            for (int r = 0; r < R; ++r) raw[r][b].load(at[r] + 16 * E * s);
+        }
+#pragma unroll
+        for (int b = 0; b < KB; ++b) {
+            if (!kAll && b >= left) continue;
+            // SQ8 reads three LDS rows: a few steps of them at a time, or
+            // the scheduler brings all of a batch's forward and spills
+            if (kSq8 && b % (8 / A) == 0) __builtin_amdgcn_sched_barrier(0);
+            float x[A], dif[A], m256[A];
+            lds_read<A>(xq + 16 * b, x);
+            if (kSq8) {
+                lds_read<A>(qdif + 16 * b, dif);
+                if (!kL2 || kBform) lds_read<A>(qmin + 16 * b, m256);
+            }
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int a = 0; a < A; ++a) {
+                    const float y = widen<V, B>(raw[r][b], a);
+                    if (kSq8 && kL2) {
+                        const float d = kBform ? x[a] * 256.0f - fmaf(y, dif[a], m256[a]) : fmaf(-y, dif[a], x[a]);
+                        acc[r][a] = fmaf(d, d, acc[r][a]);
+                    } else if (kSq8) {
+                        acc[r][a] = fmaf(x[a], fmaf(y, dif[a], m256[a]), acc[r][a]);
+                    } else if (kL2) {
+                        const float d = x[a] - y;
+                        acc[r][a] = fmaf(d, d, acc[r][a]);
+                    } else {
+                        acc[r][a] = fmaf(x[a], y, acc[r][a]);
+                    }
+                }
+        }
+    }
+
+    // The last `left` < 2 KB steps in the smallest batch that holds them.
+    template <int KB, bool kBform>
+    __device__ __forceinline__ void tail(int32_t left) {
+        if constexpr (KB > 2) {
+            if (left <= KB / 2) return tail<KB / 2, kBform>(left);
+        }
+        batch<KB, false, kBform>(left);
+    }
+
+    template <int KB, bool kBform>
+    __device__ __forceinline__ void steps(int32_t left) {
+        for (; left >= KB; left -= KB) {
+            batch<KB, true, kBform>(left);
+#pragma unroll
+            for (int r = 0; r < R; ++r) at[r] += 16 * E * KB;
+            xq += 16 * KB;
+            qdif += 16 * KB;
+            qmin += 16 * KB;
+        }
+        if (left > 0) tail<KB, kBform>(at_use(left));
+    }
+
+    // Distances of rows row[0..R); out[r] is valid in the group's first lane.
+    template <int VG>
+    __device__ __forceinline__ void run(const DeviceIndex &ix, const WaveLds &w, const uint8_t *const (&row)[R], int p,
+                                        int32_t mode, int32_t da, float (&out)[R]) {
+        constexpr int KB = VG / kRegs >= 32 ? 32 : VG / kRegs >= 16 ? 16 : VG / kRegs >= 8 ? 8 : VG / kRegs >= 4 ? 4 : 2;
+        const int ql = qf_len(ix);
+        // SQ8: SearchImpl2 and initialize_search contexts (in Search too): yy =
+        // fma(c, dif, 256min), d = 256x - yy.  Search's expansions and a bare
+        // computer: d = fma(-c, dif, 256x - 256min).
+        const bool bform = (mode & 3) == MODE_BATCH || (mode & kInitCtx);
+        xq = (V == V_SQ8_L2 && !bform ? w.qm : w.qf) + A * p;
+        qmin = w.qm + ql + A * p;
+        qdif = w.qm + 2 * ql + A * p;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            at[r] = row[r] + A * E * p;
+#pragma unroll
+            for (int a = 0; a < A; ++a) acc[r][a] = 0.0f;
+        }
+        if (V == V_SQ8_L2 && !bform) {
+            steps<KB, false>(da / 16);
+        } else {
+            steps<KB, true>(da / 16);
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) out[r] = reduce16<L, E == 1>(acc[r]);
+    }
+};
+
+template <int V, int L, int R, int VG>
+__device__ __forceinline__ void float_rows(const DeviceIndex &ix, const WaveLds &w, const uint8_t *const (&row)[R],
+                                           int p, int32_t mode, int32_t da, float (&out)[R]) {
+    FloatRows<V, L, R> f;
+    f.template run<VG>(ix, w, row, p, mode, da, out);
 }
 
 // SQ6 codes (SQ6Quantizer::encode_component, glass/quant/sq6_quant.hpp:41-62):
@@ -693,7 +797,7 @@ __device__ __forceinline__ float sq4_row4(const DeviceIndex &ix, const WaveLds &
 // the loop has no branches): each 4-lane group takes R rows per pass
 // (entries base + 16r + g) and issues every load of the pass before any
 // arithmetic, so a pass waits on memory once; each accumulator still sums
-// its elements in increasing order, as float_row4 does.
+// its elements in increasing order, as float_rows does.
 template <int VF, int R, int S>
 __device__ void rerank_rows(const DeviceIndex &ix, const WaveLds &w, int m) {
     constexpr bool kHalf = is_f16_variant(VF);
@@ -722,9 +826,11 @@ __device__ void rerank_rows(const DeviceIndex &ix, const WaveLds &w, int m) {
 #pragma unroll
                 for (int s = 0; s < S; ++s) y[r][s] = widen4<VF>(h[r][s]);
         }
-        Acc4 acc[R];
+        float acc[R][4];
 #pragma unroll
-        for (int r = 0; r < R; ++r) acc[r] = Acc4{{0.0f, 0.0f, 0.0f, 0.0f}};
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[r][e] = 0.0f;
 #pragma unroll
         for (int s = 0; s < S; ++s) {
             const float4 x = *(const float4 *)(w.qf + 16 * s + 4 * p4);
@@ -736,16 +842,16 @@ __device__ void rerank_rows(const DeviceIndex &ix, const WaveLds &w, int m) {
                 for (int e = 0; e < 4; ++e) {
                     if (is_l2_float(VF)) {
                         const float d = xs[e] - ys[e];
-                        acc[r].a[e] = fmaf(d, d, acc[r].a[e]);
+                        acc[r][e] = fmaf(d, d, acc[r][e]);
                     } else {
-                        acc[r].a[e] = fmaf(xs[e], ys[e], acc[r].a[e]);
+                        acc[r][e] = fmaf(xs[e], ys[e], acc[r][e]);
                     }
                 }
             }
         }
         float rs[R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) rs[r] = reduce16_4lanes<false>(acc[r]);
+        for (int r = 0; r < R; ++r) rs[r] = reduce16<4, false>(acc[r]);
         wave_sync();
         if (p4 == 0) {
 #pragma unroll
@@ -811,7 +917,7 @@ __device__ __forceinline__ void rerank_sq8u(const DeviceIndex &ix, const WaveLds
 // are rebuilt from the re-rank calibration and each row goes through the SQ8
 // kernel in the bare computer's rounding (glass::L2SqrSQ8_ext / IPSQ8_ext).
 // General path only, as rerank_sq8u.
-template <int VS, int KB>
+template <int VS, int VG>
 __device__ __forceinline__ void rerank_sq8(const DeviceIndex &ix, const WaveLds &w, int m) {
     const int l = lane_id();
     const int ql = qf_len(ix);
@@ -828,17 +934,18 @@ __device__ __forceinline__ void rerank_sq8(const DeviceIndex &ix, const WaveLds 
     for (int base = 0; base < m; base += 16) {
         const int j = base + g;
         const uint32_t id = w.pid[j < m ? j : m - 1] & kIdMask;
-        const uint8_t *row = (const uint8_t *)ix.rerank + (int64_t)id * ix.r_code_size;
-        const float r = float_row4<VS, KB>(ix, w, row, p4, MODE_SEARCH, ix.r_dim_align);
+        const uint8_t *row[1] = {(const uint8_t *)ix.rerank + (int64_t)id * ix.r_code_size};
+        float r[1];
+        float_rows<VS, 4, 1, VG>(ix, w, row, p4, MODE_SEARCH, ix.r_dim_align, r);
         wave_sync();
-        if (j < m && p4 == 0) w.pk[j] = key_of_float(VS == V_SQ8_IP ? -r : r);
+        if (j < m && p4 == 0) w.pk[j] = key_of_float(VS == V_SQ8_IP ? -r[0] : r[0]);
         wave_sync();
     }
 }
 
 // Exact distances of pool entries [0, m) into pk; rows longer than 128
-// values go through float_row4, one row per 4-lane group per pass.
-template <int VF, int KB>
+// values go through float_rows, one row per 4-lane group per pass.
+template <int VF, int VG>
 __device__ __forceinline__ void rerank(const DeviceIndex &ix, const WaveLds &w, int m) {
     const int da = ix.r_dim_align;  // a multiple of 16
     switch (da) {
@@ -857,10 +964,11 @@ __device__ __forceinline__ void rerank(const DeviceIndex &ix, const WaveLds &w, 
     for (int base = 0; base < m; base += 16) {
         const int j = base + g;
         const uint32_t id = w.pid[j < m ? j : m - 1] & kIdMask;
-        const uint8_t *row = (const uint8_t *)ix.rerank + (int64_t)id * da * (is_f16_variant(VF) ? 2 : 4);
-        const float rsum = float_row4<VF, KB>(ix, w, row, p4, MODE_BATCH, da);
+        const uint8_t *row[1] = {(const uint8_t *)ix.rerank + (int64_t)id * da * (is_f16_variant(VF) ? 2 : 4)};
+        float r[1];
+        float_rows<VF, 4, 1, VG>(ix, w, row, p4, MODE_BATCH, da, r);
         wave_sync();
-        if (j < m && p4 == 0) w.pk[j] = key_of_float(is_l2_float(VF) ? rsum : -rsum);
+        if (j < m && p4 == 0) w.pk[j] = key_of_float(is_l2_float(VF) ? r[0] : -r[0]);
         wave_sync();
     }
 }
@@ -925,30 +1033,85 @@ __device__ __forceinline__ float pq_row4(const DeviceIndex &ix, const float *lut
     return r;
 }
 
-template <int V, int KB = 8>
+// Candidates base + L-lane group of this wave (first, of 64 / L rows per wave)
+// and, with R = 2, the one `second` further on.
+template <int V, int L, int R, int VG>
+__device__ __forceinline__ void float_pass(const DeviceIndex &ix, const WaveLds &w, int base, int m, int second,
+                                           int32_t mode) {
+    constexpr bool neg = V == V_E5M2_IP || V == V_SQ8_IP || V == V_FP32_IP || V == V_FP16_IP || V == V_BF16_IP;
+    const int p = lane_id() & (L - 1), j = base + lane_id() / L;
+    const uint8_t *row[R];
+    float d[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int jr = j + r * second;
+        row[r] = ix.codes + (int64_t)w.ci[jr < m ? jr : m - 1] * ix.code_size;
+    }
+    float_rows<V, L, R, VG>(ix, w, row, p, mode, ix.dim_align, d);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int jr = j + r * second;
+        if (jr < m && p == 0) w.ck[jr] = key_of_float(neg ? -d[r] : d[r]);
+    }
+}
+
+// Distances of candidates ci[0..m) -> keys ck[0..m).  A wave alone takes 32
+// rows at 4 lanes each, two rows per group, while more than 24 are left: the
+// query and calibration reads from LDS, which bound long SQ8 rows, are shared
+// by the two.  Fewer rows get more lanes each (16 rows x 4, 8 x 8, 4 x 16), so
+// a pass is as short as its rows are few: a lane's arithmetic is 1 / 2 or 1 / 4
+// of a 4-lane pass.  Waves that share a query take the most lanes per row that
+// do all rows in one pass.  With 4 lanes per row and 4 loads in flight always,
+// and with this (us per batch of 8,192, ef 64): 100k x 768 SQ8 IP 4,890 and
+// 3,753; 200k x 100 FP16 IP 1,110 and 767; 200k x 128 FP32 L2 820 and 635.
+template <int V, int VG>
 __device__ __forceinline__ void float_distances(const DeviceIndex &ix, const WaveLds &w, int m, int32_t mode,
                                                 const float *lut, int first = 0, int stride = 1) {
     if (m <= 0) return;
-    const int l = lane_id();
-    const int p = l & 3, cj = l >> 2;
-    for (int base = 16 * first; base < m; base += 16 * stride) {
-        const int j = base + cj;
-        const int jj = j < m ? j : (m - 1);
-        const uint32_t id = w.ci[jj];
-        const uint8_t *row = ix.codes + (int64_t)id * ix.code_size;
-        float r;
-        if (V == V_SQ6_L2 || V == V_SQ6_IP) {
-            r = sq6_row4<V>(ix, w, row, p, mode, ix.dim_align);
-        } else if (V == V_SQ4_L2 || V == V_SQ4_IP) {
-            r = sq4_row4<V>(ix, w, row, p, ix.dim_align);
-        } else if (is_pq_variant(V)) {
-            r = pq_row4<V>(ix, lut, row, p);  // IP entries are already negated dot products
-        } else {
-            r = float_row4<V, KB>(ix, w, row, p, mode, ix.dim_align);
+    if (V == V_SQ6_L2 || V == V_SQ6_IP || V == V_SQ4_L2 || V == V_SQ4_IP || is_pq_variant(V)) {
+        const int l = lane_id();
+        const int p = l & 3, cj = l >> 2;
+        for (int base = 16 * first; base < m; base += 16 * stride) {
+            const int j = base + cj;
+            const int jj = j < m ? j : (m - 1);
+            const uint32_t id = w.ci[jj];
+            const uint8_t *row = ix.codes + (int64_t)id * ix.code_size;
+            float r;
+            if (V == V_SQ6_L2 || V == V_SQ6_IP) {
+                r = sq6_row4<V>(ix, w, row, p, mode, ix.dim_align);
+            } else if (V == V_SQ4_L2 || V == V_SQ4_IP) {
+                r = sq4_row4<V>(ix, w, row, p, ix.dim_align);
+            } else {
+                r = pq_row4<V>(ix, lut, row, p);  // IP entries are already negated dot products
+            }
+            const bool neg = V == V_SQ6_IP || V == V_SQ4_IP;
+            if (j < m && p == 0) w.ck[j] = key_of_float(neg ? -r : r);
         }
-        bool neg = (V == V_E5M2_IP || V == V_SQ8_IP || V == V_FP32_IP || V == V_FP16_IP || V == V_BF16_IP ||
-                    V == V_SQ6_IP || V == V_SQ4_IP);
-        if (j < m && p == 0) w.ck[j] = key_of_float(neg ? -r : r);
+    } else if (stride > 1) {
+        if (m <= 4 * stride) {
+            if (4 * first < m) float_pass<V, 16, 1, VG>(ix, w, 4 * first, m, 0, mode);
+        } else if (m <= 8 * stride) {
+            if (8 * first < m) float_pass<V, 8, 1, VG>(ix, w, 8 * first, m, 0, mode);
+        } else {
+            for (int base = 16 * first; base < m; base += 16 * stride) float_pass<V, 4, 1, VG>(ix, w, base, m, 0, mode);
+        }
+    } else {
+        for (int base = 0; base < m;) {
+            const int rem = m - base;
+            if (rem > 24) {
+                float_pass<V, 4, 2, VG>(ix, w, base, m, 16, mode);
+                base += 32;
+            } else if (rem > 8) {
+                float_pass<V, 4, 1, VG>(ix, w, base, m, 0, mode);
+                base += 16;
+            } else if (rem > 4) {
+                float_pass<V, 8, 1, VG>(ix, w, base, m, 0, mode);
+                base += 8;
+            } else {
+                float_pass<V, 16, 1, VG>(ix, w, base, m, 0, mode);
+                base += 4;
+            }
+        }
     }
 }
 
@@ -1502,14 +1665,13 @@ __device__ __forceinline__ void put_result(const QueryBatch &qb, int64_t pos, in
 // 128 VGPRs; left to itself the compiler schedules the re-rank's loads into
 // more registers than that).  The general path runs at 3 (168 VGPRs): its
 // pools, long rows and visited bookkeeping spill at 128, and its launches are
-// mostly held to fewer waves by LDS anyway.  The shared-query path runs at 3
-// too: at 2, a batch of 1,000 queries at 4 waves each does not fit the device
-// in one round (it spills at 128).  Of the instances with 16 dwords per lane,
-// SQ2U and SQ4U shared queries spill at 168 and run at 2, and SQ2U's common
-// path spills at 128 and runs at 3.
+// mostly held to fewer waves by LDS anyway.  The shared-query path runs at 2:
+// it is for batches that leave wave slots idle.  SQ2U's common path with 16
+// dwords per lane spills at 128 and runs at 3, and so does SQ8's, which keeps
+// two rows, the query and two calibration rows in flight.
 template <int V, int DPL, int P>
-constexpr int kWavesPerEu = P == 1 ? (V == V_SQ2U && DPL == 16 ? 3 : 4)
-                                   : ((P == 2 && (V == V_SQ2U || V == V_SQ4U) && DPL == 16) ? 2 : 3);
+constexpr int kWavesPerEu =
+    P == 1 ? ((V == V_SQ2U && DPL == 16) || V == V_SQ8_L2 || V == V_SQ8_IP ? 3 : 4) : (P == 2 ? 2 : 3);
 
 template <int V, int DPL, int P>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<V, DPL, P>))) void search_kernel(DeviceIndex ix,
@@ -1517,6 +1679,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu
                                                                                             LaunchConfig lc,
                                                                                             SlotState ss) {
     constexpr bool kFast = P == 1;
+    // registers of float rows' loads in flight, in the search and in the re-rank of long rows
+    constexpr bool kSq8 = V == V_SQ8_L2 || V == V_SQ8_IP;  // its LDS rows take registers too
+    constexpr int kRowRegs = kSq8 ? (P == 2 ? 32 : 16) : (P == 1 ? 16 : (P == 2 ? 64 : 32));
+    constexpr int kRerankRegs = P == 1 ? 32 : 48;
+    // passes of integer code rows in flight at once, as the register budget allows
+    constexpr int kAhead = DPL == 16 && (P == 1 || (P == 0 && V == V_SQ2U)) ? 1 : 2;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     const int l = lane_id();
     const int wv = threadIdx.x >> 6;
@@ -1630,9 +1798,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu
 
         auto dists = [&](int m, int32_t mode) __attribute__((always_inline)) {
             if (is_int_variant(V)) {
-                iq.distances(ix, w, m);
+                iq.template distances<kAhead>(ix, w, m);
             } else {
-                float_distances<V, kFast ? 4 : 8>(ix, w, m, mode, lut);
+                float_distances<V, kRowRegs>(ix, w, m, mode, lut);
             }
             wave_sync();
         };
@@ -1768,9 +1936,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu
                 const int m = uni(ctl[1]);
                 if (m < 0) break;
                 if (is_int_variant(V)) {
-                    iq.distances(ix, w, m, wv, W);
+                    iq.template distances<kAhead>(ix, w, m, wv, W);
                 } else {
-                    float_distances<V>(ix, w, m, qb.mode, lut, wv, W);
+                    float_distances<V, kRowRegs>(ix, w, m, qb.mode, lut, wv, W);
                 }
                 __syncthreads();
                 if (lead) {
@@ -1914,9 +2082,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu
             const int m = kk < ps.size ? kk : ps.size;
             if (ix.rerank_kind == QK_FP16) {
                 if (ix.metric == MK_L2) {
-                    rerank<V_FP16_L2, kFast ? 4 : 8>(ix, w, m);
+                    rerank<V_FP16_L2, kRerankRegs>(ix, w, m);
                 } else {
-                    rerank<V_FP16_IP, kFast ? 4 : 8>(ix, w, m);
+                    rerank<V_FP16_IP, kRerankRegs>(ix, w, m);
                 }
             } else if (!kFast && ix.rerank_kind == QK_SQ8U) {
                 if (ix.metric == MK_L2) {
@@ -1926,14 +2094,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu
                 }
             } else if (!kFast && ix.rerank_kind == QK_SQ8) {
                 if (ix.metric == MK_L2) {
-                    rerank_sq8<V_SQ8_L2, kFast ? 4 : 8>(ix, w, m);
+                    rerank_sq8<V_SQ8_L2, 8>(ix, w, m);
                 } else {
-                    rerank_sq8<V_SQ8_IP, kFast ? 4 : 8>(ix, w, m);
+                    rerank_sq8<V_SQ8_IP, 8>(ix, w, m);
                 }
             } else if (ix.metric == MK_L2) {
-                rerank<V_FP32_L2, kFast ? 4 : 8>(ix, w, m);
+                rerank<V_FP32_L2, kRerankRegs>(ix, w, m);
             } else {
-                rerank<V_FP32_IP, kFast ? 4 : 8>(ix, w, m);
+                rerank<V_FP32_IP, kRerankRegs>(ix, w, m);
             }
             wave_sync();
             // Ranks by (dist, id), with equal pairs (a repeated entry point
