@@ -274,7 +274,7 @@ struct glass_hip_searcher {
         // SQ4U, ef 64, 8,192 queries: 462 / 467 / 481 us per batch).
         int32_t team = 8, waves_per_block = 1, vis_hash = 0;
         int32_t spec = 1;  // integer codes: gather all neighbours' rows before the visited test
-        int32_t qwaves_small = 1;  // waves per query for batches that leave wave slots idle
+        int32_t qwaves_small = 0;  // waves per query for batches that leave wave slots idle (0: untuned_qwaves)
     };
     static constexpr int kBuckets = 7;  // ef <= 16, 32, 64, 128, 256, 512, larger
     Tune tune[kBuckets];
@@ -819,6 +819,24 @@ int32_t round_cap(int32_t cap) { return (std::max(cap, 1) + 15) / 16 * 16; }
 // LDS of one CU (CDNA4: 160 KiB); a workgroup's per-wave areas must fit it.
 constexpr size_t kLdsPerCu = 160 * 1024;
 
+// Waves per query, at most, of a small batch that nothing has tuned.  Waves
+// that share a query share an expansion's distances and pay two barriers for
+// it, so it is the bytes of a node's neighbour rows that decide.  Measured at
+// 64 queries, ef 128 (us per batch at 1, 2, 4 and 8 waves): 768-d SQ8, 36 KB
+// per expansion, 983 / 832 / 543 / 456; 960-d SQ8U, 61 KB, 600 / 416 / 297 /
+// 237; 300-d FP16, 29 KB, 362 / 332 / 296 / 288; 960-d SQ4U, 16 KB, 271 / 238 /
+// 218 / 210 (its rows do not fit the all-neighbour gather); 128-d FP32, 16 KB,
+// 286 / 318 / 313 / 305; 128-d SQ8U, 4 KB, 171 / 259 / 260 / 248.  SQ6's and
+// PQ8's rows cost more than their bytes: 200-d SQ6 780 / 684 / 686 / 662, 96-d
+// PQ8 325 / 273 / 274 / 257.
+int32_t untuned_qwaves(const glass_hip_searcher &s, int32_t team) {
+    if (s.quant == QK_SQ6 || s.quant == QK_PQ8) return 2;
+    const int64_t bytes = (int64_t)s.graph.K * s.code_size;
+    if (bytes >= 24 << 10) return 8;
+    const bool int_codes = s.quant == QK_SQ8U || s.quant == QK_SQ4U || s.quant == QK_SQ2U;
+    return int_codes && bytes >= 12 << 10 && !spec_fits(s, team) ? 4 : 1;
+}
+
 // Visited-set words of a launch that nothing has tuned: the most that cost no
 // resident wave the batch has a query for.  LDS per wave, most of it these
 // words, decides how many waves a CU holds, and waves in flight are what hides
@@ -907,7 +925,8 @@ int run_batch(glass_hip_searcher &s, const float *qs_dev, int32_t nq, const int3
         // round (1M x 960, ef 16-512 and k 1-100 per query, 1,000 queries:
         // 4 waves per query in 1.3 rounds, 4.30 ms, against 2 waves in one
         // round, 5.04 ms; with ef 256 for every query the 1.3 rounds lose).
-        const int32_t want = s.force_qwaves ? s.force_qwaves : tn.qwaves_small;
+        const int32_t want =
+            s.force_qwaves ? s.force_qwaves : (tn.qwaves_small ? tn.qwaves_small : untuned_qwaves(s, lc.team));
         const int64_t rounds = ef_dev ? 2 : 1;
         if (want > 1 && s.graph.K <= 64) {
             int32_t qw = want;
@@ -921,6 +940,11 @@ int run_batch(glass_hip_searcher &s, const float *qs_dev, int32_t nq, const int3
                     return (int64_t)std::max(1, max_blocks_per_cu(s.index(), mw)) * std::max(1, s.cu_count);
                 };
                 while (qw > 1 && (int64_t)nq > rounds * resident_queries(qw)) qw /= 2;
+                // 8 waves fill a CU: a batch on a caller's stream that would
+                // take more than half of them leaves the next one no room
+                // (256 queries, 960-d SQ8U, ef 128, over two streams: 448 us
+                // per batch at 8 waves, 348 at 4)
+                if (qw == 8 && !alone && 2 * (int64_t)nq > resident_queries(8)) qw = 4;
             }
             if (qw > 1) {
                 lc.qwaves = qw;
@@ -1701,7 +1725,7 @@ int glass_hip_searcher_set_query_waves(glass_hip_searcher *s, int32_t waves) {
 int glass_hip_searcher_get_query_waves(const glass_hip_searcher *s, int32_t *last, int32_t *tuned) {
     if (!s) return fail(GLASS_HIP_EINVAL, "null searcher");
     if (last) *last = s->last_launch.qwaves > 1 ? s->last_launch.qwaves : 1;
-    if (tuned) *tuned = s->tune[glass_hip_searcher::bucket(s->ef)].qwaves_small;
+    if (tuned) *tuned = std::max(1, s->tune[glass_hip_searcher::bucket(s->ef)].qwaves_small);
     return GLASS_HIP_OK;
 }
 

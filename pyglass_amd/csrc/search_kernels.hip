@@ -1674,7 +1674,7 @@ constexpr int kWavesPerEu =
     P == 1 ? ((V == V_SQ2U && DPL == 16) || V == V_SQ8_L2 || V == V_SQ8_IP ? 3 : 4) : (P == 2 ? 2 : 3);
 
 template <int V, int DPL, int P>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<V, DPL, P>))) void search_kernel(DeviceIndex ix,
+__global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<V, DPL, P>))) void search_kernel(DeviceIndex ix,
                                                                                             QueryBatch qb,
                                                                                             LaunchConfig lc,
                                                                                             SlotState ss) {
