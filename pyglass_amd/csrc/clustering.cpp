@@ -19,6 +19,7 @@
 #include <cstdio>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <random>
 #include <string>
 #include <vector>
@@ -273,44 +274,53 @@ int fit_device(const float *rows, int32_t n, int32_t d, int32_t k, int32_t epoch
     return GLASS_HIP_OK;
 }
 
+// A clustering object's stream and events, made at first use and kept with it (making one
+// takes 0.5 ms); one call at a time.
+struct Device {
+    std::mutex mu;
+    hipStream_t stream = nullptr;
+    hipEvent_t done[2] = {nullptr, nullptr};
+    ~Device() {
+        for (hipEvent_t e : done)
+            if (e) (void)hipEventDestroy(e);
+        if (stream) (void)hipStreamDestroy(stream);
+    }
+};
+
 // Nearest centroid of every row.  Rows go to the device in pieces of about
 // 16 MB while the piece before is worked on: the copy bounds the call.
-int predict_device(const float *cent, int32_t k, int32_t d, const float *x, int32_t n, int32_t *ids) {
+int predict_device(Device &dev, const float *cent, int32_t k, int32_t d, const float *x, int32_t n, int32_t *ids) {
     const int64_t piece = std::max<int64_t>(64, ((int64_t)4 << 20) / d / 64 * 64);
     const int32_t rows = (int32_t)std::min<int64_t>(n, piece);
     const int32_t bufs = n > rows ? 2 : 1;
+    if (!dev.stream) CL_TRY(hipStreamCreateWithFlags(&dev.stream, hipStreamNonBlocking));
+    for (hipEvent_t &e : dev.done)
+        if (!e) CL_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     Arena a;
     const size_t o_x = a.add(4 * (size_t)rows * d * bufs), o_cent = a.add(4 * (size_t)k * d),
                  o_ids = a.add(4 * (size_t)n), o_scratch = a.add(AssignScratch::bytes(rows, k));
     CL_TRY(a.alloc());
-    struct Lane {
-        hipStream_t stream = nullptr;
-        hipEvent_t done[2] = {nullptr, nullptr};
-        ~Lane() {
-            if (stream) (void)hipStreamSynchronize(stream);
-            for (hipEvent_t e : done)
-                if (e) (void)hipEventDestroy(e);
-            if (stream) (void)hipStreamDestroy(stream);
-        }
-    } ln;
-    CL_TRY(hipStreamCreateWithFlags(&ln.stream, hipStreamNonBlocking));
-    for (int32_t b = 0; b < bufs; ++b) CL_TRY(hipEventCreateWithFlags(&ln.done[b], hipEventDisableTiming));
+    struct Drain {  // before the arena goes
+        hipStream_t s;
+        ~Drain() { (void)hipStreamSynchronize(s); }
+    } drain{dev.stream};
     float *dc = a.at<float>(o_cent);
     int32_t *di = a.at<int32_t>(o_ids);
     AssignScratch s;
     CL_TRY(hipMemcpy(dc, cent, 4 * (size_t)k * d, hipMemcpyHostToDevice));
-    int32_t b = 0, turn = 0;
-    for (int64_t at = 0; at < n; at += rows, b ^= bufs - 1, ++turn) {
+    int32_t turn = 0;
+    for (int64_t at = 0; at < n; at += rows, ++turn) {
         const int32_t c = (int32_t)std::min<int64_t>(rows, n - at);
+        const int32_t b = turn % bufs;
         float *dx = a.at<float>(o_x) + (size_t)b * rows * d;
-        if (turn >= bufs) CL_TRY(hipEventSynchronize(ln.done[b]));
+        if (turn >= 2) CL_TRY(hipEventSynchronize(dev.done[b]));
         CL_TRY(hipMemcpy(dx, x + at * d, 4 * (size_t)c * d, hipMemcpyHostToDevice));
         s.place(a.p + o_scratch, c, k);
-        CL_TRY(launch_cluster_norms(dx, c, d, s, ln.stream));
-        CL_TRY(launch_cluster_assign(dx, c, d, dc, k, di + at, s, ln.stream));
-        CL_TRY(hipEventRecord(ln.done[b], ln.stream));
+        CL_TRY(launch_cluster_norms(dx, c, d, s, dev.stream));
+        CL_TRY(launch_cluster_assign(dx, c, d, dc, k, di + at, s, dev.stream));
+        CL_TRY(hipEventRecord(dev.done[b], dev.stream));
     }
-    CL_TRY(hipStreamSynchronize(ln.stream));
+    CL_TRY(hipStreamSynchronize(dev.stream));
     CL_TRY(hipMemcpy(ids, di, 4 * (size_t)n, hipMemcpyDeviceToHost));
     return GLASS_HIP_OK;
 }
@@ -324,6 +334,7 @@ struct glass_hip_clustering {
     int32_t k = 0, epochs = 10, dim = 0;
     bool kmeanspp = false;
     std::vector<float> centroids;
+    mutable Device dev;
 };
 
 extern "C" {
@@ -375,7 +386,8 @@ int glass_hip_clustering_predict(const glass_hip_clustering *c, const float *dat
             return set_error(GLASS_HIP_EINVAL, msg);
         }
         if (n == 0) return GLASS_HIP_OK;
-        return predict_device(c->centroids.data(), c->k, dim, data, n, ids);
+        std::lock_guard<std::mutex> lk(c->dev.mu);
+        return predict_device(c->dev, c->centroids.data(), c->k, dim, data, n, ids);
     } catch (...) {
         return exception_status();
     }

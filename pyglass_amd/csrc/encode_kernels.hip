@@ -141,6 +141,41 @@ __global__ void pad_rows_kernel(const float *data, int64_t n, int32_t dim, int32
     }
 }
 
+// Graph rows as the search expects them: each cut at its first -1, later
+// repetitions of an id removed (a repeated id is skipped by the visited test in
+// SearchImpl1/2, so dropping it leaves the visit order unchanged), the rest -1.
+// One wave per row of at most 128 entries, two per lane: every entry is
+// compared with the ones before it by a lane broadcast each, and a row that is
+// tidy already is not written.  One read of the graph: 500k x 32, 0.06 ms,
+// where sorting every row on 16 host threads took 14 ms.
+__global__ __launch_bounds__(256) void tidy_rows_kernel(int32_t *adj, int64_t n, int32_t k) {
+    const int l = threadIdx.x & 63;
+    for (int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); i < n; i += (int64_t)gridDim.x * 4) {
+        int32_t *row = adj + i * k;
+        const int32_t a = l < k ? row[l] : -1, b = l + 64 < k ? row[l + 64] : -1;
+        const unsigned long long ea = __ballot(a == -1), eb = __ballot(b == -1);
+        const int len = ea ? __builtin_ctzll(ea) : (eb ? 64 + __builtin_ctzll(eb) : 128);
+        bool ra = false, rb = false;  // repeats an entry before it
+        for (int j = 0; j < len && j < 64; ++j) {
+            const int32_t v = __builtin_amdgcn_readlane(a, j);
+            ra |= a == v && j < l;
+            rb |= b == v;
+        }
+        for (int j = 64; j < len; ++j) {
+            const int32_t v = __builtin_amdgcn_readlane(b, j - 64);
+            rb |= b == v && j - 64 < l;
+        }
+        const bool ka = l < len && !ra, kb = l + 64 < len && !rb;
+        const unsigned long long ma = __ballot(ka), mb = __ballot(kb), below = (1ull << l) - 1ull;
+        const int na = __popcll(ma), kept = na + __popcll(mb);
+        if (kept == len && !__ballot((l >= len && a != -1) || (l + 64 >= len && b != -1))) continue;
+        if (ka) row[__popcll(ma & below)] = a;
+        if (kb) row[na + __popcll(mb & below)] = b;
+        if (l >= kept && l < k) row[l] = -1;
+        if (l + 64 >= kept && l + 64 < k) row[l + 64] = -1;
+    }
+}
+
 __global__ void fill_i32_kernel(int32_t *p, int64_t n, int32_t v) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         p[i] = v;
@@ -246,6 +281,13 @@ hipError_t launch_radix_pick(int32_t ntargets, int32_t shift, const unsigned lon
                              unsigned long long *rank, hipStream_t stream) {
     hipLaunchKernelGGL(radix_pick_kernel, dim3((ntargets + 255) / 256), dim3(256), 0, stream, ntargets, shift, hist,
                        prefix, rank);
+    return hipGetLastError();
+}
+
+hipError_t launch_tidy_rows(int32_t *adj, int64_t n, int32_t k, hipStream_t stream) {
+    const int64_t blocks = (n + 3) / 4;
+    hipLaunchKernelGGL(tidy_rows_kernel, dim3((unsigned)(blocks < 65536 ? blocks : 65536)), dim3(256), 0, stream, adj, n,
+                       k);
     return hipGetLastError();
 }
 

@@ -6,6 +6,7 @@
 // drives the HIP search kernels.  Searcher semantics follow
 // glass/searcher/graph_searcher.hpp and glass/searcher/refiner.hpp.
 #include <hip/hip_runtime.h>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <atomic>
@@ -30,6 +31,7 @@
 
 #include "../../include/glass_hip.h"
 #include "glass_hip_internal.h"
+#include "staging.h"
 
 namespace glass_hip {
 hipError_t launch_encode(const float *data_dev, int64_t n, int32_t dim, int32_t code_size, int32_t quant,
@@ -38,6 +40,7 @@ hipError_t launch_encode(const float *data_dev, int64_t n, int32_t dim, int32_t 
 hipError_t launch_pad_rows(const float *data_dev, int64_t n, int32_t dim, int32_t dim_align, float *out,
                            hipStream_t stream);
 hipError_t launch_fill_i32(int32_t *p, int64_t n, int32_t v, hipStream_t stream);
+hipError_t launch_tidy_rows(int32_t *adj, int64_t n, int32_t k, hipStream_t stream);
 hipError_t launch_radix_hist(const float *data, int32_t nseg, int64_t seg_len, int64_t seg_stride, int32_t absval,
                              int32_t shift, const uint32_t *prefix, unsigned long long *hist, hipStream_t stream);
 hipError_t launch_pq_encode(const float *data_dev, int64_t n, int32_t nsq, const float *codebook, uint8_t *codes_dev,
@@ -205,9 +208,79 @@ void glass_hip::gen_random(std::mt19937 &rng, int32_t *addr, int32_t size, int32
     for (int32_t i = 0; i < size; ++i) addr[i] = (addr[i] + off) % N;
 }
 
+namespace {
+
+// fn(lo, hi) over [0, n) in up to 16 pieces of at least `least`, one host
+// thread each; pieces no thread could be started for run here.
+template <typename Fn>
+void parallel_pieces(int64_t n, int64_t least, const Fn &fn) {
+    const int64_t nt = std::min<int64_t>({16, (int64_t)std::max(1u, std::thread::hardware_concurrency()), n / least});
+    if (nt <= 1) return fn((int64_t)0, n);
+    const int64_t chunk = (n + nt - 1) / nt;
+    std::vector<std::thread> th;
+    th.reserve(nt);
+    int64_t lo = chunk;
+    try {
+        for (; lo < n; lo += chunk) th.emplace_back(fn, lo, std::min(n, lo + chunk));
+    } catch (const std::system_error &) {
+    }
+    fn((int64_t)0, std::min(n, chunk));
+    if (lo < n) fn(lo, n);
+    for (auto &t : th) t.join();
+}
+
+// The graph's rows: storage left uninitialised until it is written, in huge
+// pages where it is large, so that filling it is not one page fault per 4 KB
+// (64 MB of rows copied into a vector: 14 ms; by 16 threads into this: 2 ms).
+class Rows {
+public:
+    Rows() = default;
+    Rows(Rows &&o) noexcept : p_(o.p_), n_(o.n_) {
+        o.p_ = nullptr;
+        o.n_ = 0;
+    }
+    Rows &operator=(Rows &&o) noexcept {
+        std::swap(p_, o.p_);
+        std::swap(n_, o.n_);
+        return *this;
+    }
+    ~Rows() { std::free(p_); }
+    void resize(size_t n) {  // the contents are lost
+        constexpr size_t kHuge = (size_t)2 << 20;
+        const size_t bytes = std::max<size_t>(n, 1) * sizeof(int32_t);
+        std::free(p_);
+        n_ = 0;
+        p_ = (int32_t *)(bytes < kHuge ? std::malloc(bytes) : std::aligned_alloc(kHuge, (bytes + kHuge - 1) / kHuge * kHuge));
+        if (!p_) throw std::bad_alloc();
+        if (bytes >= kHuge) (void)madvise(p_, bytes, MADV_HUGEPAGE);
+        n_ = n;
+    }
+    void assign(size_t n, int32_t v) {
+        resize(n);
+        std::fill(p_, p_ + n, v);
+    }
+    void copy(const int32_t *from, size_t n) {
+        resize(n);
+        parallel_pieces((int64_t)n, 1 << 18,
+                        [&](int64_t lo, int64_t hi) { std::memcpy(p_ + lo, from + lo, 4 * (size_t)(hi - lo)); });
+    }
+    int32_t *data() { return p_; }
+    const int32_t *data() const { return p_; }
+    int32_t *begin() { return p_; }
+    const int32_t *begin() const { return p_; }
+    const int32_t *end() const { return p_ + n_; }
+    size_t size() const { return n_; }
+
+private:
+    int32_t *p_ = nullptr;
+    size_t n_ = 0;
+};
+
+}  // namespace
+
 struct glass_hip_graph {
     int32_t N = 0, K = 0;
-    std::vector<int32_t> adj;
+    Rows adj;
     std::vector<int32_t> eps;
     bool has_upper = false;
     int32_t up_K = 0, ep = 0;
@@ -373,46 +446,22 @@ struct glass_hip_searcher {
 
 namespace {
 
-// Graph rows as the kernels expect them: ids in range, each row cut at its
-// first -1 and later duplicates of an id removed.  A repeated id in a row is
-// skipped by the visited test in SearchImpl1/2, so dropping it leaves the
-// visit order unchanged.
-int sanitize_graph(glass_hip_graph &g) {
+// What the kernels rely on in a graph: ids in range (up to a row's first -1;
+// set_data cuts the rows there and drops repeated ids on the device), upper
+// lists that stay within their nodes' levels.
+int check_graph(const glass_hip_graph &g) {
     const int32_t N = g.N, K = g.K;
     std::atomic<int> bad{0};
-    auto work = [&](int64_t lo, int64_t hi) {
-        std::vector<int32_t> row(K), tmp(K);
-        for (int64_t i = lo; i < hi; ++i) {
-            int32_t *r = g.adj.data() + i * K;
-            int n = 0;
-            while (n < K && r[n] != -1) ++n;
-            for (int j = 0; j < n; ++j) {
-                if (r[j] < 0 || r[j] >= N) bad = 1;
-            }
-            std::copy(r, r + n, tmp.begin());
-            std::sort(tmp.begin(), tmp.begin() + n);
-            bool dup = std::adjacent_find(tmp.begin(), tmp.begin() + n) != tmp.begin() + n;
-            if (dup) {
-                int m = 0;
-                for (int j = 0; j < n; ++j) {
-                    bool seen = false;
-                    for (int t = 0; t < m; ++t) seen |= row[t] == r[j];
-                    if (!seen) row[m++] = r[j];
-                }
-                std::copy(row.begin(), row.begin() + m, r);
-                n = m;
-            }
-            for (int j = n; j < K; ++j) r[j] = -1;
-        }
-    };
-    unsigned nt = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-    std::vector<std::thread> th;
-    int64_t chunk = ((int64_t)N + nt - 1) / nt;
-    for (unsigned t = 0; t < nt; ++t) {
-        int64_t lo = t * chunk, hi = std::min<int64_t>(N, lo + chunk);
-        if (lo < hi) th.emplace_back(work, lo, hi);
-    }
-    for (auto &t : th) t.join();
+    const auto outside = [N](int32_t v) { return (uint32_t)(v + 1) > (uint32_t)N; };
+    parallel_pieces(N, 4096, [&](int64_t lo, int64_t hi) {
+        // every entry in [-1, N): the usual graph, checked without a branch per entry
+        const int32_t *r = g.adj.data() + lo * K, *end = g.adj.data() + hi * K;
+        bool any = false;
+        for (const int32_t *q = r; q < end; ++q) any |= outside(*q);
+        for (; any && r < end; r += K)
+            for (int32_t j = 0; j < K && r[j] != -1; ++j)
+                if (outside(r[j])) bad = 1;
+    });
     if (bad) return fail(GLASS_HIP_EINVAL, "graph has neighbour ids outside [0, %d)", N);
     for (int32_t e : g.eps) {
         if (e < 0 || e >= N) return fail(GLASS_HIP_EINVAL, "graph entry point %d outside [0, %d)", e, N);
@@ -1184,7 +1233,7 @@ int glass_hip_graph_create(int32_t n, int32_t k, const int32_t *adj, int32_t nep
         auto g = std::make_unique<glass_hip_graph>();
         g->N = n;
         g->K = k;
-        g->adj.assign(adj, adj + (size_t)n * k);
+        g->adj.copy(adj, (size_t)n * k);
         g->eps.assign(eps, eps + nep);
         *out = g.release();
         return GLASS_HIP_OK;
@@ -1253,8 +1302,10 @@ int glass_hip_build_graph(const char *index_type, const float *data, int32_t n, 
             // create_nsg (glass/nsg/nsg.hpp:411-434): the metric is ignored, graphs are L2
             auto g = std::make_unique<glass_hip_graph>();
             int32_t ep = 0;
-            if (glass_build::build_nsg(data, n, dim, R, L, t == "SSG", num_threads, g->adj, ep, seconds))
+            std::vector<int32_t> rows;
+            if (glass_build::build_nsg(data, n, dim, R, L, t == "SSG", num_threads, rows, ep, seconds))
                 return fail(GLASS_HIP_EINVAL, "%s build failed", index_type);
+            g->adj.copy(rows.data(), rows.size());
             g->N = n;
             g->K = R;
             g->eps = {ep};
@@ -1263,10 +1314,11 @@ int glass_hip_build_graph(const char *index_type, const float *data, int32_t n, 
         }
         if (t != "HNSW") return fail(GLASS_HIP_EINVAL, "unsupported index type '%s'", index_type);
         auto g = std::make_unique<glass_hip_graph>();
-        std::vector<int32_t> levels, lists;
+        std::vector<int32_t> rows, levels, lists;
         int32_t ep = 0;
-        if (glass_build::build_hnsw(data, n, dim, m == "IP", R, L, num_threads, g->adj, ep, levels, lists, seconds))
+        if (glass_build::build_hnsw(data, n, dim, m == "IP", R, L, num_threads, rows, ep, levels, lists, seconds))
             return fail(GLASS_HIP_EINVAL, "HNSW build failed");
+        g->adj.copy(rows.data(), rows.size());
         g->N = n;
         g->K = R;
         g->eps = {ep};
@@ -1309,7 +1361,7 @@ int glass_hip_searcher_create(glass_hip_graph *g, const char *metric, const char
         // SQ2U with IP instantiates the L2 searcher (graph_searcher.hpp:357)
         s->quant = qk;
         s->refine = rk;
-        if (int rr = sanitize_graph(s->graph)) return rr;
+        if (int rr = check_graph(s->graph)) return rr;
         *out = s.release();
         return GLASS_HIP_OK;
     } catch (...) {
@@ -1337,7 +1389,9 @@ int glass_hip_searcher_set_data(glass_hip_searcher *s, const float *data, int32_
         // graph
         const glass_hip_graph &g = s->graph;
         HIP_TRY(s->d_adj.alloc(g.adj.size()));
-        HIP_TRY(hipMemcpy(s->d_adj.p, g.adj.data(), 4 * g.adj.size(), hipMemcpyHostToDevice));
+        Stager stage;
+        HIP_TRY(stage.upload(s->d_adj.p, g.adj.data(), 4 * g.adj.size()));
+        HIP_TRY(launch_tidy_rows(s->d_adj.p, g.N, g.K, s->stream));
         HIP_TRY(s->d_eps.alloc(std::max<size_t>(1, g.eps.size())));
         if (!g.eps.empty()) HIP_TRY(hipMemcpy(s->d_eps.p, g.eps.data(), 4 * g.eps.size(), hipMemcpyHostToDevice));
         if (g.has_upper) {
@@ -1349,11 +1403,24 @@ int glass_hip_searcher_set_data(glass_hip_searcher *s, const float *data, int32_
             if (!g.up_lists.empty())
                 HIP_TRY(hipMemcpy(s->d_up_lists.p, g.up_lists.data(), 4 * g.up_lists.size(), hipMemcpyHostToDevice));
         }
-        // base rows -> device, encode there
-        DevBuf<float> raw;
-        HIP_TRY(raw.alloc((size_t)n * dim));
-        HIP_TRY(hipMemcpy(raw.p, data, sizeof(float) * (size_t)n * dim, hipMemcpyHostToDevice));
-        if (int r = train_quant(*s, raw.p, n)) return r;
+        // base rows -> device, encode there.  FP32 rows that need no padding
+        // are re-rank rows or codes as they are.
+        DevBuf<float> own;
+        float *raw = nullptr;
+        const bool rows_are_rerank = s->refine == QK_FP32 && s->r_dim_align == dim;
+        const bool rows_are_codes = s->quant == QK_FP32 && s->dim_align == dim && !rows_are_rerank;
+        if (rows_are_rerank) {
+            HIP_TRY(s->d_rerank.alloc((size_t)n * r_row_bytes));
+            raw = (float *)s->d_rerank.p;
+        } else if (rows_are_codes) {
+            HIP_TRY(s->d_codes.alloc((size_t)n * s->code_size));
+            raw = (float *)s->d_codes.p;
+        } else {
+            HIP_TRY(own.alloc((size_t)n * dim));
+            raw = own.p;
+        }
+        HIP_TRY(stage.upload(raw, data, sizeof(float) * (size_t)n * dim));
+        if (int r = train_quant(*s, raw, n)) return r;
         if (s->quant == QK_SQ8 || s->quant == QK_SQ6 || s->quant == QK_SQ4) {
             HIP_TRY(s->d_mins.alloc(s->dim_align));
             HIP_TRY(s->d_difs.alloc(s->dim_align));
@@ -1361,28 +1428,30 @@ int glass_hip_searcher_set_data(glass_hip_searcher *s, const float *data, int32_
             HIP_TRY(hipMemcpy(s->d_difs.p, s->sq8_difs.data(), 4 * (size_t)s->dim_align, hipMemcpyHostToDevice));
         }
         HIP_TRY(s->d_codes.alloc((size_t)n * s->code_size));
-        if (s->quant == QK_FP32) {
-            HIP_TRY(launch_pad_rows(raw.p, n, dim, s->dim_align, (float *)s->d_codes.p, s->stream));
+        if (rows_are_codes) {
+        } else if (s->quant == QK_FP32) {
+            HIP_TRY(launch_pad_rows(raw, n, dim, s->dim_align, (float *)s->d_codes.p, s->stream));
         } else if (s->quant == QK_PQ8) {
             // k-means on the host, as ProductQuant::train; nearest-centroid codes on the device
             pq::train(data, n, dim, s->pq_codebook);
             HIP_TRY(s->d_codebook.alloc(s->pq_codebook.size()));
             HIP_TRY(hipMemcpy(s->d_codebook.p, s->pq_codebook.data(), 4 * s->pq_codebook.size(), hipMemcpyHostToDevice));
-            HIP_TRY(launch_pq_encode(raw.p, n, s->code_size, s->d_codebook.p, s->d_codes.p, s->stream));
+            HIP_TRY(launch_pq_encode(raw, n, s->code_size, s->d_codebook.p, s->d_codes.p, s->stream));
         } else {
-            HIP_TRY(launch_encode(raw.p, n, dim, s->code_size, s->quant, s->metric, s->qmin, s->qdif, s->qmax,
+            HIP_TRY(launch_encode(raw, n, dim, s->code_size, s->quant, s->metric, s->qmin, s->qdif, s->qmax,
                                   s->d_mins.p, s->d_difs.p, s->d_codes.p, s->stream));
         }
-        if (s->refine == QK_FP32) {
+        if (rows_are_rerank) {
+        } else if (s->refine == QK_FP32) {
             HIP_TRY(s->d_rerank.alloc((size_t)n * r_row_bytes));
-            HIP_TRY(launch_pad_rows(raw.p, n, dim, s->r_dim_align, (float *)s->d_rerank.p, s->stream));
+            HIP_TRY(launch_pad_rows(raw, n, dim, s->r_dim_align, (float *)s->d_rerank.p, s->stream));
         } else if (s->refine == QK_FP16) {  // FP16Quantizer::add, as for the search codes
             HIP_TRY(s->d_rerank.alloc((size_t)n * r_row_bytes));
-            HIP_TRY(launch_encode(raw.p, n, dim, r_row_bytes, QK_FP16, s->metric, 0.0f, 0.0f, 0.0f, nullptr, nullptr,
+            HIP_TRY(launch_encode(raw, n, dim, r_row_bytes, QK_FP16, s->metric, 0.0f, 0.0f, 0.0f, nullptr, nullptr,
                                   s->d_rerank.p, s->stream));
         } else if (s->refine == QK_SQ8U || s->refine == QK_SQ8) {
             // SQ8QuantizerUniform / SQ8Quantizer trained and encoded like search codes
-            if (int r = train_refine(*s, raw.p, n)) return r;
+            if (int r = train_refine(*s, raw, n)) return r;
             if (s->refine == QK_SQ8) {
                 HIP_TRY(s->d_rmins.alloc(s->r_dim_align));
                 HIP_TRY(s->d_rdifs.alloc(s->r_dim_align));
@@ -1390,11 +1459,11 @@ int glass_hip_searcher_set_data(glass_hip_searcher *s, const float *data, int32_
                 HIP_TRY(hipMemcpy(s->d_rdifs.p, s->r_difs.data(), 4 * (size_t)s->r_dim_align, hipMemcpyHostToDevice));
             }
             HIP_TRY(s->d_rerank.alloc((size_t)n * r_row_bytes));
-            HIP_TRY(launch_encode(raw.p, n, dim, r_row_bytes, s->refine, s->metric, s->r_qmin, s->r_qdif, s->r_qmax,
+            HIP_TRY(launch_encode(raw, n, dim, r_row_bytes, s->refine, s->metric, s->r_qmin, s->r_qdif, s->r_qmax,
                                   s->d_rmins.p, s->d_rdifs.p, s->d_rerank.p, s->stream));
         }
         HIP_TRY(hipStreamSynchronize(s->stream));
-        raw.release();
+        own.release();
         // Optimize sample (graph_searcher.hpp:62-69)
         s->sample_points_num = std::min(1000, n - 1);
         if (s->sample_points_num > 0) {
@@ -1907,7 +1976,8 @@ int glass_hip_quant_train(const char *quantizer, const char *metric, const float
             if (int r = ensure_stream(t)) return r;
             DevBuf<float> raw;
             HIP_TRY(raw.alloc((size_t)n * dim));
-            HIP_TRY(hipMemcpy(raw.p, data, sizeof(float) * (size_t)n * dim, hipMemcpyHostToDevice));
+            Stager stage;
+            HIP_TRY(stage.upload(raw.p, data, sizeof(float) * (size_t)n * dim));
             if (int r = train_quant(t, raw.p, n)) return r;
         }
         return glass_hip_searcher_get_calibration(&t, params, nparams);
