@@ -119,7 +119,7 @@ int glass_hip_searcher_search_batch_dev(glass_hip_searcher *s, const float *qs_d
  * the process ends; the persistent grid is capped to the waves whose slot
  * areas fit in it (N/8 bytes each, 4 waves at least: N up to about 268M
  * rows), and larger requests fail with GLASS_HIP_EINVAL.  Requires set_data
- * first; launches eagerly (no graph replay).  Every call on a GPU shares that
+ * first.  Every call on a GPU shares that
  * GPU's array, so calls that overlap on one GPU race: order them (one stream,
  * or events). */
 int glass_hip_searcher_search_batch_dev_noalloc(glass_hip_searcher *s, const float *qs_dev, int32_t nq, int32_t k,
@@ -134,10 +134,8 @@ int glass_hip_searcher_search_batch_efk_dev(glass_hip_searcher *s, const float *
                                             const int32_t *ef_dev, const int32_t *k_dev, const int64_t *off_dev,
                                             int32_t max_ef, int32_t max_k, int32_t *dst_dev, float *scores_dev,
                                             int32_t *counters_dev, void *stream);
-/* search_batch_dev replays a captured hipGraph (counter-reset kernel +
- * search kernel) when every kernel argument and the stream repeat the
- * previous call's; the first call with new arguments runs eagerly and is
- * then captured.  on = 0 always launches eagerly.  Default on. */
+/* Accepted and without effect: search_batch_dev was two launches replayed as
+ * a captured hipGraph; it is one launch now. */
 int glass_hip_searcher_set_graph_capture(glass_hip_searcher *s, int32_t on);
 /* Re-rank depth: reorder_k = int(k * factor).  0 restores the reference's
  * get_refine_factor(quantizer) (graph_searcher.hpp:227-238: 1.5 for

@@ -283,7 +283,7 @@ class Searcher:
         _lib.check(self._L.glass_hip_searcher_set_launch(self._h, int(team), int(waves_per_block), int(blocks)))
 
     def set_graph_capture(self, on: bool = True):
-        """search_batch_dev replays a captured hipGraph when its arguments repeat."""
+        """Accepted and without effect: search_batch_dev is one launch."""
         _lib.check(self._L.glass_hip_searcher_set_graph_capture(self._h, int(bool(on))))
 
     def set_query_waves(self, waves: int = 0):

@@ -289,18 +289,7 @@ struct glass_hip_graph {
     std::vector<int32_t> up_lists;
 };
 
-// Everything one batch launch passes to its kernels, plus the stream: two
-// launches with equal keys are identical, so a captured graph can replay one.
-struct GraphKey {
-    glass_hip::DeviceIndex ix;
-    glass_hip::QueryBatch qb;
-    glass_hip::LaunchConfig lc;
-    glass_hip::SlotState ss;
-    hipStream_t stream;
-};
-
-// Launch state of one stream: its work counter, slot areas and captured
-// graph.  Launches on one stream share it (the stream orders them); launches
+// Launch state of one stream: its work counter and slot areas.  Launches on one stream share it (the stream orders them); launches
 // on different streams use different states, so they run concurrently (one
 // batch's last round overlaps the next batch's first).
 struct StreamState {
@@ -308,15 +297,12 @@ struct StreamState {
     DevBuf<uint32_t> visited;
     int32_t nslots = 0;
     DevBuf<int32_t> counter;
-    hipGraphExec_t gexec = nullptr;
-    GraphKey gkey{};
     hipEvent_t done = nullptr;  // recorded after each launch that uses this state
     uint64_t last_use = 0;
     StreamState() = default;
     StreamState(const StreamState &) = delete;
     StreamState &operator=(const StreamState &) = delete;
     ~StreamState() {
-        if (gexec) (void)hipGraphExecDestroy(gexec);
         if (done) (void)hipEventDestroy(done);
     }
 };
@@ -392,9 +378,6 @@ struct glass_hip_searcher {
     // Optimize sample (GraphSearcher::SetData keeps <=1000 base rows, graph_searcher.hpp:62-69)
     std::vector<float> optimize_queries;
     int32_t sample_points_num = 0;
-
-    // device-pointer batches replay a captured graph when their arguments repeat
-    bool graph_capture = true;
 
     ~glass_hip_searcher() {
         sstates.clear();
@@ -950,7 +933,7 @@ struct BatchState {
 int run_batch(glass_hip_searcher &s, const float *qs_dev, int32_t nq, const int32_t *ef_dev, const int32_t *k_dev,
               int32_t ef_uniform, int32_t k_uniform, int32_t max_cap, int32_t max_ef, int32_t mode,
               const int64_t *off_dev, int32_t *ids_dev, float *dists_dev, int32_t *counters_dev, hipStream_t stream,
-              const BatchState *bs = nullptr, bool graph = false, bool alone = false) {
+              const BatchState *bs = nullptr, bool alone = false) {
     if (!s.has_data) return fail(GLASS_HIP_ESTATE, "search before set_data");
     if (nq <= 0) return GLASS_HIP_OK;
     if (int r = ensure_stream(s)) return r;
@@ -1018,7 +1001,10 @@ int run_batch(glass_hip_searcher &s, const float *qs_dev, int32_t nq, const int3
     if (!bs) {
         if (int r = state_for(s, stream, &st)) return r;
         if (int r = ensure_slots(s, *st, blocks * slots_per_block(lc), stream)) return r;
-        if (!st->counter.p) HIP_TRY(st->counter.alloc(1));
+        if (!st->counter.p) {
+            HIP_TRY(st->counter.alloc(2));
+            HIP_TRY(launch_fill_i32(st->counter.p, 2, 0, stream));
+        }
     }
     int32_t *counter = bs ? bs->counter : st->counter.p;
     QueryBatch qb{};
@@ -1043,55 +1029,9 @@ int run_batch(glass_hip_searcher &s, const float *qs_dev, int32_t nq, const int3
     ss.nslots = bs ? bs->max_slots : st->nslots;
     ss.work_counter = counter;
     const DeviceIndex ix = s.index();
-    // counter reset (a fill kernel, not hipMemsetAsync, so it can sit in a graph) + search
-    auto enqueue = [&]() -> hipError_t {
-        hipError_t e = launch_fill_i32(counter, 1, 0, stream);
-        return e == hipSuccess ? launch_search(ix, qb, lc, ss, stream) : e;
-    };
     s.last_launch = lc;
-    auto mark = [&]() -> int {
-        if (st) HIP_TRY(hipEventRecord(st->done, stream));
-        return GLASS_HIP_OK;
-    };
-    if (!graph || !st) {
-        HIP_TRY(enqueue());
-        return mark();
-    }
-    // Graph replay: the key is every kernel argument plus the stream, so a
-    // replay launches exactly what an eager call with these arguments would.
-    GraphKey key{};
-    key.ix = ix;
-    key.qb = qb;
-    key.lc = lc;
-    key.ss = ss;
-    key.stream = stream;
-    if (st->gexec && std::memcmp(&key, &st->gkey, sizeof(key)) == 0) {
-        HIP_TRY(hipGraphLaunch(st->gexec, stream));
-        return mark();
-    }
-    // first call with these arguments: run eagerly (this also does any
-    // one-time set-up), then capture the same two launches for next time
-    HIP_TRY(enqueue());
-    if (int r = mark()) return r;
-    if (st->gexec) {
-        (void)hipGraphExecDestroy(st->gexec);
-        st->gexec = nullptr;
-    }
-    hipGraph_t gr = nullptr;
-    HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-    const hipError_t ce = enqueue();
-    const hipError_t ee = hipStreamEndCapture(stream, &gr);
-    if (ce != hipSuccess || ee != hipSuccess) {
-        if (gr) (void)hipGraphDestroy(gr);
-        return fail(GLASS_HIP_EDEVICE, "graph capture failed: %s", hipGetErrorString(ce != hipSuccess ? ce : ee));
-    }
-    const hipError_t ie = hipGraphInstantiate(&st->gexec, gr, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(gr);
-    if (ie != hipSuccess) {
-        st->gexec = nullptr;
-        return fail(GLASS_HIP_EDEVICE, "graph instantiate failed: %s", hipGetErrorString(ie));
-    }
-    st->gkey = key;
+    HIP_TRY(launch_search(ix, qb, lc, ss, stream));
+    if (st) HIP_TRY(hipEventRecord(st->done, stream));
     return GLASS_HIP_OK;
 }
 
@@ -1148,7 +1088,7 @@ int host_batch(glass_hip_searcher &s, const float *qs, int32_t nq, const int32_t
         d_off = s.d_off.p;
     }
     int r = run_batch(s, s.d_q.p, nq, d_ef, d_k, s.ef, k_uniform, max_cap, max_ef, mode, d_off, s.d_ids.p, s.d_dists.p,
-                      s.d_counters.p, s.stream, nullptr, false, true);
+                      s.d_counters.p, s.stream, nullptr, true);
     if (r) return r;
     HIP_TRY(hipMemcpyAsync(dst, s.d_ids.p, 4 * (size_t)total, hipMemcpyDeviceToHost, s.stream));
     if (scores)
@@ -1543,7 +1483,7 @@ int glass_hip_searcher_search_batch_dev(glass_hip_searcher *s, const float *qs_d
         const int32_t max_cap = std::max(inner_k(*s, k), s->ef);
         if (int r = check_cap(*s, max_cap)) return r;
         return run_batch(*s, qs_dev, nq, nullptr, nullptr, s->ef, k, max_cap, s->ef, mode, nullptr, dst_dev, scores_dev,
-                         counters_dev, (hipStream_t)stream, nullptr, s->graph_capture);
+                         counters_dev, (hipStream_t)stream);
     } catch (...) {
         return exception_status();
     }
@@ -1586,12 +1526,14 @@ int glass_hip_searcher_search_batch_dev_noalloc(glass_hip_searcher *s, const flo
                 lay_lut[d] = s->lut_words;
             }
         }
+        // calls that overlapped on the array may have left its counter anywhere
+        HIP_TRY(launch_fill_i32((int32_t *)base, 2, 0, stream ? (hipStream_t)stream : s->stream));
         BatchState bs;
         bs.counter = (int32_t *)base;
         bs.visited = (uint32_t *)((uint8_t *)base + 256);
         bs.max_slots = (int32_t)std::min<int64_t>(slots, 1 << 20);
         return run_batch(*s, qs_dev, nq, nullptr, nullptr, s->ef, k, max_cap, s->ef, mode, nullptr, dst_dev,
-                         scores_dev, counters_dev, (hipStream_t)stream, &bs, false);
+                         scores_dev, counters_dev, (hipStream_t)stream, &bs);
     } catch (...) {
         return exception_status();
     }
@@ -1609,7 +1551,7 @@ int glass_hip_searcher_search_batch_efk_dev(glass_hip_searcher *s, const float *
         const int32_t max_cap = std::max(inner_k(*s, max_k), max_ef);
         if (int r = check_cap(*s, max_cap)) return r;
         return run_batch(*s, qs_dev, nq, ef_dev, k_dev, 0, 0, max_cap, max_ef, MODE_BATCH, off_dev, dst_dev,
-                         scores_dev, counters_dev, (hipStream_t)stream, nullptr, s->graph_capture);
+                         scores_dev, counters_dev, (hipStream_t)stream);
     } catch (...) {
         return exception_status();
     }
@@ -1619,7 +1561,7 @@ int glass_hip_searcher_set_graph_capture(glass_hip_searcher *s, int32_t on) {
     try {
         if (!s) return fail(GLASS_HIP_EINVAL, "null searcher");
         std::lock_guard<std::mutex> lk(s->mu);
-        s->graph_capture = on != 0;
+        (void)on;  // a call is one kernel launch: there is nothing to capture
         return GLASS_HIP_OK;
     } catch (...) {
         return exception_status();
@@ -2528,7 +2470,8 @@ int glass_hip_server_create(glass_hip_searcher *s, int32_t max_batch, int32_t ma
             HIP_TRY(hipHostMalloc((void **)&sl.h_out, sv->out_bytes, hipHostMallocMapped | hipHostMallocCoherent));
             HIP_TRY(hipHostGetDevicePointer((void **)&sl.d_out, sl.h_out, 0));
             HIP_TRY(sl.d_in.alloc(sv->in_bytes));
-            HIP_TRY(sl.counter.alloc(1));
+            HIP_TRY(sl.counter.alloc(2));
+            HIP_TRY(launch_fill_i32(sl.counter.p, 2, 0, s->stream));
             sl.visited = sv->visited.p + (size_t)i * (size_t)sv->slots_per_batch * (size_t)s->vis_stride;
             HIP_TRY(hipStreamCreateWithFlags(&sl.stream, hipStreamNonBlocking));
             HIP_TRY(hipEventCreateWithFlags(&sl.done, hipEventDisableTiming));

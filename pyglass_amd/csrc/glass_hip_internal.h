@@ -87,7 +87,7 @@ struct SlotState {
     int32_t dirty_words;     // then the bitset words a query set first (multiple of 4), then the bitset
 
     int32_t nslots;
-    int32_t *work_counter;   // device counter for the persistent queue
+    int32_t *work_counter;   // two words, zero between launches: queries handed out, slots that have ended
 };
 
 // Launches the persistent search kernel for one batch on `stream`.

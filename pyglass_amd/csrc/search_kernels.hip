@@ -1673,11 +1673,25 @@ template <int V, int DPL, int P>
 constexpr int kWavesPerEu =
     P == 1 ? ((V == V_SQ2U && DPL == 16) || V == V_SQ8_L2 || V == V_SQ8_IP ? 3 : 4) : (P == 2 ? 2 : 3);
 
+struct KernelArgs {
+    DeviceIndex ix;
+    QueryBatch qb;
+    LaunchConfig lc;
+    SlotState ss;
+};
+
+// The kernel's arguments, read again from the argument segment where a phase
+// of a query begins.  Held from the kernel's start they fill the scalar
+// registers across the expansion loop, which needs few of them, and the rest
+// is spilled to lanes of vector registers and read back in the loop.
+__device__ __forceinline__ const KernelArgs &fresh_args() {
+    auto p = (const __attribute__((address_space(4))) KernelArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const KernelArgs *)p;
+}
+
 template <int V, int DPL, int P>
-__global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<V, DPL, P>))) void search_kernel(DeviceIndex ix,
-                                                                                            QueryBatch qb,
-                                                                                            LaunchConfig lc,
-                                                                                            SlotState ss) {
+__global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<V, DPL, P>))) void search_kernel(KernelArgs) {
     constexpr bool kFast = P == 1;
     // registers of float rows' loads in flight, in the search and in the re-rank of long rows
     constexpr bool kSq8 = V == V_SQ8_L2 || V == V_SQ8_IP;  // its LDS rows take registers too
@@ -1687,44 +1701,64 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
     constexpr int kAhead = DPL == 16 && (P == 1 || (P == 0 && V == V_SQ2U)) ? 1 : 2;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     const int l = lane_id();
-    const int wv = threadIdx.x >> 6;
-    const size_t wbytes = wave_lds_bytes(ix, lc.cap_max, lc.vis_hash);
+    const int wv = uni((int)(threadIdx.x >> 6));
     // Waves per query: 1 (each wave its own query), or -- the P = 2 kernel --
     // every wave of the workgroup on one query: wave 0 leads (pool, visited
     // set, merges, initializer, outputs) and all waves share each expansion's
     // distance passes.  The query's LDS area is then the workgroup's, and two
     // control words follow it (the query index, the expansion's candidates).
-    const int W = P == 2 ? at_use(lc.qwaves) : 1;
+    const int W = P == 2 ? at_use(fresh_args().lc.qwaves) : 1;
     const bool lead = W == 1 || wv == 0;
-    const WaveLds w = carve(lds_raw + (W > 1 ? (size_t)0 : (size_t)wv * wbytes), ix, lc.cap_max, lc.vis_hash);
-    int32_t *const ctl = (int32_t *)(lds_raw + wbytes);
-    const int slot = W > 1 ? (int)blockIdx.x : (int)blockIdx.x * lc.waves_per_block + wv;
-    // the slot's HBM scratch: PQ8 lookup table (lut_words), the visited
-    // bitset's dirty list (dirty_words), then the bitset
-    uint32_t *const slot_mem = ss.visited + (int64_t)slot * ss.vis_stride;
-    float *const lut = (float *)slot_mem;
-    uint32_t *const dlist = slot_mem + ss.lut_words;
-    uint32_t *const vis = dlist + ss.dirty_words;
-    const int ql = qf_len(ix);
+    const int slot = W > 1 ? (int)blockIdx.x : (int)blockIdx.x * fresh_args().lc.waves_per_block + wv;
 
+    // A batch that fits the slots gives each slot the query of its number; a
+    // larger one hands its queries out through the work counter, which the
+    // last slot to end sets back to zero, so that a launch needs no other
+    // before it.
     // The next query's index, and its row when ql <= 256 (xn, four floats
     // per lane), are requested before the current query's output phase, so
     // that their latency overlaps it.
-    int qi_next = 0;
-    if (W == 1) {
-        if (l == 0) qi_next = atomicAdd(ss.work_counter, 1);
-        qi_next = uni(qi_next);
+    auto queued = [&](const KernelArgs &a) __attribute__((always_inline)) {
+        return a.qb.nq > (W > 1 ? (int)gridDim.x : (int)gridDim.x * a.lc.waves_per_block);
+    };
+    auto take = [&](const KernelArgs &a) __attribute__((always_inline)) {  // by one lane
+        return queued(a) ? atomicAdd(a.ss.work_counter, 1) : a.qb.nq;
+    };
+    // the first query: its slot's, or the next in the queue
+    int qi_next = slot;
+    if (queued(fresh_args())) {
+        if (W > 1) {
+            const KernelArgs &a = fresh_args();
+            int32_t *const ctl = (int32_t *)(lds_raw + wave_lds_bytes(a.ix, a.lc.cap_max, a.lc.vis_hash));
+            if (lead && l == 0) ctl[0] = take(a);
+            __syncthreads();
+            qi_next = uni(ctl[0]);
+        } else {
+            int t = 0;
+            if (l == 0) t = take(fresh_args());
+            qi_next = uni(t);
+        }
     }
     bool have_row = false;
     float xn[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     for (;;) {
-        if (W > 1) {
-            if (wv == 0 && l == 0) ctl[0] = atomicAdd(ss.work_counter, 1);
-            __syncthreads();
-            qi_next = uni(ctl[0]);
-        }
+        const KernelArgs &ka = fresh_args();
+        const DeviceIndex &ix = ka.ix;
+        const QueryBatch &qb = ka.qb;
+        const LaunchConfig &lc = ka.lc;
+        const SlotState &ss = ka.ss;
         const int qi = qi_next;
         if (qi >= qb.nq) break;
+        const size_t wbytes = wave_lds_bytes(ix, lc.cap_max, lc.vis_hash);
+        const WaveLds w = carve(lds_raw + (W > 1 ? (size_t)0 : (size_t)wv * wbytes), ix, lc.cap_max, lc.vis_hash);
+        int32_t *const ctl = (int32_t *)(lds_raw + wbytes);
+        // the slot's HBM scratch: PQ8 lookup table (lut_words), the visited
+        // bitset's dirty list (dirty_words), then the bitset
+        uint32_t *const slot_mem = ss.visited + (int64_t)slot * ss.vis_stride;
+        float *const lut = (float *)slot_mem;
+        uint32_t *const dlist = slot_mem + ss.lut_words;
+        uint32_t *const vis = dlist + ss.dirty_words;
+        const int ql = qf_len(ix);
 
         const int32_t ef = uni(qb.ef ? qb.ef[qi] : qb.ef_uniform);
         const int32_t k = uni(qb.k ? qb.k[qi] : qb.k_uniform);
@@ -1955,8 +1989,9 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
                 }
             }
         } else {
-        const int nj = spec ? l / iq.slot : l;  // adjacency entry this lane reads
-        const uint64_t lead_k = ballot(iq.part == 0 && nj < ix.K);  // first lane of each group with an entry
+        const int nj = is_int_variant(V) && spec ? l / iq.slot : l;  // adjacency entry this lane reads
+        // first lane of each group with an entry
+        const uint64_t lead_k = is_int_variant(V) ? ballot(iq.part == 0 && nj < ix.K) : 0;
         uint32_t pred = kIdMask;
         int32_t pred_row = -1;
         const int njc = nj < ix.K ? nj : ix.K - 1;  // lanes past K read the last entry and drop it
@@ -1965,7 +2000,7 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
             cnt_e += 1;
             const int32_t vr = (u == pred) ? pred_row : ix.adj[(int64_t)u * ix.K + njc];
             const int32_t v = nj < ix.K ? vr : -1;
-            if (kFast ? is_int_variant(V) : at_use(spec) != 0) {
+            if (is_int_variant(V) && (kFast || at_use(spec) != 0)) {
                 const bool lead = iq.part == 0;
                 const uint64_t inv = lead_k & ballot(v == -1);
                 const int n = inv ? __builtin_ctzll(inv) / iq.slot : ix.K;
@@ -2047,23 +2082,24 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
         }  // one wave per query
         if (lead) vs.cleanup();
         // take the next query now (see above)
+        const KernelArgs &ko = fresh_args();
         if (W == 1) {
             int t = 0;
-            if (l == 0) t = atomicAdd(ss.work_counter, 1);
+            if (l == 0) t = take(ko);
             qi_next = uni(t);
-            have_row = qi_next < qb.nq && ql <= 256;
+            have_row = qi_next < ko.qb.nq && qf_len(ko.ix) <= 256;
             if (have_row) {
-                const float *xq = qb.queries + (int64_t)qi_next * qb.dim;
+                const float *xq = ko.qb.queries + (int64_t)qi_next * ko.qb.dim;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int j = l + 64 * r;
-                    xn[r] = j < ix.dim ? xq[j] : 0.0f;
+                    xn[r] = j < ko.ix.dim ? xq[j] : 0.0f;
                 }
             }
         }
 
         // outputs
-        const int64_t ob = qb.out_off ? qb.out_off[qi] : (int64_t)qi * qb.k_uniform;
+        const int64_t ob = ko.qb.out_off ? ko.qb.out_off[qi] : (int64_t)qi * ko.qb.k_uniform;
         if (!lead) {
         } else if (!refine) {
             // LinearPool::to_sorted (neighbor.hpp:421-428)
@@ -2074,34 +2110,34 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
                     id = (int32_t)(w.pid[i] & kIdMask);
                     d = is_int_variant(V) ? (float)int_of_key(w.pk[i]) : float_of_key(w.pk[i]);
                 }
-                put_result(qb, ob + i, id, d);
+                put_result(ko.qb, ob + i, id, d);
             }
         } else {
             // Refiner::RefineImpl (refiner.hpp:92-110): exact FP32 distances of the
             // first reorder_k pool entries, the k smallest by (dist, id) ascending.
             const int m = kk < ps.size ? kk : ps.size;
-            if (ix.rerank_kind == QK_FP16) {
-                if (ix.metric == MK_L2) {
-                    rerank<V_FP16_L2, kRerankRegs>(ix, w, m);
+            if (ko.ix.rerank_kind == QK_FP16) {
+                if (ko.ix.metric == MK_L2) {
+                    rerank<V_FP16_L2, kRerankRegs>(ko.ix, w, m);
                 } else {
-                    rerank<V_FP16_IP, kRerankRegs>(ix, w, m);
+                    rerank<V_FP16_IP, kRerankRegs>(ko.ix, w, m);
                 }
-            } else if (!kFast && ix.rerank_kind == QK_SQ8U) {
-                if (ix.metric == MK_L2) {
-                    rerank_sq8u<true>(ix, w, m);
+            } else if (!kFast && ko.ix.rerank_kind == QK_SQ8U) {
+                if (ko.ix.metric == MK_L2) {
+                    rerank_sq8u<true>(ko.ix, w, m);
                 } else {
-                    rerank_sq8u<false>(ix, w, m);
+                    rerank_sq8u<false>(ko.ix, w, m);
                 }
-            } else if (!kFast && ix.rerank_kind == QK_SQ8) {
-                if (ix.metric == MK_L2) {
-                    rerank_sq8<V_SQ8_L2, 8>(ix, w, m);
+            } else if (!kFast && ko.ix.rerank_kind == QK_SQ8) {
+                if (ko.ix.metric == MK_L2) {
+                    rerank_sq8<V_SQ8_L2, 8>(ko.ix, w, m);
                 } else {
-                    rerank_sq8<V_SQ8_IP, 8>(ix, w, m);
+                    rerank_sq8<V_SQ8_IP, 8>(ko.ix, w, m);
                 }
-            } else if (ix.metric == MK_L2) {
-                rerank<V_FP32_L2, kRerankRegs>(ix, w, m);
+            } else if (ko.ix.metric == MK_L2) {
+                rerank<V_FP32_L2, kRerankRegs>(ko.ix, w, m);
             } else {
-                rerank<V_FP32_IP, kRerankRegs>(ix, w, m);
+                rerank<V_FP32_IP, kRerankRegs>(ko.ix, w, m);
             }
             wave_sync();
             // Ranks by (dist, id), with equal pairs (a repeated entry point
@@ -2129,8 +2165,8 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
                     ra += ci < ca;  // every i here is after position l
                     rb += (ci < cb) | ((ci == cb) & (i < j1));
                 }
-                if (l < m && ra < k) put_result(qb, ob + ra, (int32_t)ia, float_of_key(ka));
-                if (j1 < m && rb < k) put_result(qb, ob + rb, (int32_t)ib, float_of_key(kb));
+                if (l < m && ra < k) put_result(ko.qb, ob + ra, (int32_t)ia, float_of_key(ka));
+                if (j1 < m && rb < k) put_result(ko.qb, ob + rb, (int32_t)ib, float_of_key(kb));
             } else {
                 for (int j = l; j < m; j += 64) {
                     const uint32_t kj = w.pk[j], ij = w.pid[j] & kIdMask;
@@ -2139,20 +2175,31 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
                         const uint32_t ki = w.pk[i], ii = w.pid[i] & kIdMask;
                         rank += (ki < kj) | ((ki == kj) & (ii < ij)) | ((ki == kj) & (ii == ij) & (i < j));
                     }
-                    if (rank < k) put_result(qb, ob + rank, (int32_t)ij, float_of_key(kj));
+                    if (rank < k) put_result(ko.qb, ob + rank, (int32_t)ij, float_of_key(kj));
                 }
             }
-            for (int i = m + l; i < k; i += 64) put_result(qb, ob + i, -1, __builtin_inff());
+            for (int i = m + l; i < k; i += 64) put_result(ko.qb, ob + i, -1, __builtin_inff());
         }
-        if (qb.out_counters && lead && l == 0) {
-            qb.out_counters[(int64_t)qi * 3 + 0] = cnt_d;
-            qb.out_counters[(int64_t)qi * 3 + 1] = cnt_e;
-            qb.out_counters[(int64_t)qi * 3 + 2] = cnt_u;
+        if (ko.qb.out_counters && lead && l == 0) {
+            ko.qb.out_counters[(int64_t)qi * 3 + 0] = cnt_d;
+            ko.qb.out_counters[(int64_t)qi * 3 + 1] = cnt_e;
+            ko.qb.out_counters[(int64_t)qi * 3 + 2] = cnt_u;
         }
         if (W > 1) {
+            if (lead && l == 0) ctl[0] = take(ko);
             __syncthreads();
+            qi_next = uni(ctl[0]);
         } else {
             wave_sync();
+        }
+    }
+    const KernelArgs &ke = fresh_args();
+    if (queued(ke) && lead && l == 0) {
+        const int nslots = W > 1 ? (int)gridDim.x : (int)gridDim.x * ke.lc.waves_per_block;
+        // every slot's last take came before its own count here
+        if (atomicAdd(ke.ss.work_counter + 1, 1) == nslots - 1) {
+            atomicExch(ke.ss.work_counter, 0);
+            atomicExch(ke.ss.work_counter + 1, 0);
         }
     }
 }
@@ -2204,13 +2251,13 @@ hipError_t launch_one(const DeviceIndex &ix, const QueryBatch &qb, const LaunchC
     }
     if (lc.qwaves > 1) {
         hipLaunchKernelGGL((search_kernel<V, DPL, 2>), dim3(lc.blocks), dim3(64 * lc.waves_per_block), lds, stream,
-                           ix, qb, lc, ss);
+                           KernelArgs{ix, qb, lc, ss});
     } else if (fast_path<V, DPL>(ix, lc)) {
         hipLaunchKernelGGL((search_kernel<V, DPL, 1>), dim3(lc.blocks), dim3(64 * lc.waves_per_block), lds, stream,
-                           ix, qb, lc, ss);
+                           KernelArgs{ix, qb, lc, ss});
     } else {
         hipLaunchKernelGGL((search_kernel<V, DPL, 0>), dim3(lc.blocks), dim3(64 * lc.waves_per_block), lds, stream,
-                           ix, qb, lc, ss);
+                           KernelArgs{ix, qb, lc, ss});
     }
     return hipGetLastError();
 }
