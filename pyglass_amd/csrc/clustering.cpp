@@ -274,8 +274,9 @@ int fit_device(const float *rows, int32_t n, int32_t d, int32_t k, int32_t epoch
     return GLASS_HIP_OK;
 }
 
-// A clustering object's stream and events, made at first use and kept with it (making one
-// takes 0.5 ms); one call at a time.
+// A clustering object's stream and events, made by the first call that has
+// pieces to overlap and kept with it (making them takes 0.5 ms, more than all
+// of a call on a few thousand rows); one call at a time.
 struct Device {
     std::mutex mu;
     hipStream_t stream = nullptr;
@@ -293,9 +294,12 @@ int predict_device(Device &dev, const float *cent, int32_t k, int32_t d, const f
     const int64_t piece = std::max<int64_t>(64, ((int64_t)4 << 20) / d / 64 * 64);
     const int32_t rows = (int32_t)std::min<int64_t>(n, piece);
     const int32_t bufs = n > rows ? 2 : 1;
-    if (!dev.stream) CL_TRY(hipStreamCreateWithFlags(&dev.stream, hipStreamNonBlocking));
-    for (hipEvent_t &e : dev.done)
-        if (!e) CL_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    if (bufs > 1) {
+        if (!dev.stream) CL_TRY(hipStreamCreateWithFlags(&dev.stream, hipStreamNonBlocking));
+        for (hipEvent_t &e : dev.done)
+            if (!e) CL_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    }
+    const hipStream_t stream = bufs > 1 ? dev.stream : nullptr;
     Arena a;
     const size_t o_x = a.add(4 * (size_t)rows * d * bufs), o_cent = a.add(4 * (size_t)k * d),
                  o_ids = a.add(4 * (size_t)n), o_scratch = a.add(AssignScratch::bytes(rows, k));
@@ -303,7 +307,7 @@ int predict_device(Device &dev, const float *cent, int32_t k, int32_t d, const f
     struct Drain {  // before the arena goes
         hipStream_t s;
         ~Drain() { (void)hipStreamSynchronize(s); }
-    } drain{dev.stream};
+    } drain{stream};
     float *dc = a.at<float>(o_cent);
     int32_t *di = a.at<int32_t>(o_ids);
     AssignScratch s;
@@ -316,11 +320,11 @@ int predict_device(Device &dev, const float *cent, int32_t k, int32_t d, const f
         if (turn >= 2) CL_TRY(hipEventSynchronize(dev.done[b]));
         CL_TRY(hipMemcpy(dx, x + at * d, 4 * (size_t)c * d, hipMemcpyHostToDevice));
         s.place(a.p + o_scratch, c, k);
-        CL_TRY(launch_cluster_norms(dx, c, d, s, dev.stream));
-        CL_TRY(launch_cluster_assign(dx, c, d, dc, k, di + at, s, dev.stream));
-        CL_TRY(hipEventRecord(dev.done[b], dev.stream));
+        CL_TRY(launch_cluster_norms(dx, c, d, s, stream));
+        CL_TRY(launch_cluster_assign(dx, c, d, dc, k, di + at, s, stream));
+        if (bufs > 1) CL_TRY(hipEventRecord(dev.done[b], stream));
     }
-    CL_TRY(hipStreamSynchronize(dev.stream));
+    CL_TRY(hipStreamSynchronize(stream));
     CL_TRY(hipMemcpy(ids, di, 4 * (size_t)n, hipMemcpyDeviceToHost));
     return GLASS_HIP_OK;
 }
