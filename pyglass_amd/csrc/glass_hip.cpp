@@ -1028,8 +1028,8 @@ int run_batch(glass_hip_searcher &s, const float *qs_dev, int32_t nq, const int3
         if (int r = state_for(s, stream, &st)) return r;
         if (int r = ensure_slots(s, *st, blocks * slots_per_block(lc), stream)) return r;
         if (!st->counter.p) {
-            HIP_TRY(st->counter.alloc(2));
-            HIP_TRY(launch_fill_i32(st->counter.p, 2, 0, stream));
+            HIP_TRY(st->counter.alloc(kWorkWords));
+            HIP_TRY(launch_fill_i32(st->counter.p, kWorkWords, 0, stream));
         }
     }
     int32_t *counter = bs ? bs->counter : st->counter.p;
@@ -1550,12 +1550,12 @@ int glass_hip_searcher_search_batch_dev_noalloc(glass_hip_searcher *s, const flo
         std::lock_guard<std::mutex> lk(s->mu);
         const int32_t max_cap = std::max(inner_k(*s, k), s->ef);
         if (int r = check_cap(*s, max_cap)) return r;
-        // the device's scratch array: [work counter | 256 bytes][one slot area per resident wave]
+        // the device's scratch array: [work counters][one slot area per resident wave]
         void *base = nullptr;
         size_t bytes = 0;
         if (int r = noalloc_scratch(s->device, &base, &bytes)) return r;
         const int64_t slot_bytes = 4 * slot_stride(*s);
-        const int64_t slots = ((int64_t)bytes - 256) / slot_bytes;
+        const int64_t slots = ((int64_t)bytes - 4 * kWorkWords) / slot_bytes;
         if (slots < 4)
             return fail(GLASS_HIP_EINVAL,
                         "%d rows need %lld bytes of scratch per wave: the %zu-byte no-alloc scratch holds fewer "
@@ -1578,10 +1578,10 @@ int glass_hip_searcher_search_batch_dev_noalloc(glass_hip_searcher *s, const flo
             }
         }
         // calls that overlapped on the array may have left its counter anywhere
-        HIP_TRY(launch_fill_i32((int32_t *)base, 2, 0, stream ? (hipStream_t)stream : s->stream));
+        HIP_TRY(launch_fill_i32((int32_t *)base, kWorkWords, 0, stream ? (hipStream_t)stream : s->stream));
         BatchState bs;
         bs.counter = (int32_t *)base;
-        bs.visited = (uint32_t *)((uint8_t *)base + 256);
+        bs.visited = (uint32_t *)base + kWorkWords;
         bs.max_slots = (int32_t)std::min<int64_t>(slots, 1 << 20);
         return run_batch(*s, qs_dev, nq, nullptr, nullptr, s->ef, k, max_cap, s->ef, mode, nullptr, dst_dev,
                          scores_dev, counters_dev, (hipStream_t)stream, &bs);
@@ -2521,8 +2521,8 @@ int glass_hip_server_create(glass_hip_searcher *s, int32_t max_batch, int32_t ma
             HIP_TRY(hipHostMalloc((void **)&sl.h_out, sv->out_bytes, hipHostMallocMapped | hipHostMallocCoherent));
             HIP_TRY(hipHostGetDevicePointer((void **)&sl.d_out, sl.h_out, 0));
             HIP_TRY(sl.d_in.alloc(sv->in_bytes));
-            HIP_TRY(sl.counter.alloc(2));
-            HIP_TRY(launch_fill_i32(sl.counter.p, 2, 0, s->stream));
+            HIP_TRY(sl.counter.alloc(kWorkWords));
+            HIP_TRY(launch_fill_i32(sl.counter.p, kWorkWords, 0, s->stream));
             sl.visited = sv->visited.p + (size_t)i * (size_t)sv->slots_per_batch * (size_t)s->vis_stride;
             HIP_TRY(hipStreamCreateWithFlags(&sl.stream, hipStreamNonBlocking));
             HIP_TRY(hipEventCreateWithFlags(&sl.done, hipEventDisableTiming));

@@ -79,6 +79,11 @@ struct LaunchConfig {
     int32_t qwaves;          // waves per query: 1, or 2 / 4 (waves_per_block) waves of a workgroup on one query
 };
 
+// Work counters of a launch: kWorkLines lines of kWorkLineWords words, each of
+// them [queries handed out, slots that have ended], and a word for the lines
+// whose slots have all ended.
+constexpr int32_t kWorkLines = 16, kWorkLineWords = 32, kWorkWords = (kWorkLines + 1) * kWorkLineWords;
+
 struct SlotState {
     uint32_t *visited;       // nslots x vis_stride words, each slot: [LUT | dirty list | visited bitset]; the
                              // bitsets are all zero between queries
@@ -87,7 +92,7 @@ struct SlotState {
     int32_t dirty_words;     // then the bitset words a query set first (multiple of 4), then the bitset
 
     int32_t nslots;
-    int32_t *work_counter;   // two words, zero between launches: queries handed out, slots that have ended
+    int32_t *work_counter;   // kWorkWords words, zero between launches
 };
 
 // Launches the persistent search kernel for one batch on `stream`.

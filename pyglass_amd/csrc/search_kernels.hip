@@ -1690,6 +1690,47 @@ __device__ __forceinline__ const KernelArgs &fresh_args() {
     return *(const KernelArgs *)p;
 }
 
+// The work counters of a launch with more queries than slots.  An atomic on
+// one address takes about 17 ns from anywhere on the device, so one counter
+// serves 60 queries per us: 4,000 queries of 337k x 63 SQ8U, ef 25, took 190 us
+// with it and 127 without.  kWorkLines of them, on lines of their own, take
+// 13,616 such queries from 383 to 339 us (10,000 of 1M x 128 SQ4U, ef 64, from
+// 872 to 842).  Counter h hands out the queries h, h + kWorkLines, ..., and a
+// slot that finds its own counter's all handed out takes from the next that
+// has some.  One wave; returns nq when none is left.
+__device__ __forceinline__ int take_query(int32_t *ctr, int nq, int slot) {
+    const int l = lane_id();
+    int h = slot % kWorkLines;
+    for (;;) {  // a pass that takes none has found one more counter used up
+        int t = 0;
+        if (l == 0) t = atomicAdd(ctr + h * kWorkLineWords, 1);
+        t = uni(t);
+        if (t <= (nq - 1 - h) / kWorkLines && h < nq) return t * kWorkLines + h;
+        const int v = l < kWorkLines && l < nq
+                          ? __hip_atomic_load(ctr + l * kWorkLineWords, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                          : 0x7fffffff;
+        const uint32_t left = (uint32_t)__ballot(v <= (nq - 1 - l) / kWorkLines);
+        if (!left) return nq;
+        const uint32_t after = left & (0xfffffffeu << h);
+        h = __builtin_ctz(after ? after : left);
+    }
+}
+
+// Counts a slot that takes no more; the last of the launch sets the counters
+// back to zero, so that a launch needs no other before it.  One lane.
+__device__ __forceinline__ void end_slot(int32_t *ctr, int nslots, int slot) {
+    const int h = slot % kWorkLines;
+    // every slot's last take came before its own count here
+    if (atomicAdd(ctr + h * kWorkLineWords + 1, 1) != (nslots - 1 - h) / kWorkLines) return;
+    const int groups = nslots < kWorkLines ? nslots : kWorkLines;
+    if (atomicAdd(ctr + kWorkLines * kWorkLineWords, 1) != groups - 1) return;
+    for (int i = 0; i < kWorkLines; ++i) {
+        atomicExch(ctr + i * kWorkLineWords, 0);
+        atomicExch(ctr + i * kWorkLineWords + 1, 0);
+    }
+    atomicExch(ctr + kWorkLines * kWorkLineWords, 0);
+}
+
 template <int V, int DPL, int P>
 __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<V, DPL, P>))) void search_kernel(KernelArgs) {
     constexpr bool kFast = P == 1;
@@ -1712,17 +1753,15 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
     const int slot = W > 1 ? (int)blockIdx.x : (int)blockIdx.x * fresh_args().lc.waves_per_block + wv;
 
     // A batch that fits the slots gives each slot the query of its number; a
-    // larger one hands its queries out through the work counter, which the
-    // last slot to end sets back to zero, so that a launch needs no other
-    // before it.
+    // larger one hands its queries out through the work counters.
     // The next query's index, and its row when ql <= 256 (xn, four floats
     // per lane), are requested before the current query's output phase, so
     // that their latency overlaps it.
     auto queued = [&](const KernelArgs &a) __attribute__((always_inline)) {
         return a.qb.nq > (W > 1 ? (int)gridDim.x : (int)gridDim.x * a.lc.waves_per_block);
     };
-    auto take = [&](const KernelArgs &a) __attribute__((always_inline)) {  // by one lane
-        return queued(a) ? atomicAdd(a.ss.work_counter, 1) : a.qb.nq;
+    auto take = [&](const KernelArgs &a) __attribute__((always_inline)) {  // by one wave
+        return queued(a) ? take_query(a.ss.work_counter, a.qb.nq, slot) : a.qb.nq;
     };
     // the first query: its slot's, or the next in the queue
     int qi_next = slot;
@@ -1730,13 +1769,14 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
         if (W > 1) {
             const KernelArgs &a = fresh_args();
             int32_t *const ctl = (int32_t *)(lds_raw + wave_lds_bytes(a.ix, a.lc.cap_max, a.lc.vis_hash));
-            if (lead && l == 0) ctl[0] = take(a);
+            if (lead) {
+                const int t = take(a);
+                if (l == 0) ctl[0] = t;
+            }
             __syncthreads();
             qi_next = uni(ctl[0]);
         } else {
-            int t = 0;
-            if (l == 0) t = take(fresh_args());
-            qi_next = uni(t);
+            qi_next = take(fresh_args());
         }
     }
     bool have_row = false;
@@ -2084,9 +2124,7 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
         // take the next query now (see above)
         const KernelArgs &ko = fresh_args();
         if (W == 1) {
-            int t = 0;
-            if (l == 0) t = take(ko);
-            qi_next = uni(t);
+            qi_next = take(ko);
             have_row = qi_next < ko.qb.nq && qf_len(ko.ix) <= 256;
             if (have_row) {
                 const float *xq = ko.qb.queries + (int64_t)qi_next * ko.qb.dim;
@@ -2186,7 +2224,10 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
             ko.qb.out_counters[(int64_t)qi * 3 + 2] = cnt_u;
         }
         if (W > 1) {
-            if (lead && l == 0) ctl[0] = take(ko);
+            if (lead) {
+                const int t = take(ko);
+                if (l == 0) ctl[0] = t;
+            }
             __syncthreads();
             qi_next = uni(ctl[0]);
         } else {
@@ -2194,14 +2235,8 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
         }
     }
     const KernelArgs &ke = fresh_args();
-    if (queued(ke) && lead && l == 0) {
-        const int nslots = W > 1 ? (int)gridDim.x : (int)gridDim.x * ke.lc.waves_per_block;
-        // every slot's last take came before its own count here
-        if (atomicAdd(ke.ss.work_counter + 1, 1) == nslots - 1) {
-            atomicExch(ke.ss.work_counter, 0);
-            atomicExch(ke.ss.work_counter + 1, 0);
-        }
-    }
+    if (queued(ke) && lead && l == 0)
+        end_slot(ke.ss.work_counter, W > 1 ? (int)gridDim.x : (int)gridDim.x * ke.lc.waves_per_block, slot);
 }
 
 // Whether a launch runs the P = 1 kernel: pools of at most 128 entries and,
@@ -2319,11 +2354,11 @@ hipError_t launch_int(const DeviceIndex &ix, const QueryBatch &qb, const LaunchC
 }  // namespace
 
 // Scratch of glass_hip_searcher_search_batch_dev_noalloc: the persistent
-// grid's work counter and one slot area (PQ8 lookup table, overflow visited
+// grid's work counters and one slot area (PQ8 lookup table, overflow visited
 // bitset) per resident wave, for callers that cannot allocate device memory.
 // Each device holds its own copy from module load until the process ends.
 // Host code uses the address noalloc_scratch returns, never this name.
-constexpr size_t kNoAllocScratchBytes = (size_t)128 << 20;
+constexpr size_t kNoAllocScratchBytes = ((size_t)128 << 20) - 256 + 4 * kWorkWords;
 static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 
 int noalloc_scratch(int device, void **ptr, size_t *bytes) {
