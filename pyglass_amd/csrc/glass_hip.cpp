@@ -906,7 +906,9 @@ int32_t untuned_qwaves(const glass_hip_searcher &s, int32_t team) {
 // 4,096 238, 1,024 265.  A wave or two are given for a table that holds what a
 // search is expected to visit, 3/8 of the rows that it expands, where the
 // other would not: 1M x 128 SQ2U, ef 128, 20,000 queries: 2,048 words (15
-// waves) 2,482, 1,024 (16 waves) 4,596, 4,096 (8 waves) 3,048.  Batches that
+// waves) 2,482, 1,024 (16 waves) 4,596, 4,096 (8 waves) 3,048; and for one that
+// is a bitset of every row: 60k x 96 SQ2U, ef 100, 12,000 queries: 2,048 words
+// (15 waves) 863, 1,024 (16 waves) 1,087.  Batches that
 // leave LDS unused take the words that make the set a bitset of every row
 // (graphs of up to 524k rows); a table beyond 4,096 words, 6,144 ids, would be
 // cleared for nothing.  A host call's batch is alone on the device until it
@@ -929,9 +931,8 @@ int32_t untuned_vis(const glass_hip_searcher &s, LaunchConfig lc, int64_t nq, in
     auto holds = [&](int32_t v) { return ix.N <= 32 * v || 3 * (int64_t)v / 2 >= visits + visits / 4; };
     int32_t v = 4096;
     while (v > 256 && blocks(v) < want) v /= 2;
-    if (!holds(v))
-        for (int32_t u = 2 * v; u <= 4096 && 20 * blocks(u) >= 17 * want; u *= 2)
-            if (holds(u)) return u;
+    for (int32_t u = 2 * v; u <= 4096 && 20 * blocks(u) >= 17 * want; u *= 2)
+        if ((!holds(v) && holds(u)) || (ix.N > 32 * v && ix.N <= 32 * u)) return u;
     return v;
 }
 
