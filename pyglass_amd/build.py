@@ -10,6 +10,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -18,6 +19,8 @@ LIB = os.path.join(HERE, "libglass_hip.so")
 
 SOURCES = ["search_kernels.hip", "encode_kernels.hip", "cluster_kernels.hip", "glass_hip.cpp", "clustering.cpp"]
 HOST_SOURCES = ["graph_build.cpp"]
+# Sources compiled as several units, told apart by -D<name>=0, 1, ...
+SOURCE_PARTS = {"search_kernels.hip": ("GLASS_SEARCH_PART", 7)}
 ARCH = os.environ.get("GLASS_HIP_ARCH", "gfx950")
 
 HIPCC_FLAGS = [
@@ -50,18 +53,28 @@ def build(verbose: bool = False) -> str:
     objs = []
     obj_dir = os.path.join(CSRC, "_build")
     os.makedirs(obj_dir, exist_ok=True)
+    units = []
     for src in SOURCES:
-        obj = os.path.join(obj_dir, os.path.splitext(src)[0] + ".o")
-        cmd = [hipcc(), *HIPCC_FLAGS, *SOURCE_FLAGS.get(src, []), "-c", os.path.join(CSRC, src), "-o", obj]
-        if verbose:
-            print(" ".join(cmd), flush=True)
-        r = subprocess.run(cmd, capture_output=True, text=True)
-        errs = "\n".join(ln for ln in (r.stderr or "").splitlines() if "packed-fp32-ops" not in ln)
-        if r.returncode != 0:
-            raise RuntimeError(f"hipcc failed for {src}:\n{errs}")
-        if verbose and errs.strip():
-            print(errs)
-        objs.append(obj)
+        name, parts = SOURCE_PARTS.get(src, (None, 1))
+        for part in range(parts):
+            obj = os.path.join(obj_dir, os.path.splitext(src)[0] + (f"_{part}" if name else "") + ".o")
+            define = [f"-D{name}={part}"] if name else []
+            units.append((src, obj, [hipcc(), *HIPCC_FLAGS, *SOURCE_FLAGS.get(src, []), *define, "-c",
+                                     os.path.join(CSRC, src), "-o", obj]))
+
+    def compile_unit(unit):
+        return subprocess.run(unit[2], capture_output=True, text=True)
+
+    with ThreadPoolExecutor(min(len(units), os.cpu_count() or 1, 8)) as pool:
+        for (src, obj, cmd), r in zip(units, pool.map(compile_unit, units)):
+            if verbose:
+                print(" ".join(cmd), flush=True)
+            errs = "\n".join(ln for ln in (r.stderr or "").splitlines() if "packed-fp32-ops" not in ln)
+            if r.returncode != 0:
+                raise RuntimeError(f"hipcc failed for {src}:\n{errs}")
+            if verbose and errs.strip():
+                print(errs)
+            objs.append(obj)
     # CPU graph builder: plain C++ for the host (AVX2/FMA baseline shared by
     # the build container and the GPU hosts)
     for src in HOST_SOURCES:

@@ -26,7 +26,25 @@
 #include "glass_hip.h"
 #include "glass_hip_internal.h"
 
+// The kernels take minutes to compile in one unit; GLASS_SEARCH_PART = 0..6
+// compiles the file to one of seven units that together are the whole.
+#ifdef GLASS_SEARCH_PART
+#define GLASS_SEARCH_HAS(part) (GLASS_SEARCH_PART == (part))
+#else
+#define GLASS_SEARCH_HAS(part) 1
+#endif
+
 namespace glass_hip {
+
+// What a launch needs of one quantizer's kernels.
+struct KernelOps {
+    int (*vgprs)(const DeviceIndex &, const LaunchConfig &);
+    int (*blocks_per_cu)(const DeviceIndex &, const LaunchConfig &);
+    hipError_t (*launch)(const DeviceIndex &, const QueryBatch &, const LaunchConfig &, const SlotState &, hipStream_t);
+};
+const KernelOps *ops_sq8u_l2(int32_t team), *ops_sq8u_ip(int32_t team), *ops_sq4u(int32_t team), *ops_sq2u(int32_t team);
+const KernelOps *ops_sq8(bool l2), *ops_e5m2(bool l2), *ops_fp32(bool l2), *ops_fp16(bool l2), *ops_bf16(bool l2),
+    *ops_sq6(bool l2), *ops_sq4(bool l2), *ops_pq8(bool l2);
 
 namespace {
 
@@ -1489,9 +1507,13 @@ __device__ __forceinline__ void pool_merge_lds(const WaveLds &w, PoolState &ps, 
     ps.cur = uni(new_cur);
 }
 
+// v_writelane: `old` with lane `lane`'s word replaced by `v` (both uniform).
+// It takes the lane from m0, which costs the two-chunk merge what it saves.
+extern "C" __device__ int writelane(int v, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
+
 // Pools of up to kMaxChunks*64 entries are merged from registers: lane l
-// holds entries l, l+64, ... of the pool, NCH chunks of 64 (NCH = 2 when the
-// launch's pools hold at most 128 entries, else 4).  Each candidate's insertion point
+// holds entries l, l+64, ... of the pool, NCH chunks of 64 (NCH = 1 or 2 when the
+// launch's pools hold at most 64 or 128 entries, else 4).  Each candidate's insertion point
 // (entries with key <= its key) is a sum of ballots, the first moved entry
 // and the first inserted position come from the rank-0 candidate, and all
 // writes happen after all reads.  The node the next pop will take is known
@@ -1588,7 +1610,11 @@ __device__ __forceinline__ uint32_t pool_merge_reg(const DeviceIndex &ix, const 
         uint64_t mm = am;
         while (mm) {
             const int i = __builtin_ctzll(mm);
-            mm &= ~(1ull << i);
+            if (NCH == 1) {
+                asm("s_bitset0_b64 %0, %1" : "+s"(mm) : "s"(i));  // one instruction for the two of the other form
+            } else {
+                mm &= ~(1ull << i);
+            }
             const uint32_t ki = (uint32_t)__builtin_amdgcn_readlane((int)kj, i);
             r += (((uint64_t)ki << 32) | (uint32_t)i) < kl;
             // unused chunks hold kKeyMax, which no distance key reaches, so
@@ -1600,7 +1626,7 @@ __device__ __forceinline__ uint32_t pool_merge_reg(const DeviceIndex &ix, const 
                 cnt += __builtin_popcountll(ballot(below));
                 le[c] += below;
             }
-            ub = (l == i) ? cnt : ub;
+            ub = NCH == 1 ? writelane(cnt, i, ub) : ((l == i) ? cnt : ub);
         }
     }
     if (am) {
@@ -1656,10 +1682,15 @@ __device__ __forceinline__ void put_result(const QueryBatch &qb, int64_t pos, in
 // The search kernel.  P = 1 is the common case compiled on its own: pools of
 // at most 128 entries (two-chunk register merge) and, for integer codes, the
 // all-neighbour gather; the other paths are left out, which keeps the hot
-// loop small and its scalar registers unspilled.  P = 0 handles everything
-// with one wave per query; P = 2 is the same with the waves of a workgroup
-// sharing each query (LaunchConfig::qwaves), compiled apart so that the
-// other two carry none of its code.
+// loop small and its scalar registers unspilled.  P = 3 is that for pools of
+// at most 64 entries, merged as one chunk: a third of the merge's
+// instructions, and its loop is what one wave waits for between two nodes'
+// loads.  (200k x 128 SQ4U, ef 48, 1 / 1,000 / 8,000 queries: 103 / 237 / 497 us
+// with two chunks, 95 / 227 / 468 with one; both merges in one kernel cost pools
+// of more than 64 entries 3%.)  P = 0 handles everything with one wave per
+// query; P = 2 is the same with the waves of a workgroup sharing each query
+// (LaunchConfig::qwaves), compiled apart so that the others carry none of its
+// code.
 
 // Register budgets: the common path keeps at least 4 waves per SIMD (at most
 // 128 VGPRs; left to itself the compiler schedules the re-rank's loads into
@@ -1671,7 +1702,7 @@ __device__ __forceinline__ void put_result(const QueryBatch &qb, int64_t pos, in
 // two rows, the query and two calibration rows in flight.
 template <int V, int DPL, int P>
 constexpr int kWavesPerEu =
-    P == 1 ? ((V == V_SQ2U && DPL == 16) || V == V_SQ8_L2 || V == V_SQ8_IP ? 3 : 4) : (P == 2 ? 2 : 3);
+    P == 1 || P == 3 ? ((V == V_SQ2U && DPL == 16) || V == V_SQ8_L2 || V == V_SQ8_IP ? 3 : 4) : (P == 2 ? 2 : 3);
 
 struct KernelArgs {
     DeviceIndex ix;
@@ -1733,13 +1764,14 @@ __device__ __forceinline__ void end_slot(int32_t *ctr, int nslots, int slot) {
 
 template <int V, int DPL, int P>
 __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<V, DPL, P>))) void search_kernel(KernelArgs) {
-    constexpr bool kFast = P == 1;
+    constexpr bool kFast = P == 1 || P == 3;
+    constexpr int kChunks = P == 3 ? 1 : 2;  // of a register merge
     // registers of float rows' loads in flight, in the search and in the re-rank of long rows
     constexpr bool kSq8 = V == V_SQ8_L2 || V == V_SQ8_IP;  // its LDS rows take registers too
-    constexpr int kRowRegs = kSq8 ? (P == 2 ? 32 : 16) : (P == 1 ? 16 : (P == 2 ? 64 : 32));
-    constexpr int kRerankRegs = P == 1 ? 32 : 48;
+    constexpr int kRowRegs = kSq8 ? (P == 2 ? 32 : 16) : (kFast ? 16 : (P == 2 ? 64 : 32));
+    constexpr int kRerankRegs = kFast ? 32 : 48;
     // passes of integer code rows in flight at once, as the register budget allows
-    constexpr int kAhead = DPL == 16 && (P == 1 || (P == 0 && V == V_SQ2U)) ? 1 : 2;
+    constexpr int kAhead = DPL == 16 && (kFast || (P == 0 && V == V_SQ2U)) ? 1 : 2;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     const int l = lane_id();
     const int wv = uni((int)(threadIdx.x >> 6));
@@ -2017,7 +2049,9 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
                 __syncthreads();
                 if (lead) {
                     cnt_d += m;
-                    if (at_use(lc.cap_max) <= 128) {
+                    if (ps.cap <= 64) {
+                        pred = pool_merge_reg_lds<1>(ix, w, ps, m, pred_row);
+                    } else if (at_use(lc.cap_max) <= 128) {
                         pred = pool_merge_reg_lds<2>(ix, w, ps, m, pred_row);
                     } else if (lc.cap_max <= 64 * kMaxChunks) {
                         pred = pool_merge_reg_lds<kMaxChunks>(ix, w, ps, m, pred_row);
@@ -2061,7 +2095,7 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
                 vs.account(m, (uint32_t)v);
                 cnt_d += m;
                 if (kFast || at_use(lc.cap_max) <= 128) {
-                    pred = pool_merge_reg<2>(ix, w, ps, kj, (uint32_t)v, isnew, nm, nj, pred_row);
+                    pred = pool_merge_reg<kChunks>(ix, w, ps, kj, (uint32_t)v, isnew, nm, nj, pred_row);
                 } else if (lc.cap_max <= 64 * kMaxChunks) {
                     pred = pool_merge_reg<kMaxChunks>(ix, w, ps, kj, (uint32_t)v, isnew, nm, nj, pred_row);
                 } else {
@@ -2098,7 +2132,7 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
                     dists(m, qb.mode);
                     cnt_d += m;
                     if (kFast || at_use(lc.cap_max) <= 128) {
-                        pred = pool_merge_reg_lds<2>(ix, w, ps, m, pred_row);
+                        pred = pool_merge_reg_lds<kChunks>(ix, w, ps, m, pred_row);
                     } else if (lc.cap_max <= 64 * kMaxChunks) {
                         pred = pool_merge_reg_lds<kMaxChunks>(ix, w, ps, m, pred_row);
                     } else {
@@ -2239,7 +2273,7 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
         end_slot(ke.ss.work_counter, W > 1 ? (int)gridDim.x : (int)gridDim.x * ke.lc.waves_per_block, slot);
 }
 
-// Whether a launch runs the P = 1 kernel: pools of at most 128 entries and,
+// Whether a launch runs the P = 1 or P = 3 kernel: pools of at most 128 entries and,
 // for integer codes, the all-neighbour gather with one lane group per
 // neighbour (slot * K <= 64, slot as IntQuery::init computes it).
 template <int V, int DPL>
@@ -2255,11 +2289,17 @@ bool fast_path(const DeviceIndex &ix, const LaunchConfig &lc) {
     return slot * ix.K <= 64;
 }
 
+// P of the kernel that a launch runs.
 template <int V, int DPL>
-const void *kernel_fn(const DeviceIndex &ix, const LaunchConfig &lc) {
-    if (lc.qwaves > 1) return (const void *)search_kernel<V, DPL, 2>;
-    return fast_path<V, DPL>(ix, lc) ? (const void *)search_kernel<V, DPL, 1> : (const void *)search_kernel<V, DPL, 0>;
+int path_of(const DeviceIndex &ix, const LaunchConfig &lc) {
+    if (lc.qwaves > 1) return 2;
+    if (!fast_path<V, DPL>(ix, lc)) return 0;
+    return lc.cap_max <= 64 ? 3 : 1;
 }
+
+template <int V, int DPL>
+constexpr void (*kKernels[4])(KernelArgs) = {search_kernel<V, DPL, 0>, search_kernel<V, DPL, 1>,
+                                             search_kernel<V, DPL, 2>, search_kernel<V, DPL, 3>};
 
 // A workgroup whose waves share one query: its query area plus the two
 // control words (query index, candidates of the expansion), rounded to 16.
@@ -2276,24 +2316,12 @@ hipError_t launch_one(const DeviceIndex &ix, const QueryBatch &qb, const LaunchC
     const size_t lds = block_lds_bytes(ix, lc);
     static bool attr_set = false;
     if (!attr_set) {
-        (void)hipFuncSetAttribute((const void *)search_kernel<V, DPL, 0>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  160 * 1024);
-        (void)hipFuncSetAttribute((const void *)search_kernel<V, DPL, 1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  160 * 1024);
-        (void)hipFuncSetAttribute((const void *)search_kernel<V, DPL, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  160 * 1024);
+        for (auto f : kKernels<V, DPL>)
+            (void)hipFuncSetAttribute((const void *)f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         attr_set = true;
     }
-    if (lc.qwaves > 1) {
-        hipLaunchKernelGGL((search_kernel<V, DPL, 2>), dim3(lc.blocks), dim3(64 * lc.waves_per_block), lds, stream,
-                           KernelArgs{ix, qb, lc, ss});
-    } else if (fast_path<V, DPL>(ix, lc)) {
-        hipLaunchKernelGGL((search_kernel<V, DPL, 1>), dim3(lc.blocks), dim3(64 * lc.waves_per_block), lds, stream,
-                           KernelArgs{ix, qb, lc, ss});
-    } else {
-        hipLaunchKernelGGL((search_kernel<V, DPL, 0>), dim3(lc.blocks), dim3(64 * lc.waves_per_block), lds, stream,
-                           KernelArgs{ix, qb, lc, ss});
-    }
+    hipLaunchKernelGGL((kKernels<V, DPL>[path_of<V, DPL>(ix, lc)]), dim3(lc.blocks), dim3(64 * lc.waves_per_block), lds,
+                       stream, KernelArgs{ix, qb, lc, ss});
     return hipGetLastError();
 }
 
@@ -2301,12 +2329,12 @@ hipError_t launch_one(const DeviceIndex &ix, const QueryBatch &qb, const LaunchC
 // (the launch rules look at several shapes per call).  0 on error.
 template <int V, int DPL>
 int vgprs_one(const DeviceIndex &ix, const LaunchConfig &lc) {
-    static std::atomic<int> known[3] = {};
-    const int path = lc.qwaves > 1 ? 2 : (fast_path<V, DPL>(ix, lc) ? 1 : 0);
+    static std::atomic<int> known[4] = {};
+    const int path = path_of<V, DPL>(ix, lc);
     int v = known[path].load(std::memory_order_relaxed);
     if (v == 0) {
         hipFuncAttributes attr;
-        if (hipFuncGetAttributes(&attr, kernel_fn<V, DPL>(ix, lc)) != hipSuccess) return 0;
+        if (hipFuncGetAttributes(&attr, (const void *)kKernels<V, DPL>[path]) != hipSuccess) return 0;
         v = attr.numRegs;
         known[path].store(v, std::memory_order_relaxed);
     }
@@ -2330,28 +2358,68 @@ int occupancy_one(const DeviceIndex &ix, const LaunchConfig &lc) {
     return nb;
 }
 
-template <int V>
-int occupancy_int(const DeviceIndex &ix, const LaunchConfig &lc) {
-    switch (lc.team) {
-        case 4: return occupancy_one<V, 4>(ix, lc);
-        case 8: return occupancy_one<V, 8>(ix, lc);
-        case 16: return occupancy_one<V, 16>(ix, lc);
-        default: return 0;
-    }
-}
+template <int V, int DPL>
+constexpr KernelOps kOps = {vgprs_one<V, DPL>, occupancy_one<V, DPL>, launch_one<V, DPL>};
 
+// The kernels of an integer quantizer by team; the others always use 16-lane segments.
 template <int V>
-hipError_t launch_int(const DeviceIndex &ix, const QueryBatch &qb, const LaunchConfig &lc, const SlotState &ss,
-                      hipStream_t stream) {
-    switch (lc.team) {
-        case 4: return launch_one<V, 4>(ix, qb, lc, ss, stream);
-        case 8: return launch_one<V, 8>(ix, qb, lc, ss, stream);
-        case 16: return launch_one<V, 16>(ix, qb, lc, ss, stream);
-        default: return hipErrorInvalidValue;
+const KernelOps *int_ops(int32_t team) {
+    switch (team) {
+        case 4: return &kOps<V, 4>;
+        case 8: return &kOps<V, 8>;
+        case 16: return &kOps<V, 16>;
+        default: return nullptr;
     }
 }
 
 }  // namespace
+
+#if GLASS_SEARCH_HAS(0)
+const KernelOps *ops_sq8u_l2(int32_t team) { return int_ops<V_SQ8U_L2>(team); }
+#endif
+#if GLASS_SEARCH_HAS(1)
+const KernelOps *ops_sq8u_ip(int32_t team) { return int_ops<V_SQ8U_IP>(team); }
+#endif
+#if GLASS_SEARCH_HAS(2)
+const KernelOps *ops_sq4u(int32_t team) { return int_ops<V_SQ4U>(team); }
+#endif
+#if GLASS_SEARCH_HAS(3)
+const KernelOps *ops_sq2u(int32_t team) { return int_ops<V_SQ2U>(team); }
+#endif
+#if GLASS_SEARCH_HAS(4)
+const KernelOps *ops_sq8(bool l2) { return l2 ? &kOps<V_SQ8_L2, 4> : &kOps<V_SQ8_IP, 4>; }
+const KernelOps *ops_e5m2(bool l2) { return l2 ? &kOps<V_E5M2_L2, 4> : &kOps<V_E5M2_IP, 4>; }
+#endif
+#if GLASS_SEARCH_HAS(5)
+const KernelOps *ops_fp32(bool l2) { return l2 ? &kOps<V_FP32_L2, 4> : &kOps<V_FP32_IP, 4>; }
+const KernelOps *ops_fp16(bool l2) { return l2 ? &kOps<V_FP16_L2, 4> : &kOps<V_FP16_IP, 4>; }
+const KernelOps *ops_bf16(bool l2) { return l2 ? &kOps<V_BF16_L2, 4> : &kOps<V_BF16_IP, 4>; }
+#endif
+#if GLASS_SEARCH_HAS(6)
+const KernelOps *ops_sq6(bool l2) { return l2 ? &kOps<V_SQ6_L2, 4> : &kOps<V_SQ6_IP, 4>; }
+const KernelOps *ops_sq4(bool l2) { return l2 ? &kOps<V_SQ4_L2, 4> : &kOps<V_SQ4_IP, 4>; }
+const KernelOps *ops_pq8(bool l2) { return l2 ? &kOps<V_PQ8_L2, 4> : &kOps<V_PQ8_IP, 4>; }
+#endif
+
+#if GLASS_SEARCH_HAS(0)
+// The kernels of an index, or null.
+static const KernelOps *ops_of(const DeviceIndex &ix, const LaunchConfig &lc) {
+    const bool l2 = ix.metric == MK_L2;
+    switch (ix.quant) {
+        case QK_SQ8U: return l2 ? ops_sq8u_l2(lc.team) : ops_sq8u_ip(lc.team);
+        case QK_SQ4U: return ops_sq4u(lc.team);
+        case QK_SQ2U: return ops_sq2u(lc.team);
+        case QK_E5M2: return ops_e5m2(l2);
+        case QK_SQ8: return ops_sq8(l2);
+        case QK_FP32: return ops_fp32(l2);
+        case QK_FP16: return ops_fp16(l2);
+        case QK_BF16: return ops_bf16(l2);
+        case QK_SQ6: return ops_sq6(l2);
+        case QK_SQ4: return ops_sq4(l2);
+        case QK_PQ8: return ops_pq8(l2);
+        default: return nullptr;
+    }
+}
 
 // Scratch of glass_hip_searcher_search_batch_dev_noalloc: the persistent
 // grid's work counters and one slot area (PQ8 lookup table, overflow visited
@@ -2388,50 +2456,14 @@ size_t lds_bytes_per_wave(const DeviceIndex &ix, int32_t cap_max, int32_t vis_ha
 
 size_t lds_bytes_per_block(const DeviceIndex &ix, const LaunchConfig &lc) { return block_lds_bytes(ix, lc); }
 
-template <int V>
-int vgprs_int(const DeviceIndex &ix, const LaunchConfig &lc) {
-    switch (lc.team) {
-        case 4: return vgprs_one<V, 4>(ix, lc);
-        case 8: return vgprs_one<V, 8>(ix, lc);
-        case 16: return vgprs_one<V, 16>(ix, lc);
-        default: return 0;
-    }
-}
-
 int kernel_vgprs(const DeviceIndex &ix, const LaunchConfig &lc) {
-    const bool l2 = ix.metric == MK_L2;
-    switch (ix.quant) {
-        case QK_SQ8U: return l2 ? vgprs_int<V_SQ8U_L2>(ix, lc) : vgprs_int<V_SQ8U_IP>(ix, lc);
-        case QK_SQ4U: return vgprs_int<V_SQ4U>(ix, lc);
-        case QK_SQ2U: return vgprs_int<V_SQ2U>(ix, lc);
-        case QK_E5M2: return l2 ? vgprs_one<V_E5M2_L2, 4>(ix, lc) : vgprs_one<V_E5M2_IP, 4>(ix, lc);
-        case QK_SQ8: return l2 ? vgprs_one<V_SQ8_L2, 4>(ix, lc) : vgprs_one<V_SQ8_IP, 4>(ix, lc);
-        case QK_FP32: return l2 ? vgprs_one<V_FP32_L2, 4>(ix, lc) : vgprs_one<V_FP32_IP, 4>(ix, lc);
-        case QK_FP16: return l2 ? vgprs_one<V_FP16_L2, 4>(ix, lc) : vgprs_one<V_FP16_IP, 4>(ix, lc);
-        case QK_BF16: return l2 ? vgprs_one<V_BF16_L2, 4>(ix, lc) : vgprs_one<V_BF16_IP, 4>(ix, lc);
-        case QK_SQ6: return l2 ? vgprs_one<V_SQ6_L2, 4>(ix, lc) : vgprs_one<V_SQ6_IP, 4>(ix, lc);
-        case QK_SQ4: return l2 ? vgprs_one<V_SQ4_L2, 4>(ix, lc) : vgprs_one<V_SQ4_IP, 4>(ix, lc);
-        case QK_PQ8: return l2 ? vgprs_one<V_PQ8_L2, 4>(ix, lc) : vgprs_one<V_PQ8_IP, 4>(ix, lc);
-        default: return 0;
-    }
+    const KernelOps *ops = ops_of(ix, lc);
+    return ops ? ops->vgprs(ix, lc) : 0;
 }
 
 int max_blocks_per_cu(const DeviceIndex &ix, const LaunchConfig &lc) {
-    const bool l2 = ix.metric == MK_L2;
-    switch (ix.quant) {
-        case QK_SQ8U: return l2 ? occupancy_int<V_SQ8U_L2>(ix, lc) : occupancy_int<V_SQ8U_IP>(ix, lc);
-        case QK_SQ4U: return occupancy_int<V_SQ4U>(ix, lc);
-        case QK_SQ2U: return occupancy_int<V_SQ2U>(ix, lc);
-        case QK_E5M2: return l2 ? occupancy_one<V_E5M2_L2, 4>(ix, lc) : occupancy_one<V_E5M2_IP, 4>(ix, lc);
-        case QK_SQ8: return l2 ? occupancy_one<V_SQ8_L2, 4>(ix, lc) : occupancy_one<V_SQ8_IP, 4>(ix, lc);
-        case QK_FP32: return l2 ? occupancy_one<V_FP32_L2, 4>(ix, lc) : occupancy_one<V_FP32_IP, 4>(ix, lc);
-        case QK_FP16: return l2 ? occupancy_one<V_FP16_L2, 4>(ix, lc) : occupancy_one<V_FP16_IP, 4>(ix, lc);
-        case QK_BF16: return l2 ? occupancy_one<V_BF16_L2, 4>(ix, lc) : occupancy_one<V_BF16_IP, 4>(ix, lc);
-        case QK_SQ6: return l2 ? occupancy_one<V_SQ6_L2, 4>(ix, lc) : occupancy_one<V_SQ6_IP, 4>(ix, lc);
-        case QK_SQ4: return l2 ? occupancy_one<V_SQ4_L2, 4>(ix, lc) : occupancy_one<V_SQ4_IP, 4>(ix, lc);
-        case QK_PQ8: return l2 ? occupancy_one<V_PQ8_L2, 4>(ix, lc) : occupancy_one<V_PQ8_IP, 4>(ix, lc);
-        default: return 0;
-    }
+    const KernelOps *ops = ops_of(ix, lc);
+    return ops ? ops->blocks_per_cu(ix, lc) : 0;
 }
 
 bool team_valid(const DeviceIndex &ix, int32_t team) {
@@ -2451,25 +2483,11 @@ int32_t default_team(const DeviceIndex &ix) {
     return 16;
 }
 
-// Per-dword "DPL" is the team selector for integer quantizers; float
-// quantizers always use 16-lane segments.
 hipError_t launch_search(const DeviceIndex &ix, const QueryBatch &qb, const LaunchConfig &lc, const SlotState &ss,
                          hipStream_t stream) {
-    const bool l2 = ix.metric == MK_L2;
-    switch (ix.quant) {
-        case QK_SQ8U: return l2 ? launch_int<V_SQ8U_L2>(ix, qb, lc, ss, stream) : launch_int<V_SQ8U_IP>(ix, qb, lc, ss, stream);
-        case QK_SQ4U: return launch_int<V_SQ4U>(ix, qb, lc, ss, stream);
-        case QK_SQ2U: return launch_int<V_SQ2U>(ix, qb, lc, ss, stream);
-        case QK_E5M2: return l2 ? launch_one<V_E5M2_L2, 4>(ix, qb, lc, ss, stream) : launch_one<V_E5M2_IP, 4>(ix, qb, lc, ss, stream);
-        case QK_SQ8: return l2 ? launch_one<V_SQ8_L2, 4>(ix, qb, lc, ss, stream) : launch_one<V_SQ8_IP, 4>(ix, qb, lc, ss, stream);
-        case QK_FP32: return l2 ? launch_one<V_FP32_L2, 4>(ix, qb, lc, ss, stream) : launch_one<V_FP32_IP, 4>(ix, qb, lc, ss, stream);
-        case QK_FP16: return l2 ? launch_one<V_FP16_L2, 4>(ix, qb, lc, ss, stream) : launch_one<V_FP16_IP, 4>(ix, qb, lc, ss, stream);
-        case QK_BF16: return l2 ? launch_one<V_BF16_L2, 4>(ix, qb, lc, ss, stream) : launch_one<V_BF16_IP, 4>(ix, qb, lc, ss, stream);
-        case QK_SQ6: return l2 ? launch_one<V_SQ6_L2, 4>(ix, qb, lc, ss, stream) : launch_one<V_SQ6_IP, 4>(ix, qb, lc, ss, stream);
-        case QK_SQ4: return l2 ? launch_one<V_SQ4_L2, 4>(ix, qb, lc, ss, stream) : launch_one<V_SQ4_IP, 4>(ix, qb, lc, ss, stream);
-        case QK_PQ8: return l2 ? launch_one<V_PQ8_L2, 4>(ix, qb, lc, ss, stream) : launch_one<V_PQ8_IP, 4>(ix, qb, lc, ss, stream);
-        default: return hipErrorInvalidValue;
-    }
+    const KernelOps *ops = ops_of(ix, lc);
+    return ops ? ops->launch(ix, qb, lc, ss, stream) : hipErrorInvalidValue;
 }
+#endif  // part 0
 
 }  // namespace glass_hip
