@@ -812,9 +812,11 @@ int32_t slots_per_block(const LaunchConfig &lc) { return lc.qwaves > 1 ? 1 : lc.
 // is 256 KB and more, and the list is longer: a query's first thousands of
 // ids come from its table, recorded one word each.  Above 64M rows it is short
 // again: the fixed scratch array of the no-alloc entry point is nearly used up
-// by four bitsets there.
+// by four bitsets there.  A list longer than a quarter of a small bitset saves
+// little of its clearing and is most of the slot.
 int32_t dirty_words(const glass_hip_searcher &s) {
-    return s.graph.N > (2 << 20) && s.graph.N <= (64 << 20) ? 16384 : 4096;
+    const int32_t words = s.graph.N > (2 << 20) && s.graph.N <= (64 << 20) ? 16384 : 4096;
+    return std::min(words, std::max(64, (s.graph.N / 32 / 4 + 3) / 4 * 4));
 }
 
 // Words of slot scratch per resident wave: the PQ8 lookup table, the dirty
