@@ -18,7 +18,7 @@
 //     merge reproduces sequential LinearPool::insert exactly: the pool after
 //     inserting c_1..c_m in order holds the `cap` smallest (dist, insertion
 //     order) keys, and `cur_` is the first unchecked index.
-// A persistent grid pulls queries from a device work counter, so one launch
+// A persistent grid pulls queries from device work counters, so one launch
 // serves any number of queries with per-query ef / k.
 #include <atomic>
 #include <mutex>
