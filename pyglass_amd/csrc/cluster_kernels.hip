@@ -2,6 +2,8 @@
 // glass/algorithms/clustering.hpp:198-232), the centroid update
 // (clustering.hpp:234-256) and the distances of k-means++ seeding
 // (clustering.hpp:138-196).  Every result is bit-equal to the reference's.
+#include <algorithm>
+
 #include "glass_hip_internal.h"
 
 namespace glass_hip {
@@ -392,8 +394,12 @@ int32_t filter_splits(int32_t n, int32_t k) {
 
 }  // namespace
 
+// Fewer rows are split further, so the layout for fewer rows can be the larger
+// one: with b = ceil(c / 64) workgroups, the splits times the rows c are at most
+// (1023 + b) / b * 64 b, and at most cent_tiles times the rows.
 size_t AssignScratch::bytes(int32_t n, int32_t k) {
-    const size_t part = (size_t)filter_splits(n, k) * n;
+    const size_t blocks = ((size_t)n + kRows - 1) / kRows;
+    const size_t part = std::min((size_t)cent_tiles(k) * n, (1023 + blocks) * kRows);
     return 4 * (2 * (size_t)n + (size_t)k + 3 * part + 2);
 }
 

@@ -158,7 +158,7 @@ struct AssignScratch {
     float *x2, *c2, *m1, *m2;  // squared norms of rows and centroids, least and second least values
     int32_t *i1, *list, *count;
     uint32_t *c2max;
-    static size_t bytes(int32_t n, int32_t k);
+    static size_t bytes(int32_t n, int32_t k);  // what place() takes for any number of rows up to n
     void place(void *p, int32_t n, int32_t k);
 };
 
