@@ -2524,10 +2524,12 @@ int glass_hip_server_create(glass_hip_searcher *s, int32_t max_batch, int32_t ma
             HIP_TRY(hipHostMalloc((void **)&sl.h_out, sv->out_bytes, hipHostMallocMapped | hipHostMallocCoherent));
             HIP_TRY(hipHostGetDevicePointer((void **)&sl.d_out, sl.h_out, 0));
             HIP_TRY(sl.d_in.alloc(sv->in_bytes));
-            HIP_TRY(sl.counter.alloc(kWorkWords));
-            HIP_TRY(launch_fill_i32(sl.counter.p, kWorkWords, 0, s->stream));
             sl.visited = sv->visited.p + (size_t)i * (size_t)sv->slots_per_batch * (size_t)s->vis_stride;
             HIP_TRY(hipStreamCreateWithFlags(&sl.stream, hipStreamNonBlocking));
+            // cleared on the stream that the slot's batches run on: the searcher's
+            // may be held up by other callers' work
+            HIP_TRY(sl.counter.alloc(kWorkWords));
+            HIP_TRY(launch_fill_i32(sl.counter.p, kWorkWords, 0, sl.stream));
             HIP_TRY(hipEventCreateWithFlags(&sl.done, hipEventDisableTiming));
         }
         glass_hip_server *p = sv.get();
