@@ -1565,19 +1565,21 @@ int glass_hip_searcher_search_batch_dev_noalloc(glass_hip_searcher *s, const flo
                         "than 4 waves",
                         s->graph.N, (long long)slot_bytes, bytes);
         // The bitsets must be all zero between queries; every query leaves
-        // its own so, but a different slot layout (another searcher's N or
-        // PQ8 table) reads other words as bitsets: zero the array then.
+        // its own so, but a different slot layout (another searcher's N, PQ8
+        // table or dirty list, which N sets too: slots of one size can be
+        // divided in two ways) reads other words as bitsets: zero the array then.
         {
             static std::mutex lay_mu;
-            static int64_t lay_stride[64] = {}, lay_lut[64] = {};
+            static int64_t lay_stride[64] = {}, lay_lut[64] = {}, lay_dirty[64] = {};
             const int d = s->device;
             std::lock_guard<std::mutex> g(lay_mu);
             if (d < 0 || d >= 64) return fail(GLASS_HIP_EINVAL, "device index out of range");
-            if (lay_stride[d] != slot_stride(*s) || lay_lut[d] != s->lut_words) {
+            if (lay_stride[d] != slot_stride(*s) || lay_lut[d] != s->lut_words || lay_dirty[d] != dirty_words(*s)) {
                 hipStream_t st = stream ? (hipStream_t)stream : s->stream;
                 HIP_TRY(launch_fill_i32((int32_t *)base, (int64_t)(bytes / 4), 0, st));
                 lay_stride[d] = slot_stride(*s);
                 lay_lut[d] = s->lut_words;
+                lay_dirty[d] = dirty_words(*s);
             }
         }
         // calls that overlapped on the array may have left its counter anywhere
