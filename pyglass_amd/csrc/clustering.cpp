@@ -276,15 +276,31 @@ int fit_device(const float *rows, int32_t n, int32_t d, int32_t k, int32_t epoch
 
 // A clustering object's stream and events, made by the first call that has
 // pieces to overlap and kept with it (making them takes 0.5 ms, more than all
-// of a call on a few thousand rows); one call at a time.
+// of a call on a few thousand rows); one call at a time.  They belong to the
+// device that was current then: a call under another one makes its own.
 struct Device {
     std::mutex mu;
+    int index = -1;
     hipStream_t stream = nullptr;
     hipEvent_t done[2] = {nullptr, nullptr};
-    ~Device() {
-        for (hipEvent_t e : done)
+    ~Device() { release(); }
+    void release() {
+        for (hipEvent_t &e : done) {
             if (e) (void)hipEventDestroy(e);
+            e = nullptr;
+        }
         if (stream) (void)hipStreamDestroy(stream);
+        stream = nullptr;
+    }
+    int make() {  // for the current device
+        int current = 0;
+        CL_TRY(hipGetDevice(&current));
+        if (current != index) release();
+        index = current;
+        if (!stream) CL_TRY(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+        for (hipEvent_t &e : done)
+            if (!e) CL_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        return GLASS_HIP_OK;
     }
 };
 
@@ -294,11 +310,8 @@ int predict_device(Device &dev, const float *cent, int32_t k, int32_t d, const f
     const int64_t piece = std::max<int64_t>(64, ((int64_t)4 << 20) / d / 64 * 64);
     const int32_t rows = (int32_t)std::min<int64_t>(n, piece);
     const int32_t bufs = n > rows ? 2 : 1;
-    if (bufs > 1) {
-        if (!dev.stream) CL_TRY(hipStreamCreateWithFlags(&dev.stream, hipStreamNonBlocking));
-        for (hipEvent_t &e : dev.done)
-            if (!e) CL_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    }
+    if (bufs > 1)
+        if (const int r = dev.make()) return r;
     const hipStream_t stream = bufs > 1 ? dev.stream : nullptr;
     Arena a;
     const size_t o_x = a.add(4 * (size_t)rows * d * bufs), o_cent = a.add(4 * (size_t)k * d),
