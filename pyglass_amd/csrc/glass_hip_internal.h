@@ -80,8 +80,8 @@ struct LaunchConfig {
 };
 
 // Work counters of a launch: kWorkLines lines of kWorkLineWords words, each of
-// them [queries handed out, slots that have ended], and a word for the lines
-// whose slots have all ended.
+// them [queries handed out, slots that have ended], and a line of [lines whose
+// slots have all ended, a bit per line whose queries are all handed out].
 constexpr int32_t kWorkLines = 16, kWorkLineWords = 32, kWorkWords = (kWorkLines + 1) * kWorkLineWords;
 
 struct SlotState {
