@@ -78,6 +78,16 @@ __device__ __forceinline__ float float_of_key(uint32_t k) {
 // (__ballot goes through an int and compares again).
 __device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 
+// The lesser of each pair of 16-bit halves.
+__device__ __forceinline__ uint32_t pk_min_u16(uint32_t a, uint32_t b) {
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+
+// The lane's bit of a mask, as a condition (the mask becomes the exec mask of
+// what depends on it: no shift and compare per lane).
+__device__ __forceinline__ bool in_mask(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
 // Marks a wave-uniform value as such (moves it to a scalar register), so that
 // branches on it are scalar branches and arithmetic on it runs on the SALU.
 __device__ __forceinline__ int32_t uni(int32_t v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -1168,187 +1178,176 @@ struct VisitedSet {
     // odd, and its inverse modulo 2^32 (and so, masked, modulo any 2^b)
     static constexpr uint32_t kMul = 0x9E3779B1u, kMulInverse = 0x0E8B2F51u;
     uint32_t *tab;
-    uint32_t bmask, rb, smask;  // id bits, remainder bits, buckets - 1
-    bool wide;           // 32-bit entries
-    bool direct;         // the LDS words are a bitset of every row
-    int32_t count, thr;
-    bool global;
+    uint32_t bmask, rmask;      // an id's bits, its remainder's
+    uint32_t rb, smask;         // remainder bits, buckets - 1
+    int32_t es;          // bit of a word's second entry: 16, or 0 for entries of 32 bits
+    int32_t count;       // ids inserted
+    int32_t limit;       // the table is in use up to this many; -1: the LDS words are a bitset of every row
     uint32_t *gbits;
     int64_t gwords;
     uint32_t *dirty;     // the slot's dirty list: bitset words this query set first
     int32_t dirty_cap;   // its capacity in words
     int32_t ndirty;      // words recorded (past dirty_cap: the whole bitset is cleared)
-    bool pend = false;   // this lane's compare-and-swap of test_set is still to be looked at:
-    uint32_t p_at, p_e, p_old, p_got;  // its word, entry, and the word before and as found
+
+    // A lane's compare-and-swap of test_set, looked at by account(): its bucket
+    // and entry, and the word before and as found (equal for lanes without one).
+    struct Claim {
+        uint32_t s, e, old, got;
+    };
+
+    // A word with entry e shifted in: it held none or, of 16 bits, one.
+    static __device__ __forceinline__ uint32_t with(uint32_t old, uint32_t e) { return (old << 16) | e; }
 
     __device__ __forceinline__ void reset(uint32_t *t, int32_t words, int32_t n, uint32_t *g, int64_t gw, uint32_t *dl,
                                           int32_t dcap) {
         tab = t;
-        direct = n <= 32 * words;
+        const bool direct = n <= 32 * words;
         const uint32_t sb = (uint32_t)__builtin_ctz((uint32_t)words) - 1u;  // bucket bits
         const uint32_t nb = 32u - (uint32_t)__builtin_clz((uint32_t)(n - 1) | 1u);
         const uint32_t b = nb > sb ? nb : sb;
         rb = b - sb;
-        wide = rb > 14u;
+        es = rb > 14u ? 0 : 16;
         bmask = (1u << b) - 1u;  // rows are counted in 31 bits
+        rmask = (1u << rb) - 1u;
         smask = ((uint32_t)words >> 1) - 1u;
         count = 0;
-        thr = direct ? 0x7fffffff : (int32_t)((uint32_t)words * kVisLoad / (wide ? 8u : 4u));
-        global = false;
+        // a chunk of an adjacency row inserts at most 64 ids
+        limit = direct ? -1 : (int32_t)((uint32_t)words * kVisLoad / (es ? 4u : 8u)) - 64;
         gbits = g;
         gwords = gw;
         dirty = dl;
         dirty_cap = dcap;
         ndirty = 0;
-        pend = false;
-        p_at = p_e = p_old = p_got = 0u;
         const int32_t used = direct ? (n + 31) >> 5 : words;
         uint4 *t4 = (uint4 *)t;
         for (int i = lane_id(); i < (used + 3) >> 2; i += 64) t4[i] = make_uint4(0, 0, 0, 0);
         wave_sync();
     }
 
+    __device__ __forceinline__ bool in_table() const { return count <= limit; }
+
     // Records the bitset words of the lanes of `m` as set by this query.
     __device__ __forceinline__ void record(uint64_t m, uint32_t v) {
         const int pos = ndirty + mbcnt(m);
-        if (((m >> lane_id()) & 1) && pos < dirty_cap) dirty[pos] = v >> 5;
+        if (in_mask(m) && pos < dirty_cap) dirty[pos] = v >> 5;
         ndirty += __builtin_popcountll(m);
     }
 
-    // Looks v up in the table.  The home bucket, or the first one after it with
-    // room, decides: ids tested together are distinct, so a lane without a hit
-    // is new whether its compare-and-swap (issued here) succeeds or another
-    // lane of the wave took the entry; finish() looks at that later, off the
-    // path to the new ids.  Returns 0 visited, 1 new, 2 for the bitset.
-    template <bool kWide>
-    __device__ __forceinline__ int look(uint32_t v) {
-        constexpr uint32_t kMost = kWide ? 0xffffffffu : 0xffffu;
-        const uint32_t h = (v * kMul) & bmask;
-        uint32_t s = h >> rb;
-        uint32_t e = (h & ((1u << rb) - 1u)) + 1u;
-        uint2 *tb = (uint2 *)tab;
-        for (;;) {
-            const uint2 w = tb[s];
-            bool hit, full;
-            if (kWide) {
-                hit = w.x == e || w.y == e;
-                full = w.y != 0u;
-            } else {
-                // a zero half of x or y: an entry equal to e
-                const uint32_t ee = e | (e << 16), x = w.x ^ ee, y = w.y ^ ee;
-                hit = (((x - 0x00010001u) & ~x) | ((y - 0x00010001u) & ~y)) & 0x80008000u;
-                full = w.y > 0xffffu;
-            }
-            if (hit) return 0;
-            if (!full) {
-                // the bucket's first word with room: its entry, or its second one
-                const bool second = kWide ? w.x != 0u : w.x > 0xffffu;
-                const uint32_t o = second ? w.y : w.x;
-                p_at = 2u * s + (second ? 1u : 0u);
-                p_e = e;
-                p_old = o;
-                p_got = atomicCAS(&tab[p_at], o, kWide || o == 0u ? e : o | (e << 16));
-                return 1;
-            }
-            // the next bucket, its displacement one more
-            if (e > kMost - (1u << rb)) return 2;
-            e += 1u << rb;
-            s = (s + 1u) & smask;
-        }
-    }
-
-    // true when v had not been visited; marks it visited.
-    __device__ __forceinline__ bool test_set(uint32_t v, bool active) {
+    // The lanes of `m` whose v is new to the slot's bitset; sets them there.
+    __device__ __forceinline__ uint64_t to_bitset(uint32_t v, uint64_t m) {
+        asm volatile("" : "+v"(v));  // its address is not worth computing ahead
         const uint32_t bit = 1u << (v & 31u);
-        pend = false;
-        if (direct) {
-            bool isnew = false;
-            if (active) isnew = !(atomicOr(&tab[v >> 5], bit) & bit);
-            return isnew;
-        }
-        bool isnew = false, spill = active;
-        if (!global) {
-            int r = 0;
-            if (wide) {
-                if (active) r = look<true>(v);
-            } else {
-                if (active) r = look<false>(v);
-            }
-            isnew = pend = r == 1;
-            spill = r == 2;
-            if (ballot(spill) == 0) return isnew;
-        }
-        bool fresh = false;
-        if (spill) {
-            const uint32_t was =
-                __hip_atomic_fetch_or(&gbits[v >> 5], bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            isnew = !(was & bit);
-            fresh = was == 0u;  // lanes on one word are serialised: one sees 0
-        }
-        const uint64_t fm = ballot(fresh);
-        if (fm) record(fm, v);
-        return isnew;
+        uint32_t was = 0xffffffffu;
+        if (in_mask(m)) was = __hip_atomic_fetch_or(&gbits[v >> 5], bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const uint64_t fresh = ballot(was == 0u);  // lanes on one word are serialised: one sees 0
+        if (fresh) record(fresh, v);
+        return m & ballot((was & bit) == 0u);
     }
 
-    // The entries that test_set's compare-and-swap did not get: tried again
-    // from the word the other lane left.
-    __device__ __forceinline__ void finish(uint32_t v) {
-        bool again = pend && p_got != p_old;
-        while (ballot(again)) {
-            if (again) {
-                again = false;
-                const uint32_t room = wide ? 1u : 0x10000u;  // words from here on are full
-                uint32_t at = p_at, e = p_e, w = p_got;
-                for (;;) {
-                    if (w < room) {
-                        const uint32_t got = atomicCAS(&tab[at], w, w == 0u ? e : w | (e << 16));
-                        if (got == w) break;
-                        w = got;
-                        continue;
-                    }
-                    at = (at + 1u) & (2u * smask + 1u);
-                    if ((at & 1u) == 0u) {  // the next bucket
-                        if (e > (wide ? 0xffffffffu : 0xffffu) - (1u << rb)) {
-                            again = true;  // the bitset takes it, below
-                            break;
-                        }
-                        e += 1u << rb;
-                    }
-                    w = tab[at];
+    // The lanes of `active` whose v had not been visited; marks them visited.
+    // In the table the home bucket, or the first one after it with room,
+    // decides: ids tested together are distinct, so a lane without a hit is
+    // new whether its compare-and-swap (issued here) succeeds or another lane
+    // of the wave takes the entry; account() looks at that later, off the path
+    // to the new ids.  A device full of waves is bound by instruction issue, so
+    // the code is one line for lanes whose home bucket decides, the same for
+    // both entry sizes, and lanes are selected by masks.
+    __device__ __forceinline__ uint64_t test_set(uint32_t v, uint64_t active, Claim &c) {
+        if (in_table()) {
+            const uint32_t sh = (uint32_t)at_use(es), room = 1u << sh;
+            // the product modulo 2^b; up to 24 bits of it by the full-rate multiplication
+            const uint32_t h = bmask < 1u << 24 ? __umul24(v, kMul) : v * kMul;
+            uint32_t s = (h & bmask) >> rb, e = (h & rmask) + 1u;
+            const uint2 *const tb = (const uint2 *)tab;
+            uint2 w = tb[s];
+            auto hits = [&]() __attribute__((always_inline)) -> uint64_t {
+                if (sh == 0u) return ballot(w.x == e || w.y == e);
+                // an entry equal to e: a zero half of x or y
+                const uint32_t ee = e | (e << 16), x = w.x ^ ee, y = w.y ^ ee;
+                const uint32_t m = pk_min_u16(x, y);
+                return ballot(((m - 0x00010001u) & ~m & 0x80008000u) != 0u);
+            };
+            uint64_t fresh = active & ~hits();
+            uint64_t next = fresh & ballot(w.y >= room), spill = 0;  // full: the next bucket, its displacement one more
+            while (__builtin_expect(next != 0, 0)) {
+                spill |= next & ballot(e > (0xffffffffu >> sh) - (1u << rb));
+                if (in_mask(next)) {
+                    e += 1u << rb;
+                    s = (s + 1u) & smask;
+                    w = tb[s];
                 }
+                fresh = active & ~spill & ~hits();
+                next &= fresh & ballot(w.y >= room);
             }
-            if (ballot(again)) {
-                bool fresh = false;
-                if (again)
-                    fresh = __hip_atomic_fetch_or(&gbits[v >> 5], 1u << (v & 31u), __ATOMIC_RELAXED,
-                                                  __HIP_MEMORY_SCOPE_WORKGROUP) == 0u;
-                const uint64_t fm = ballot(fresh);
-                if (fm) record(fm, v);
-            }
-            again = false;
+            // the bucket's first word with room: its entry, or its second one
+            const bool second = w.x >= room;
+            c.s = s;
+            c.e = e;
+            c.old = second ? w.y : w.x;
+            c.got = c.old;
+            uint32_t *const word = (uint32_t *)(tb + s);
+            const uint32_t made = with(c.old, e);
+            if (in_mask(fresh)) c.got = atomicCAS(second ? word + 1 : word, c.old, made);
+            if (__builtin_expect(spill != 0, 0)) fresh |= to_bitset(v, spill);
+            return fresh;
         }
-        pend = false;
+        c = Claim{0u, 0u, 0u, 0u};
+        if (limit < 0) {
+            const uint32_t bit = 1u << (v & 31u);
+            uint32_t was = bit;
+            if (in_mask(active)) was = atomicOr(&tab[v >> 5], bit);
+            return ballot((was & bit) == 0u);
+        }
+        return to_bitset(v, active);
+    }
+
+    // The entries that test_set's compare-and-swap did not get, because other
+    // lanes took the room: tried again from the same bucket on.
+    __device__ __forceinline__ void retry(uint32_t v, const Claim &c) {
+        bool spill = false;
+        if (c.got != c.old) {
+            const uint32_t room = 1u << (uint32_t)es;
+            uint32_t s = c.s, e = c.e;
+            for (;;) {
+                const uint2 w = ((const uint2 *)tab)[s];
+                if (w.y < room) {
+                    const bool second = w.x >= room;
+                    const uint32_t old = second ? w.y : w.x;
+                    if (atomicCAS(&tab[2u * s + (second ? 1u : 0u)], old, with(old, e)) == old) break;
+                    continue;
+                }
+                if (e > (0xffffffffu >> (uint32_t)es) - (1u << rb)) {
+                    spill = true;  // the bitset takes it
+                    break;
+                }
+                e += 1u << rb;
+                s = (s + 1u) & smask;
+            }
+        }
+        const uint64_t m = ballot(spill);
+        if (m) (void)to_bitset(v, m);
     }
 
     // Moves the table's ids to the bitset.  Their words are recorded without
     // waiting for what they held, so a word may be recorded twice.
     __device__ __forceinline__ void migrate() {
+        const bool wide = es == 0;
         const unsigned long long *tb = (const unsigned long long *)tab;
-        for (uint32_t i = lane_id(); i <= smask; i += 64) {  // a multiple of 64 buckets
+        for (uint32_t i0 = 0; i0 <= smask; i0 += 64) {  // a multiple of 64 buckets
+            const uint32_t i = i0 + (uint32_t)lane_id();
             const unsigned long long w = tb[i];
             for (uint32_t at = 0; at < 64u; at += wide ? 32u : 16u) {
                 const uint32_t e = (uint32_t)(w >> at) & (wide ? 0xffffffffu : 0xffffu);
                 const uint64_t m = ballot(e != 0u);
                 if (m == 0) break;
                 const uint32_t home = (i - ((e - 1u) >> rb)) & smask;
-                const uint32_t v = (((home << rb) | ((e - 1u) & ((1u << rb) - 1u))) * kMulInverse) & bmask;
+                const uint32_t v = (((home << rb) | ((e - 1u) & rmask)) * kMulInverse) & bmask;
                 if (e != 0u)
                     (void)__hip_atomic_fetch_or(&gbits[v >> 5], 1u << (v & 31u), __ATOMIC_RELAXED,
                                                 __HIP_MEMORY_SCOPE_WORKGROUP);
                 record(m, v);
             }
         }
-        global = true;
     }
 
     // End of a query: the bitset words it set back to zero.
@@ -1368,12 +1367,12 @@ struct VisitedSet {
     }
 
     // Account for the ids v that test_set found new; switch to the global bitset (all
-    // zero, see above) before the table could pass its limit (a row inserts
-    // at most 64 ids).
-    __device__ __forceinline__ void account(int inserted, uint32_t v) {
-        finish(v);
+    // zero, see above) before the table could pass its limit.
+    __device__ __forceinline__ void account(int inserted, uint32_t v, const Claim &c) {
+        const bool table = in_table();
+        if (table && __builtin_expect(ballot(c.got != c.old) != 0, 0)) retry(v, c);
         count += inserted;
-        if (count > thr - 64 && !global) migrate();
+        if (table && __builtin_expect(!in_table(), 0)) migrate();
     }
 };
 
@@ -1975,8 +1974,9 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
                 w.pk[0] = du;
                 w.pid[0] = u;
             }
-            vs.test_set(u, l == 0);
-            vs.count = 1;  // the table was empty: nothing to try again, no limit near
+            VisitedSet::Claim c;  // the table was empty: nothing to try again, no limit near
+            vs.test_set(u, 1ull, c);
+            vs.count = 1;
             ps.size = 1;
             ps.cur = 0;
             wave_sync();
@@ -1999,8 +1999,9 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
                     pool_settle(w, ps);
                     pool_merge_lds(w, ps, nep);
                 }
-                vs.test_set(ep, l < nep);
-                vs.account(nep, ep);
+                VisitedSet::Claim c;
+                vs.test_set(ep, ballot(l < nep), c);
+                vs.account(nep, ep, c);
             }
         }
 
@@ -2033,12 +2034,12 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
                         const int32_t v = (u == pred) ? pred_row : (l < ix.K ? ix.adj[(int64_t)u * ix.K + l] : -1);
                         const uint64_t inv = ballot(l < ix.K && v == -1);
                         const int n = inv ? __builtin_ctzll(inv) : ix.K;
-                        const bool isnew = vs.test_set((uint32_t)v, l < n);
-                        const uint64_t nm = ballot(isnew);
+                        VisitedSet::Claim c;
+                        const uint64_t nm = vs.test_set((uint32_t)v, ballot(l < n), c);
                         if (nm) {
                             m = __builtin_popcountll(nm);
-                            vs.account(m, (uint32_t)v);
-                            if (isnew) w.ci[mbcnt(nm)] = (uint32_t)v;
+                            vs.account(m, (uint32_t)v, c);
+                            if (in_mask(nm)) w.ci[mbcnt(nm)] = (uint32_t)v;
                             break;
                         }
                         pred = kIdMask;
@@ -2087,14 +2088,15 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
             const int32_t vr = (u == pred) ? pred_row : ix.adj[(int64_t)u * ix.K + njc];
             const int32_t v = nj < ix.K ? vr : -1;
             if (is_int_variant(V) && (kFast || at_use(spec) != 0)) {
-                const bool lead = iq.part == 0;
                 const uint64_t inv = lead_k & ballot(v == -1);
                 const int n = inv ? __builtin_ctzll(inv) / iq.slot : ix.K;
                 const bool valid = nj < n;
                 uint4 c4[DPL / 4];
                 iq.load_row(ix, (uint32_t)v, valid, c4);
-                const bool isnew = vs.test_set((uint32_t)v, lead && valid);
-                const uint64_t nm = ballot(isnew);
+                VisitedSet::Claim c;
+                // the first lane of each group before the first without a neighbour
+                const uint64_t nm = vs.test_set((uint32_t)v, lead_k & ((inv & (0ull - inv)) - 1ull), c);
+                const bool isnew = in_mask(nm);
                 pred = kIdMask;
                 if (nm == 0) {
                     pool_settle(w, ps);
@@ -2104,7 +2106,7 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
                 }
                 const int m = __builtin_popcountll(nm);
                 const uint32_t kj = key_of_int(iq.row_dist(c4, valid));
-                vs.account(m, (uint32_t)v);
+                vs.account(m, (uint32_t)v, c);
                 cnt_d += m;
                 if (kFast || at_use(lc.cap_max) <= 128) {
                     pred = pool_merge_reg<kChunks>(ix, w, ps, kj, (uint32_t)v, isnew, nm, nj, pred_row);
@@ -2134,13 +2136,13 @@ __global__ __launch_bounds__(P == 2 ? 512 : 256) __attribute__((amdgpu_waves_per
                 const int rem = ix.K - c0;  // row entries from c0 on
                 const uint64_t inv = ballot(l < rem && vc == -1);
                 const int n = inv ? __builtin_ctzll(inv) : (rem < 64 ? rem : 64);
-                const bool isnew = vs.test_set((uint32_t)vc, l < n);
-                const uint64_t nm = ballot(isnew);
+                VisitedSet::Claim c;
+                const uint64_t nm = vs.test_set((uint32_t)vc, ballot(l < n), c);
                 if (nm) {
                     const int m = __builtin_popcountll(nm);
-                    if (isnew) w.ci[mbcnt(nm)] = (uint32_t)vc;
+                    if (in_mask(nm)) w.ci[mbcnt(nm)] = (uint32_t)vc;
                     wave_sync();
-                    vs.account(m, (uint32_t)vc);
+                    vs.account(m, (uint32_t)vc, c);
                     dists(m, qb.mode);
                     cnt_d += m;
                     if (kFast || at_use(lc.cap_max) <= 128) {
