@@ -17,54 +17,75 @@ namespace {
 // the tail of d mod 16 elements takes one 8-wide step (squares rounded,
 // u_i = s_(i+4) + s_i, (u1 + u3) + (u0 + u2)), one 4-wide step
 // ((s1 + s3) + (s0 + s2), added), then fused multiply-adds; body + tail.
-__device__ float l2_helpa(const float *x, const float *y, int32_t d) {
+// C rows y, y + d, ... at once: out[c] is x's distance to the c-th.
+template <int C, typename Y>
+__device__ __forceinline__ void l2_helpa(const float *x, Y y, int32_t d, float (&out)[C]) {
     const int32_t da = d / 16 * 16;
-    float A = 0.0f;
-    if (da > 0) {
-        float a[16];
+    float A[C], T[C];
 #pragma unroll
-        for (int l = 0; l < 16; ++l) a[l] = 0.0f;
+    for (int c = 0; c < C; ++c) A[c] = T[c] = 0.0f;
+    if (da > 0) {
+        float a[C][16];
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int l = 0; l < 16; ++l) a[c][l] = 0.0f;
         for (int32_t i = 0; i < da; i += 16) {
 #pragma unroll
-            for (int l = 0; l < 16; ++l) {
-                const float t = x[i + l] - y[i + l];
-                a[l] = fmaf(t, t, a[l]);
-            }
+            for (int c = 0; c < C; ++c)
+#pragma unroll
+                for (int l = 0; l < 16; ++l) {
+                    const float t = x[i + l] - y[(int64_t)c * d + i + l];
+                    a[c][l] = fmaf(t, t, a[c][l]);
+                }
         }
-        float b[8], c[4];
 #pragma unroll
-        for (int l = 0; l < 8; ++l) b[l] = a[l + 8] + a[l];
+        for (int c = 0; c < C; ++c) {
+            float b[8], q[4];
 #pragma unroll
-        for (int l = 0; l < 4; ++l) c[l] = b[l + 4] + b[l];
-        A = (c[0] + c[2]) + (c[1] + c[3]);
+            for (int l = 0; l < 8; ++l) b[l] = a[c][l + 8] + a[c][l];
+#pragma unroll
+            for (int l = 0; l < 4; ++l) q[l] = b[l + 4] + b[l];
+            A[c] = (q[0] + q[2]) + (q[1] + q[3]);
+        }
     }
-    float T = 0.0f;
     int32_t i = da;
     if (d - i >= 8) {
-        float u[4];
 #pragma unroll
-        for (int l = 0; l < 4; ++l) {
-            const float t0 = x[i + l] - y[i + l], t1 = x[i + 4 + l] - y[i + 4 + l];
-            u[l] = t1 * t1 + t0 * t0;
+        for (int c = 0; c < C; ++c) {
+            float u[4];
+#pragma unroll
+            for (int l = 0; l < 4; ++l) {
+                const float t0 = x[i + l] - y[(int64_t)c * d + i + l];
+                const float t1 = x[i + 4 + l] - y[(int64_t)c * d + i + 4 + l];
+                u[l] = t1 * t1 + t0 * t0;
+            }
+            T[c] = (u[1] + u[3]) + (u[0] + u[2]);
         }
-        T = (u[1] + u[3]) + (u[0] + u[2]);
         i += 8;
     }
     if (d - i >= 4) {
-        float q[4];
 #pragma unroll
-        for (int l = 0; l < 4; ++l) {
-            const float t = x[i + l] - y[i + l];
-            q[l] = t * t;
+        for (int c = 0; c < C; ++c) {
+            float q[4];
+#pragma unroll
+            for (int l = 0; l < 4; ++l) {
+                const float t = x[i + l] - y[(int64_t)c * d + i + l];
+                q[l] = t * t;
+            }
+            T[c] = T[c] + ((q[1] + q[3]) + (q[0] + q[2]));
         }
-        T = T + ((q[1] + q[3]) + (q[0] + q[2]));
         i += 4;
     }
     for (; i < d; ++i) {
-        const float t = x[i] - y[i];
-        T = fmaf(t, t, T);
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const float t = x[i] - y[(int64_t)c * d + i];
+            T[c] = fmaf(t, t, T[c]);
+        }
     }
-    return A + T;
+#pragma unroll
+    for (int c = 0; c < C; ++c) out[c] = A[c] + T[c];
 }
 
 // ---------------------------------------------------------------------------
@@ -251,47 +272,93 @@ __global__ __launch_bounds__(256) void cluster_decide_kernel(int32_t n, int32_t 
     }
 }
 
-// Each listed row's (every row's where list is null) first nearest centroid in
-// the reference's order: one workgroup per row, one thread per centroid.
-__global__ __launch_bounds__(256) void cluster_exact_kernel(const float *x, int32_t n, int32_t d, const float *cent,
-                                                            int32_t k, const int32_t *list, const int32_t *count,
-                                                            int32_t *ids) {
-    __shared__ float sv[4];
-    __shared__ int32_t si[4];
-    const int32_t rows = list ? *count : n;
-    for (int32_t i = blockIdx.x; i < rows; i += gridDim.x) {
-        const int32_t row = list ? list[i] : i;
-        const float *xi = x + (int64_t)row * d;
-        float best = __builtin_inff();
-        int32_t bid = 0x7fffffff;  // none: no distance compares less than infinity
-        for (int32_t j = threadIdx.x; j < k; j += 256) {
-            const float v = l2_helpa(xi, cent + (int64_t)j * d, d);
-            if (v < best) {
-                best = v;
-                bid = j;
-            }
-        }
-        for (int o = 32; o > 0; o >>= 1) {
-            const float v = __shfl_xor(best, o);
-            const int32_t j = __shfl_xor(bid, o);
-            if (v < best || (v == best && j < bid)) {
-                best = v;
-                bid = j;
-            }
-        }
-        __syncthreads();
-        if ((threadIdx.x & 63) == 0) {
-            sv[threadIdx.x >> 6] = best;
-            si[threadIdx.x >> 6] = bid;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            for (int w = 1; w < 4; ++w)
-                if (sv[w] < best || (sv[w] == best && si[w] < bid)) {
-                    best = sv[w];
-                    bid = si[w];
+constexpr int32_t kNone = 0x7fffffff;
+
+// The first of the least distances so far; kNone while none compared less
+// than infinity.
+struct Near {
+    float v = __builtin_inff();
+    int32_t j = kNone;
+    __device__ __forceinline__ void next(float v2, int32_t j2) {  // j2 above all before
+        j = v2 < v ? j2 : j;
+        v = v2 < v ? v2 : v;
+    }
+    __device__ __forceinline__ void join(float v2, int32_t j2) {  // another's, over other centroids
+        const bool t = v2 < v || (v2 == v && j2 < j);
+        v = t ? v2 : v;
+        j = t ? j2 : j;
+    }
+};
+
+// Each listed row's first nearest centroid in the reference's order, in one of
+// two forms.  Few rows take a workgroup each, a thread per centroid: a row is
+// short work then, and there are no others to share the centroids with.  Many
+// are taken 64 to a workgroup, a row per lane, and its waves take four
+// centroids at a time in turn: those are the same for all lanes, so they come
+// through scalar loads, and a row's elements are read once for four of them.
+// The first form is bound by its lanes' reads of one centroid each (0.5 ps per
+// dimension), the second by the chain of a wave's 16-dimension steps (1 us
+// each) until the rows fill the device.  20,000 rows x 128 that the filter
+// cannot decide, 1,024 centroids: 1,380 us by rows, 470 by tiles; 1,000 of
+// them: 70 and 400.
+__global__ __launch_bounds__(256) void cluster_exact_kernel(const float *x, int32_t d, const float *cent, int32_t k,
+                                                            const int32_t *list, const int32_t *count, int32_t *ids) {
+    __shared__ float near_v[4][64];
+    __shared__ int32_t near_j[4][64];
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
+    const int32_t rows = *count;
+    if (exact_by_row_ps(rows, d, k) > exact_by_tile_ps(rows, d, k)) {
+        typedef const __attribute__((address_space(4))) float *Scalar;
+        const Scalar sc = (Scalar)cent;
+        for (int32_t at = blockIdx.x * 64; at < rows; at += gridDim.x * 64) {
+            const int32_t r = at + l < rows ? at + l : rows - 1;
+            const int32_t row = list[r];
+            const float *xi = x + (int64_t)row * d;
+            Near b;
+            for (int32_t j = 4 * wv; j < k; j += 16) {
+                if (j + 4 <= k) {
+                    float v[4];
+                    l2_helpa<4>(xi, sc + (int64_t)j * d, d, v);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) b.next(v[c], j + c);
+                } else {
+                    for (int32_t c = j; c < k; ++c) {
+                        float v[1];
+                        l2_helpa<1>(xi, sc + (int64_t)c * d, d, v);
+                        b.next(v[0], c);
+                    }
                 }
-            ids[row] = bid == 0x7fffffff ? -1 : bid;
+            }
+            __syncthreads();
+            near_v[wv][l] = b.v;
+            near_j[wv][l] = b.j;
+            __syncthreads();
+            if (wv == 0 && at + l < rows) {
+                for (int w = 1; w < 4; ++w) b.join(near_v[w][l], near_j[w][l]);
+                ids[row] = b.j == kNone ? -1 : b.j;
+            }
+        }
+        return;
+    }
+    for (int32_t i = blockIdx.x; i < rows; i += gridDim.x) {
+        const int32_t row = list[i];
+        const float *xi = x + (int64_t)row * d;
+        Near b;
+        for (int32_t j = tid; j < k; j += 256) {
+            float v[1];
+            l2_helpa<1>(xi, cent + (int64_t)j * d, d, v);
+            b.next(v[0], j);
+        }
+        for (int o = 32; o > 0; o >>= 1) b.join(__shfl_xor(b.v, o), __shfl_xor(b.j, o));
+        __syncthreads();
+        if (l == 0) {
+            near_v[wv][0] = b.v;
+            near_j[wv][0] = b.j;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            for (int w = 1; w < 4; ++w) b.join(near_v[w][0], near_j[w][0]);
+            ids[row] = b.j == kNone ? -1 : b.j;
         }
     }
 }
@@ -301,7 +368,9 @@ __global__ __launch_bounds__(256) void cluster_exact_kernel(const float *x, int3
 __global__ void cluster_dist_kernel(const float *x, int32_t n, int32_t d, const float *pivot, float *out) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    out[i] = l2_helpa(pivot, x + i * d, d);
+    float v[1];
+    l2_helpa<1>(pivot, x + i * d, d, v);
+    out[i] = v[0];
 }
 
 // update_mediods (clustering.hpp:234-256): a centroid is the float sum of its
@@ -392,6 +461,9 @@ int32_t filter_splits(int32_t n, int32_t k) {
     return want < cent_tiles(k) ? want : cent_tiles(k);
 }
 
+// The exact kernel's workgroups for up to n rows in either form.
+int32_t exact_blocks(int32_t n) { return std::max(std::min(n, 1024), std::min((n + 63) / 64, 4096)); }
+
 }  // namespace
 
 // Fewer rows are split further, so the layout for fewer rows can be the larger
@@ -435,7 +507,7 @@ hipError_t launch_cluster_assign(const float *x, int32_t n, int32_t d, const flo
                        cent, k, s.c2, tiles, s.m1, s.m2, s.i1);
     hipLaunchKernelGGL(cluster_decide_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, n, d, splits, s.x2, s.c2max,
                        s.m1, s.m2, s.i1, ids, s.list, s.count);
-    hipLaunchKernelGGL(cluster_exact_kernel, dim3(n < 1024 ? n : 1024), dim3(256), 0, stream, x, n, d, cent, k, s.list,
+    hipLaunchKernelGGL(cluster_exact_kernel, dim3(exact_blocks(n)), dim3(256), 0, stream, x, d, cent, k, s.list,
                        s.count, ids);
     return hipGetLastError();
 }

@@ -153,6 +153,14 @@ void fit_host(const float *rows, int32_t n, int32_t d, int32_t k, int32_t epochs
 
 }  // namespace km
 
+// What the exact nearest-centroid kernel takes for n rows of d against k
+// centroids, in picoseconds as measured, in its two forms (cluster_kernels.hip):
+// a workgroup per row, and 64 rows to a workgroup.
+constexpr int64_t exact_by_row_ps(int64_t n, int64_t d, int64_t k) { return n * (1800 + d * k / 2); }
+constexpr int64_t exact_by_tile_ps(int64_t n, int64_t d, int64_t k) {
+    return (d + 15) / 16 * ((k + 15) / 16) * 1000000 + n * (d * k * 3 / 20);
+}
+
 // Device scratch of launch_cluster_assign for n rows and k centroids.
 struct AssignScratch {
     float *x2, *c2, *m1, *m2;  // squared norms of rows and centroids, least and second least values
