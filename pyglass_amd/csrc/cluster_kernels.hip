@@ -290,29 +290,30 @@ struct Near {
     }
 };
 
-// Each listed row's first nearest centroid in the reference's order, in one of
-// two forms.  Few rows take a workgroup each, a thread per centroid: a row is
-// short work then, and there are no others to share the centroids with.  Many
-// are taken 64 to a workgroup, a row per lane, and its waves take four
-// centroids at a time in turn: those are the same for all lanes, so they come
-// through scalar loads, and a row's elements are read once for four of them.
-// The first form is bound by its lanes' reads of one centroid each (0.5 ps per
-// dimension), the second by the chain of a wave's 16-dimension steps (1 us
-// each) until the rows fill the device.  20,000 rows x 128 that the filter
-// cannot decide, 1,024 centroids: 1,380 us by rows, 470 by tiles; 1,000 of
-// them: 70 and 400.
-__global__ __launch_bounds__(256) void cluster_exact_kernel(const float *x, int32_t d, const float *cent, int32_t k,
-                                                            const int32_t *list, const int32_t *count, int32_t *ids) {
+// Each listed row's (every row's where list is null) first nearest centroid in
+// the reference's order, in one of two forms.  Few rows take a workgroup each,
+// a thread per centroid: a row is short work then, and there are no others to
+// share the centroids with.  Many are taken 64 to a workgroup, a row per lane,
+// and its waves take four centroids at a time in turn: those are the same for
+// all lanes, so they come through scalar loads, and a row's elements are read
+// once for four of them.  The first form is bound by its lanes' reads of one
+// centroid each (0.5 ps per dimension), the second by the chain of a wave's
+// 16-dimension steps (1 us each) until the rows fill the device.  20,000 rows x
+// 128 that the filter cannot decide, 1,024 centroids: 1,380 us by rows, 470 by
+// tiles; 1,000 of them: 70 and 400.
+__global__ __launch_bounds__(256) void cluster_exact_kernel(const float *x, int32_t n, int32_t d, const float *cent,
+                                                            int32_t k, const int32_t *list, const int32_t *count,
+                                                            int32_t *ids) {
     __shared__ float near_v[4][64];
     __shared__ int32_t near_j[4][64];
     const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
-    const int32_t rows = *count;
+    const int32_t rows = list ? *count : n;
     if (exact_by_row_ps(rows, d, k) > exact_by_tile_ps(rows, d, k)) {
         typedef const __attribute__((address_space(4))) float *Scalar;
         const Scalar sc = (Scalar)cent;
         for (int32_t at = blockIdx.x * 64; at < rows; at += gridDim.x * 64) {
             const int32_t r = at + l < rows ? at + l : rows - 1;
-            const int32_t row = list[r];
+            const int32_t row = list ? list[r] : r;
             const float *xi = x + (int64_t)row * d;
             Near b;
             for (int32_t j = 4 * wv; j < k; j += 16) {
@@ -341,7 +342,7 @@ __global__ __launch_bounds__(256) void cluster_exact_kernel(const float *x, int3
         return;
     }
     for (int32_t i = blockIdx.x; i < rows; i += gridDim.x) {
-        const int32_t row = list[i];
+        const int32_t row = list ? list[i] : i;
         const float *xi = x + (int64_t)row * d;
         Near b;
         for (int32_t j = tid; j < k; j += 256) {
@@ -490,6 +491,7 @@ void AssignScratch::place(void *p, int32_t n, int32_t k) {
 hipError_t launch_fill_i32(int32_t *p, int64_t n, int32_t v, hipStream_t stream);
 
 hipError_t launch_cluster_norms(const float *x, int32_t n, int32_t d, const AssignScratch &s, hipStream_t stream) {
+    if (!filter_pays(n, d, (int32_t)(s.m1 - s.c2))) return hipSuccess;  // nothing reads them; c2 has k words
     hipLaunchKernelGGL(cluster_norms_kernel, dim3((n + 3) / 4 < 8192 ? (n + 3) / 4 : 8192), dim3(256), 0, stream, x, n,
                        d, s.x2, (uint32_t *)nullptr);
     return hipGetLastError();
@@ -497,6 +499,11 @@ hipError_t launch_cluster_norms(const float *x, int32_t n, int32_t d, const Assi
 
 hipError_t launch_cluster_assign(const float *x, int32_t n, int32_t d, const float *cent, int32_t k, int32_t *ids,
                                  const AssignScratch &s, hipStream_t stream) {
+    if (!filter_pays(n, d, k)) {
+        hipLaunchKernelGGL(cluster_exact_kernel, dim3(exact_blocks(n)), dim3(256), 0, stream, x, n, d, cent, k,
+                           (const int32_t *)nullptr, (const int32_t *)nullptr, ids);
+        return hipGetLastError();
+    }
     const int32_t splits = filter_splits(n, k);
     const int32_t tiles = (cent_tiles(k) + splits - 1) / splits;
     // count and c2max are neighbours
@@ -507,7 +514,7 @@ hipError_t launch_cluster_assign(const float *x, int32_t n, int32_t d, const flo
                        cent, k, s.c2, tiles, s.m1, s.m2, s.i1);
     hipLaunchKernelGGL(cluster_decide_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, n, d, splits, s.x2, s.c2max,
                        s.m1, s.m2, s.i1, ids, s.list, s.count);
-    hipLaunchKernelGGL(cluster_exact_kernel, dim3(exact_blocks(n)), dim3(256), 0, stream, x, d, cent, k, s.list,
+    hipLaunchKernelGGL(cluster_exact_kernel, dim3(exact_blocks(n)), dim3(256), 0, stream, x, n, d, cent, k, s.list,
                        s.count, ids);
     return hipGetLastError();
 }

@@ -160,8 +160,16 @@ constexpr int64_t exact_by_row_ps(int64_t n, int64_t d, int64_t k) { return n * 
 constexpr int64_t exact_by_tile_ps(int64_t n, int64_t d, int64_t k) {
     return (d + 15) / 16 * ((k + 15) / 16) * 1000000 + n * (d * k * 3 / 20);
 }
+// Whether launch_cluster_assign filters rows first: the filter's launches cost
+// about 35 us whatever the size (predict() of 300 x 32, 16 clusters: 105 us with
+// it, 56 without; 4,000 x 64, 256 clusters: 123 and 132; 1,000 x 64, 1,024
+// clusters: 107 and 108).  More rows are never less worth it.
+constexpr bool filter_pays(int64_t n, int64_t d, int64_t k) {
+    return exact_by_row_ps(n, d, k) > 35000000 && exact_by_tile_ps(n, d, k) > 35000000;
+}
 
-// Device scratch of launch_cluster_assign for n rows and k centroids.
+// Device scratch of launch_cluster_assign for n rows and k centroids, where
+// filter_pays.
 struct AssignScratch {
     float *x2, *c2, *m1, *m2;  // squared norms of rows and centroids, least and second least values
     int32_t *i1, *list, *count;
@@ -170,7 +178,7 @@ struct AssignScratch {
     void place(void *p, int32_t n, int32_t k);
 };
 
-// Squared norms of the rows into s.x2, once for any number of sweeps.
+// Squared norms of the rows into s.x2 (where filter_pays), once for any number of sweeps.
 hipError_t launch_cluster_norms(const float *x, int32_t n, int32_t d, const AssignScratch &s, hipStream_t stream);
 // ids[i] = first nearest of the k centroids to row i (-1: none compares less than +inf).
 hipError_t launch_cluster_assign(const float *x, int32_t n, int32_t d, const float *cent, int32_t k, int32_t *ids,
