@@ -808,21 +808,22 @@ int32_t grid_blocks(const glass_hip_searcher &s, const LaunchConfig &lc, int32_t
 int32_t slots_per_block(const LaunchConfig &lc) { return lc.qwaves > 1 ? 1 : lc.waves_per_block; }
 
 // Dirty-list words per slot: the bitset words a query may record as set; a
-// query that sets more clears its whole bitset at its end.  Above 2M rows that
-// is 256 KB and more, and the list is longer: a query's first thousands of
-// ids come from its table, recorded one word each.  Above 64M rows it is short
-// again: the fixed scratch array of the no-alloc entry point is nearly used up
-// by four bitsets there.  A list longer than a quarter of a small bitset saves
-// little of its clearing and is most of the slot.
-int32_t dirty_words(const glass_hip_searcher &s) {
-    const int32_t words = s.graph.N > (2 << 20) && s.graph.N <= (64 << 20) ? 16384 : 4096;
+// query that sets more clears its whole bitset at its end.  From 2M to 64M rows
+// that is 256 KB and more, and the list is longer: a query's first thousands
+// of ids come from its table, recorded one word each.  In scratch of a fixed
+// size a longer list takes the place of waves in flight and is not worth them
+// (2.3M x 32 SQ4U, ef 128, 4,000 queries in the no-alloc array: 441 slots NOALLOC4K us,
+// 382 with 16,384 words each 3,506).  A list longer than a quarter of a small
+// bitset saves little of its clearing and is most of the slot.
+int32_t dirty_words(const glass_hip_searcher &s, bool fixed_scratch) {
+    const int32_t words = !fixed_scratch && s.graph.N > (2 << 20) && s.graph.N <= (64 << 20) ? 16384 : 4096;
     return std::min(words, std::max(64, (s.graph.N / 32 / 4 + 3) / 4 * 4));
 }
 
 // Words of slot scratch per resident wave: the PQ8 lookup table, the dirty
 // list, then an N-bit visited bitset (each a multiple of 4 words).
-int64_t slot_stride(const glass_hip_searcher &s) {
-    return s.lut_words + dirty_words(s) + ((int64_t)(s.graph.N + 31) / 32 + 3) / 4 * 4;
+int64_t slot_stride(const glass_hip_searcher &s, bool fixed_scratch = false) {
+    return s.lut_words + dirty_words(s, fixed_scratch) + ((int64_t)(s.graph.N + 31) / 32 + 3) / 4 * 4;
 }
 
 // Slot areas start zeroed (the visited bitsets must be all zero between
@@ -949,10 +950,12 @@ int check_cap(const glass_hip_searcher &s, int32_t max_cap) {
 }
 
 // Per-launch state for batches that run concurrently on several streams:
-// their own work counter and visited bitsets (max_slots x vis_stride words),
-// and optionally (id, dist) pair outputs.
+// their own work counter and slot areas (max_slots of them, in the no-alloc
+// entry point's array or as vis_stride says), and optionally (id, dist) pair
+// outputs.
 struct BatchState {
     uint32_t *visited = nullptr;
+    bool fixed_scratch = false;
     int32_t max_slots = 0;
     int32_t *counter = nullptr;
     uint64_t *out_pairs = nullptr;
@@ -1014,7 +1017,10 @@ int run_batch(glass_hip_searcher &s, const float *qs_dev, int32_t nq, const int3
             }
         }
     }
-    if (!lc.vis_hash) lc.vis_hash = untuned_vis(s, lc, nq, max_ef, alone);
+    // scratch of a fixed size may hold fewer slots than there are queries: LDS
+    // is for the waves that have one
+    if (!lc.vis_hash)
+        lc.vis_hash = untuned_vis(s, lc, bs && bs->fixed_scratch ? std::min(nq, bs->max_slots) : nq, max_ef, alone);
     // Large pools: fewer waves per workgroup, then a smaller visited table
     // (exact at any size: it moves to the global bitset when it fills), until
     // a workgroup's LDS fits the CU.
@@ -1052,9 +1058,10 @@ int run_batch(glass_hip_searcher &s, const float *qs_dev, int32_t nq, const int3
     qb.out_pairs = bs ? bs->out_pairs : nullptr;
     SlotState ss{};
     ss.visited = bs ? bs->visited : st->visited.p;
-    ss.vis_stride = s.vis_stride;
+    const bool fixed = bs && bs->fixed_scratch;
+    ss.vis_stride = fixed ? slot_stride(s, true) : s.vis_stride;
     ss.lut_words = s.lut_words;
-    ss.dirty_words = dirty_words(s);
+    ss.dirty_words = dirty_words(s, fixed);
     ss.nslots = bs ? bs->max_slots : st->nslots;
     ss.work_counter = counter;
     const DeviceIndex ix = s.index();
@@ -1557,7 +1564,8 @@ int glass_hip_searcher_search_batch_dev_noalloc(glass_hip_searcher *s, const flo
         void *base = nullptr;
         size_t bytes = 0;
         if (int r = noalloc_scratch(s->device, &base, &bytes)) return r;
-        const int64_t slot_bytes = 4 * slot_stride(*s);
+        const int64_t stride = slot_stride(*s, true), slot_bytes = 4 * stride;
+        const int32_t dirty = dirty_words(*s, true);
         const int64_t slots = ((int64_t)bytes - 4 * kWorkWords) / slot_bytes;
         if (slots < 4)
             return fail(GLASS_HIP_EINVAL,
@@ -1574,18 +1582,19 @@ int glass_hip_searcher_search_batch_dev_noalloc(glass_hip_searcher *s, const flo
             const int d = s->device;
             std::lock_guard<std::mutex> g(lay_mu);
             if (d < 0 || d >= 64) return fail(GLASS_HIP_EINVAL, "device index out of range");
-            if (lay_stride[d] != slot_stride(*s) || lay_lut[d] != s->lut_words || lay_dirty[d] != dirty_words(*s)) {
+            if (lay_stride[d] != stride || lay_lut[d] != s->lut_words || lay_dirty[d] != dirty) {
                 hipStream_t st = stream ? (hipStream_t)stream : s->stream;
                 HIP_TRY(launch_fill_i32((int32_t *)base, (int64_t)(bytes / 4), 0, st));
-                lay_stride[d] = slot_stride(*s);
+                lay_stride[d] = stride;
                 lay_lut[d] = s->lut_words;
-                lay_dirty[d] = dirty_words(*s);
+                lay_dirty[d] = dirty;
             }
         }
         // calls that overlapped on the array may have left its counter anywhere
         HIP_TRY(launch_fill_i32((int32_t *)base, kWorkWords, 0, stream ? (hipStream_t)stream : s->stream));
         BatchState bs;
         bs.counter = (int32_t *)base;
+        bs.fixed_scratch = true;
         bs.visited = (uint32_t *)base + kWorkWords;
         bs.max_slots = (int32_t)std::min<int64_t>(slots, 1 << 20);
         return run_batch(*s, qs_dev, nq, nullptr, nullptr, s->ef, k, max_cap, s->ef, mode, nullptr, dst_dev,
