@@ -812,9 +812,9 @@ int32_t slots_per_block(const LaunchConfig &lc) { return lc.qwaves > 1 ? 1 : lc.
 // that is 256 KB and more, and the list is longer: a query's first thousands
 // of ids come from its table, recorded one word each.  In scratch of a fixed
 // size a longer list takes the place of waves in flight and is not worth them
-// (2.3M x 32 SQ4U, ef 128, 4,000 queries in the no-alloc array: 441 slots NOALLOC4K us,
-// 382 with 16,384 words each 3,506).  A list longer than a quarter of a small
-// bitset saves little of its clearing and is most of the slot.
+// (2.3M x 32 SQ4U, ef 128, 4,000 queries in the no-alloc array: 441 slots
+// 3,127 us, 382 with 16,384 words each 3,507).  A list longer than a quarter of
+// a small bitset saves little of its clearing and is most of the slot.
 int32_t dirty_words(const glass_hip_searcher &s, bool fixed_scratch) {
     const int32_t words = !fixed_scratch && s.graph.N > (2 << 20) && s.graph.N <= (64 << 20) ? 16384 : 4096;
     return std::min(words, std::max(64, (s.graph.N / 32 / 4 + 3) / 4 * 4));
@@ -888,11 +888,16 @@ constexpr size_t kLdsPerCu = 160 * 1024;
 // 237; 300-d FP16, 29 KB, 362 / 332 / 296 / 288; 960-d SQ4U, 16 KB, 271 / 238 /
 // 218 / 210 (its rows do not fit the all-neighbour gather); 128-d FP32, 16 KB,
 // 286 / 318 / 313 / 305; 128-d SQ8U, 4 KB, 171 / 259 / 260 / 248.  SQ6's and
-// PQ8's rows cost more than their bytes: 200-d SQ6 780 / 684 / 686 / 662, 96-d
-// PQ8 325 / 273 / 274 / 257.
+// PQ8's rows cost more than their bytes: two waves gain where a node has more
+// neighbours than the 16 that one wave does at a time (us at 1 and 2 waves, 64
+// queries, ef 128: 96-d PQ8 of degree 16, 32 and 64 494 and 538, 504 and 451,
+// 698 and 562; 768-d SQ6 1,707 and 1,982, 1,872 and 1,690, 2,644 and 1,976),
+// but for degrees to 32 of short SQ6 rows (96-d, 2.3 KB, degree 32: 374 and
+// 390; 200-d, 4.8 KB, 751 and 677).
 int32_t untuned_qwaves(const glass_hip_searcher &s, int32_t team) {
-    if (s.quant == QK_SQ6 || s.quant == QK_PQ8) return 2;
     const int64_t bytes = (int64_t)s.graph.K * s.code_size;
+    if (s.quant == QK_SQ6) return s.graph.K > 32 || (s.graph.K > 16 && bytes >= 4 << 10) ? 2 : 1;
+    if (s.quant == QK_PQ8) return s.graph.K > 16 ? 2 : 1;
     if (bytes >= 24 << 10) return 8;
     const bool int_codes = s.quant == QK_SQ8U || s.quant == QK_SQ4U || s.quant == QK_SQ2U;
     return int_codes && bytes >= 12 << 10 && !spec_fits(s, team) ? 4 : 1;
