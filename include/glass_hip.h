@@ -159,8 +159,9 @@ int glass_hip_searcher_set_gather(glass_hip_searcher *s, int32_t mode);
  * distances), which cuts a query's latency where code rows are long or the
  * batch is too small to fill the device (graphs of at most 64 neighbours per
  * row).  0 (default) = the choice optimize() tunes per ef bucket on a batch
- * of a quarter of the resident waves, or without it up to 8 by the bytes of a
- * node's neighbour rows, used when a batch would leave most wave slots idle. */
+ * of a quarter of the resident waves, or without it (and where it chose 4) up
+ * to 8 by the bytes of a node's neighbour rows, used when a batch would leave
+ * most wave slots idle. */
 int glass_hip_searcher_set_query_waves(glass_hip_searcher *s, int32_t waves);
 /* Waves per query of the last launch, and optimize()'s choice for small
  * batches at the current ef. */

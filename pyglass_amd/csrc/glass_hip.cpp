@@ -994,8 +994,13 @@ int run_batch(glass_hip_searcher &s, const float *qs_dev, int32_t nq, const int3
         // round (1M x 960, ef 16-512 and k 1-100 per query, 1,000 queries:
         // 4 waves per query in 1.3 rounds, 4.30 ms, against 2 waves in one
         // round, 5.04 ms; with ef 256 for every query the 1.3 rounds lose).
-        const int32_t want =
-            s.force_qwaves ? s.force_qwaves : (tn.qwaves_small ? tn.qwaves_small : untuned_qwaves(s, lc.team));
+        // The tuner times up to 4 waves, on a batch that 8 do not fit: where 4
+        // were the best it tried, the row bytes' 8 stay for the batches that
+        // they do fit (13 and 26 KB rows of eight quantizers, 1 and 32 queries:
+        // equal to 13% faster).
+        const int32_t by_rows = untuned_qwaves(s, lc.team);
+        const int32_t tuned = tn.qwaves_small == 4 ? std::max(4, by_rows) : tn.qwaves_small;
+        const int32_t want = s.force_qwaves ? s.force_qwaves : (tuned ? tuned : by_rows);
         const int64_t rounds = ef_dev ? 2 : 1;
         if (want > 1 && s.graph.K <= 64) {
             int32_t qw = want;

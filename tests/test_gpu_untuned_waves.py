@@ -30,3 +30,28 @@ def test_untuned_waves_per_query(quant, dim, degree, waves):
     Io, Do = o.batch_search(Q, 10)
     np.testing.assert_array_equal(I, Io)
     np.testing.assert_array_equal(D, Do)
+
+
+def test_tuning_keeps_eight_waves_of_wide_rows():
+    """optimize() tries at most 4 waves per query; where it takes 4, wide rows
+    still get 8 in batches that leave room for them."""
+    if pg.device_count() < 1:
+        pytest.skip("no HIP device")
+    rng = np.random.default_rng(8)
+    X = rng.standard_normal((3000, 832)).astype(np.float32)
+    adj = rng.integers(0, 3000, (3000, 32)).astype(np.int32)
+    Q = rng.standard_normal((4, 832)).astype(np.float32)
+    s = pg.Searcher(pg.Graph.from_arrays(adj, [3]), X, "L2", "SQ8")
+    o = O.Searcher(O.Graph(adj=adj, eps=[3]), X, "L2", "SQ8")
+    s.set_ef(30)
+    o.set_ef(30)
+    print("waves per query: untuned, tuned", flush=True)
+    s.batch_search(Q, 10)
+    assert s.get_query_waves()[0] == 8
+    s.optimize()
+    I, D = s.batch_search(Q, 10)
+    last, tuned = s.get_query_waves()
+    assert last == (8 if tuned == 4 else tuned)
+    Io, Do = o.batch_search(Q, 10)
+    np.testing.assert_array_equal(I, Io)
+    np.testing.assert_array_equal(D, Do)
