@@ -324,6 +324,7 @@ struct StreamState {
     hipStream_t stream = nullptr;
     DevBuf<uint32_t> visited;
     int32_t nslots = 0;
+    int32_t most_slots = INT32_MAX;  // what device memory had room for when it did not suffice
     DevBuf<int32_t> counter;
     hipEvent_t done = nullptr;  // recorded after each launch that uses this state
     uint64_t last_use = 0;
@@ -828,11 +829,26 @@ int64_t slot_stride(const glass_hip_searcher &s, bool fixed_scratch = false) {
 
 // Slot areas start zeroed (the visited bitsets must be all zero between
 // queries); a fill kernel on the launch's stream, not hipMemsetAsync, so the
-// launch that follows is ordered after it.
-int ensure_slots(glass_hip_searcher &s, StreamState &st, int32_t slots, hipStream_t stream) {
+// launch that follows is ordered after it.  Where memory does not suffice for
+// the slots of every wave that could be resident (1 MB each at 8M rows, 4 GB in
+// all), as many as three quarters of what is free holds take the queries in
+// turn: `slots` is lowered to them.
+int ensure_slots(glass_hip_searcher &s, StreamState &st, int32_t &slots, hipStream_t stream) {
+    slots = std::min(slots, st.most_slots);
     if (slots <= st.nslots && st.visited.p) return GLASS_HIP_OK;
     s.vis_stride = slot_stride(s);
-    HIP_TRY(st.visited.alloc((size_t)slots * (size_t)s.vis_stride));
+    st.nslots = 0;
+    hipError_t e = st.visited.alloc((size_t)slots * (size_t)s.vis_stride);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        size_t free_b = 0, total_b = 0;
+        HIP_TRY(hipMemGetInfo(&free_b, &total_b));
+        const size_t fit = free_b / 4 * 3 / (4 * (size_t)s.vis_stride);
+        slots = st.most_slots = (int32_t)std::min<size_t>((size_t)slots, std::max<size_t>(fit, 4));
+        e = st.visited.alloc((size_t)slots * (size_t)s.vis_stride);
+        if (e != hipSuccess) st.most_slots = INT32_MAX;  // nothing is kept: the next call asks again
+    }
+    HIP_TRY(e);
     HIP_TRY(launch_fill_i32((int32_t *)st.visited.p, (int64_t)slots * s.vis_stride, 0, stream));
     st.nslots = slots;
     return GLASS_HIP_OK;
@@ -1045,7 +1061,9 @@ int run_batch(glass_hip_searcher &s, const float *qs_dev, int32_t nq, const int3
     StreamState *st = nullptr;
     if (!bs) {
         if (int r = state_for(s, stream, &st)) return r;
-        if (int r = ensure_slots(s, *st, blocks * slots_per_block(lc), stream)) return r;
+        int32_t slots = blocks * slots_per_block(lc);
+        if (int r = ensure_slots(s, *st, slots, stream)) return r;
+        lc.blocks = slots / slots_per_block(lc);
         if (!st->counter.p) {
             HIP_TRY(st->counter.alloc(kWorkWords));
             HIP_TRY(launch_fill_i32(st->counter.p, kWorkWords, 0, stream));
@@ -1392,7 +1410,10 @@ int glass_hip_searcher_set_data(glass_hip_searcher *s, const float *data, int32_
         s->dim = dim;
         quant_layout(s->quant, dim, &s->dim_align, &s->code_size);
         s->lut_words = s->quant == QK_PQ8 ? (int64_t)s->code_size * 256 : 0;
-        for (auto &st : s->sstates) st->nslots = 0;  // the slot stride depends on lut_words and N: re-sized at the next launch
+        for (auto &st : s->sstates) {  // the slot stride depends on lut_words and N: re-sized at the next launch
+            st->nslots = 0;
+            st->most_slots = INT32_MAX;
+        }
         s->vis_stride = slot_stride(*s);
         int32_t r_row_bytes = 0;
         if (s->refine != QK_NONE) quant_layout(s->refine, dim, &s->r_dim_align, &r_row_bytes);
