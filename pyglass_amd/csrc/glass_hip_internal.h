@@ -76,7 +76,7 @@ struct LaunchConfig {
     int32_t cap_max;         // LDS pool capacity per wave (>= every query's max(k',ef))
     int32_t vis_hash;        // LDS visited-set words per wave (power of two >= 256)
     int32_t spec;            // integer codes: gather every neighbour's row before the visited test
-    int32_t qwaves;          // waves per query: 1, or 2 / 4 (waves_per_block) waves of a workgroup on one query
+    int32_t qwaves;          // waves per query: 1, or the 2, 4 or 8 (waves_per_block) of a workgroup on one query
 };
 
 // Work counters of a launch: kWorkLines lines of kWorkLineWords words, each of

@@ -6,9 +6,9 @@
 //     kept sorted in LDS as (key, id|checked) pairs;
 //   * the R neighbours of a popped node are loaded from the adjacency row
 //     (one coalesced 4R-byte read), tested-and-set in an exact visited set
-//     (a per-wave LDS hash table that moves to the slot's global bitset if
-//     it fills past half) and kept in adjacency order
-//     (glass/searcher/graph_searcher.hpp:196-224);
+//     (in the wave's LDS: a bitset of a graph that fits, else a table that
+//     moves to the slot's global bitset when 6/8 of its entries are taken)
+//     and kept in adjacency order (glass/searcher/graph_searcher.hpp:196-224);
 //   * their distances are computed by "teams" of lanes from coalesced code
 //     gathers (integer quantizers: |q|^2 + |c|^2 - 2 q.c with packed dot
 //     products, exact; float quantizers: the reference's 16 accumulators and
