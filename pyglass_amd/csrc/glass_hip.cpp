@@ -1421,7 +1421,7 @@ int glass_hip_searcher_set_data(glass_hip_searcher *s, const float *data, int32_
         // graph
         const glass_hip_graph &g = s->graph;
         HIP_TRY(s->d_adj.alloc(g.adj.size()));
-        Stager stage;
+        Stager stage(s->stream);
         HIP_TRY(stage.upload(s->d_adj.p, g.adj.data(), 4 * g.adj.size()));
         HIP_TRY(launch_tidy_rows(s->d_adj.p, g.N, g.K, s->stream));
         HIP_TRY(s->d_eps.alloc(std::max<size_t>(1, g.eps.size())));
@@ -2014,7 +2014,7 @@ int glass_hip_quant_train(const char *quantizer, const char *metric, const float
             if (int r = ensure_stream(t)) return r;
             DevBuf<float> raw;
             HIP_TRY(raw.alloc((size_t)n * dim));
-            Stager stage;
+            Stager stage(t.stream);
             HIP_TRY(stage.upload(raw.p, data, sizeof(float) * (size_t)n * dim));
             if (int r = train_quant(t, raw.p, n)) return r;
         }
