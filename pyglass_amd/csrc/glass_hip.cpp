@@ -2093,8 +2093,8 @@ struct ServerSlot {
     uint64_t *h_out = nullptr;
     uint64_t *d_out = nullptr;       // device address of h_out
     DevBuf<uint8_t> d_in;
-    DevBuf<int32_t> counter;
-    uint32_t *visited = nullptr;     // this slot's share of the server's visited bitsets
+    int32_t *counter = nullptr;      // this slot's work counters and slot areas, in the server's array
+    uint32_t *visited = nullptr;
     hipStream_t stream = nullptr;
     hipEvent_t done = nullptr;
     // A part is queries [q0, q0 + nq) of one request.  r is cleared once the
@@ -2292,7 +2292,7 @@ int server_launch(glass_hip_server &sv, ServerSlot &sl) {
     BatchState bs;
     bs.visited = sl.visited;
     bs.max_slots = sv.slots_per_batch;
-    bs.counter = sl.counter.p;
+    bs.counter = sl.counter;
     bs.out_pairs = sl.d_out;
     if (int r = run_batch(s, d_q, pos, d_ef, d_k, 0, 0, max_cap, max_ef, MODE_BATCH, d_off, nullptr, nullptr, nullptr,
                           sl.stream, &bs))
@@ -2517,6 +2517,7 @@ int glass_hip_server_create(glass_hip_searcher *s, int32_t max_batch, int32_t ma
         sv->in_meta = 16 * (size_t)max_batch;
         sv->in_bytes = sv->in_meta + sizeof(float) * (size_t)max_batch * s->dim;
         sv->out_bytes = 8 * (size_t)max_batch * max_k;
+        size_t ctr_words = 0;
         {
             std::lock_guard<std::mutex> lk(s->mu);
             if (int r = ensure_stream(*s)) return r;
@@ -2553,8 +2554,11 @@ int glass_hip_server_create(glass_hip_searcher *s, int32_t max_batch, int32_t ma
             if (fit < 1) return fail(GLASS_HIP_ENOMEM, "no device memory for one batch in flight (%zu bytes)", per_batch);
             max_inflight = (int32_t)std::min<size_t>((size_t)max_inflight, fit);
             sv->max_inflight = max_inflight;
-            // the server's own slot areas, zeroed (bitsets are all zero between queries)
-            const size_t words = (size_t)max_inflight * (size_t)most * (size_t)s->vis_stride;
+            // The server's own work counters, then its slot areas, zero between
+            // launches and queries: cleared once, by one kernel that is waited
+            // for here, before any slot's stream exists.
+            ctr_words = ((size_t)max_inflight * kWorkWords + 63) / 64 * 64;
+            const size_t words = ctr_words + (size_t)max_inflight * (size_t)most * (size_t)s->vis_stride;
             HIP_TRY(sv->visited.alloc(words));
             HIP_TRY(launch_fill_i32((int32_t *)sv->visited.p, (int64_t)words, 0, s->stream));
             HIP_TRY(hipStreamSynchronize(s->stream));
@@ -2566,12 +2570,10 @@ int glass_hip_server_create(glass_hip_searcher *s, int32_t max_batch, int32_t ma
             HIP_TRY(hipHostMalloc((void **)&sl.h_out, sv->out_bytes, hipHostMallocMapped | hipHostMallocCoherent));
             HIP_TRY(hipHostGetDevicePointer((void **)&sl.d_out, sl.h_out, 0));
             HIP_TRY(sl.d_in.alloc(sv->in_bytes));
-            sl.visited = sv->visited.p + (size_t)i * (size_t)sv->slots_per_batch * (size_t)s->vis_stride;
+            sl.counter = (int32_t *)sv->visited.p + (size_t)i * kWorkWords;
+            sl.visited =
+                sv->visited.p + ctr_words + (size_t)i * (size_t)sv->slots_per_batch * (size_t)s->vis_stride;
             HIP_TRY(hipStreamCreateWithFlags(&sl.stream, hipStreamNonBlocking));
-            // cleared on the stream that the slot's batches run on: the searcher's
-            // may be held up by other callers' work
-            HIP_TRY(sl.counter.alloc(kWorkWords));
-            HIP_TRY(launch_fill_i32(sl.counter.p, kWorkWords, 0, sl.stream));
             HIP_TRY(hipEventCreateWithFlags(&sl.done, hipEventDisableTiming));
         }
         glass_hip_server *p = sv.get();
