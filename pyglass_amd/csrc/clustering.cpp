@@ -276,8 +276,8 @@ int fit_device(const float *rows, int32_t n, int32_t d, int32_t k, int32_t epoch
 }
 
 // A clustering object's stream and events, made by the first call that has
-// pieces to overlap and kept with it (making them takes 0.5 ms, more than all
-// of a call on a few thousand rows); one call at a time.  They belong to the
+// pieces to overlap and kept with it (making them takes 0.05 ms, and 3 the
+// first few times in a process); one call at a time.  They belong to the
 // device that was current then: a call under another one makes its own.
 struct Device {
     std::mutex mu;
@@ -305,11 +305,15 @@ struct Device {
     }
 };
 
-// Nearest centroid of every row.  Rows go to the device in pieces of about
-// 16 MB while the piece before is worked on: the copy bounds the call.
+// Nearest centroid of every row.  More than 24 MB of rows go to the device in
+// pieces of about 16 MB while the piece before is worked on: the copy bounds the
+// call.  Fewer go in one: 35,000 x 128 (18 MB) to 16 and 1,000 clusters take 630
+// and 850 us in two pieces, 595 and 840 in one, and the first call of a process
+// 5.5 ms, 2.2 in one: a stream is another hardware queue.  200,000 x 96 (77 MB)
+// to 1,000: 3,090 in pieces, 3,700 in one.
 int predict_device(Device &dev, const float *cent, int32_t k, int32_t d, const float *x, int32_t n, int32_t *ids) {
     const int64_t piece = std::max<int64_t>(64, ((int64_t)4 << 20) / d / 64 * 64);
-    const int32_t rows = (int32_t)std::min<int64_t>(n, piece);
+    const int32_t rows = (int64_t)n * d <= (6 << 20) ? n : (int32_t)std::min<int64_t>(n, piece);
     const int32_t bufs = n > rows ? 2 : 1;
     if (bufs > 1)
         if (const int r = dev.make()) return r;
